@@ -57,7 +57,11 @@ constexpr int64_t kMaxSegTiles = 256;
 
 struct Plan {
     int SP = 0, S = 0, R = 0, nslice = 1, Spad = 0;
-    bool parts = false;  // partial outputs + slice sum (sliced<T, KB>() instantiations)
+    // slices that the buffer sizes count: fp32 buffers keep the room of
+    // 32-bucket slices' partial outputs, which programs may have sized by that
+    // rule, also where one workgroup holds all buckets
+    int wslice = 0;
+    bool parts = false;  // partial outputs + slice sum (sliced<KB>() instantiations)
     int64_t N = 0, ntiles = 0;
     int nseg = 0, tps = 0;
     int fnseg = 0, fmul = 1;  // forward segments; forward segments per segment of this plan
@@ -71,12 +75,12 @@ struct Plan {
     size_t gfws = 0, gbws = 0, tok_bytes = 0;
 };
 
-// Bucket slices: a workgroup handles SP buckets (bf16: 32, 64 or 128; fp32:
-// 32, the LDS capacity of the backward tile kernels).  bf16 with K <= 4 and
-// L*2^K <= 128 runs one slice of the padded bucket count; everything else
-// runs ceil(S / SP) slices whose partial outputs are summed.
+// Bucket slices: a workgroup handles SP buckets.  K <= 4 (at most 128 buckets
+// in 32 projection columns) runs one slice of the padded bucket count, 32, 64
+// or 128; wider tables run ceil(S / SP) slices of 128 (fp32: 32) buckets whose
+// partial outputs are summed.
 void slice_plan(int dtype, int K, int S, int &SP, int &nslice) {
-    if (dtype == RACE_DTYPE_BF16 && K <= 4 && S <= 128) {
+    if (K <= 4) {
         SP = (S + 31) / 32 * 32;
         if (SP == 96) SP = 128;
         nslice = 1;
@@ -120,7 +124,7 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true) 
     p.S = d->L * p.R;
     slice_plan(d->dtype, d->K, p.S, p.SP, p.nslice);
     p.Spad = p.nslice * p.SP;
-    p.parts = d->dtype != RACE_DTYPE_BF16 || d->K > 4;
+    p.parts = d->K > 4;
     p.N = d->M * d->B * d->H;
     if (p.N > 65535) return fail(RACE_E_UNSUPPORTED, "M*B*H=%lld streams exceed 65535", (long long)p.N);
     p.ntiles = (d->T + TT - 1) / TT;
@@ -173,14 +177,16 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true) 
     if (p.parts && (p.N * ((d->T + 16 * DXF_BLK - 1) / (16 * DXF_BLK)) + 3) / 4 * 256 > kMaxWorkItems)
         return fail(RACE_E_UNSUPPORTED, "M*B*H*T=%lld token-heads exceed one dX launch's 2^32 work-items",
                     (long long)(p.N * d->T));
-    p.part_bytes = p.parts ? align16((size_t)p.nslice * p.N * d->T * D * p.esize) : 0;
-    const size_t xesize = xpart_f32(d->dtype == RACE_DTYPE_BF16, p.SP, d->K) ? sizeof(float) : p.esize;
-    p.xpart_bytes = p.parts ? align16((size_t)p.nslice * p.N * d->T * xcols_of(p.SP, d->K) * xesize) : 0;
+    const bool f32 = d->dtype == RACE_DTYPE_F32;
+    p.wslice = f32 ? (p.S + 31) / 32 : (p.parts ? p.nslice : 0);
+    p.part_bytes = align16((size_t)p.wslice * p.N * d->T * D * p.esize);
+    const size_t xesize = xpart_f32(!f32, p.SP, d->K) ? sizeof(float) : p.esize;
+    p.xpart_bytes = align16((size_t)p.wslice * p.N * d->T * xcols_of(f32 ? 32 : p.SP, d->K) * xesize);
     p.fws = p.fws_core + p.part_bytes;                         // partial O
     p.bws = p.bws_core + 2 * p.xpart_bytes + p.part_bytes;     // dproj columns for dQ, dK; partial dV
     p.tok_bytes = align16((size_t)p.N * d->T * sizeof(float));
-    p.gfws = p.fws + (p.parts ? p.nslice * p.tok_bytes : 0);
-    p.gbws = p.bws + 2 * p.tok_bytes + (p.parts ? p.nslice * p.tok_bytes : 0);  // + the slices' gsum
+    p.gfws = p.fws + p.wslice * p.tok_bytes;
+    p.gbws = p.bws + (2 + p.wslice) * p.tok_bytes;  // + the slices' gsum
     return RACE_OK;
 }
 
@@ -353,7 +359,7 @@ template <typename T, int SP, int KB> int fwd_impl(const race_desc *d, const Pla
             k_fwd_out<T, SP, true, KB, false><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_fwd_out<T, SP, false, KB, false><<<grid, threads_of(SP), 0, s>>>(a);
-        if (sliced<T, KB>()) {
+        if (sliced<KB>()) {
             slice_sum<T>(p, d, a.opart, d->o_stride, a.out, s);
             if (a.den) {
                 const int64_t nt = p.N * d->T;
@@ -376,22 +382,25 @@ int bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_inv_temp, hi
             k_bwd_reduce<T, SP, true, KB, false><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_bwd_reduce<T, SP, false, KB, false><<<grid, threads_of(SP), 0, s>>>(a);
-        if (sliced<T, KB>()) dx_finish<T>(p, d, a.dqpart, a, d->g_stride, a.dq, s);
+        if (sliced<KB>()) dx_finish<T>(p, d, a.dqpart, a, d->g_stride, a.dq, s);
     }
     const int elems = p.Spad * SROW;
     if (run_phase(d, RACE_PHASE_SCAN))
         k_bwd_scan<<<dim3((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N), SCAN_THREADS, 0, s>>>(a.rstate, a.rdelta, p.nseg, elems,
                                                                             d->causal);
     if (run_phase(d, RACE_PHASE_OUT)) {
-        if (d->causal && al && exact_walk(d))
-            k_bwd_out<T, SP, true, KB, false, ALC, true><<<grid, threads_of(SP), 0, s>>>(a);
-        else if (d->causal && al)
-            k_bwd_out<T, SP, true, KB, false, ALC><<<grid, threads_of(SP), 0, s>>>(a);
-        else if (d->causal)
+        if (d->causal && al) {
+            if constexpr (ALC) {
+                if (exact_walk(d))
+                    k_bwd_out<T, SP, true, KB, false, true, true><<<grid, threads_of(SP), 0, s>>>(a);
+                else
+                    k_bwd_out<T, SP, true, KB, false, true><<<grid, threads_of(SP), 0, s>>>(a);
+            }
+        } else if (d->causal)
             k_bwd_out<T, SP, true, KB, false><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_bwd_out<T, SP, false, KB, false><<<grid, threads_of(SP), 0, s>>>(a);
-        if (sliced<T, KB>()) {
+        if (sliced<KB>()) {
             dx_finish<T>(p, d, a.dkpart, a, d->g_stride, a.dk, s);
             slice_sum<T>(p, d, a.dvpart, d->g_stride, a.dv, s);
         }
@@ -421,7 +430,7 @@ template <typename T, int SP, int KB> int gn_fwd_impl(const race_desc *d, const 
             k_fwd_out<T, SP, true, KB, true, ALC><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_fwd_out<T, SP, true, KB, true><<<grid, threads_of(SP), 0, s>>>(a);
-        if (sliced<T, KB>()) {
+        if (sliced<KB>()) {
             const int64_t n4 = p.N * d->T * (D / 4);
             k_slice_sum_gn<T><<<elem_blocks(n4), ELEM_THREADS, 0, s>>>(
                 (const T *)a.opart, a.denpart, p.nslice, p.N, d->T, (int)d->B, (int)d->H, strides_of(d->o_stride), (T *)a.out,
@@ -439,7 +448,7 @@ int gn_bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_beta, hip
     constexpr bool ALC = al_compiled<T, SP, KB>();
     const bool al = ALC && whole_tiles(d, p);
     if (run_phase(d, RACE_PHASE_REDUCE)) {
-        if constexpr (sliced<T, KB>()) {
+        if constexpr (sliced<KB>()) {
             // each slice's share of sum_s P_Q G per token, then rd and gd
             if (al)
                 k_bwd_reduce<T, SP, true, KB, true, ALC, true><<<grid, threads_of(SP), 0, s>>>(a);
@@ -453,7 +462,7 @@ int gn_bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_beta, hip
             k_bwd_reduce<T, SP, true, KB, true, ALC><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_bwd_reduce<T, SP, true, KB, true><<<grid, threads_of(SP), 0, s>>>(a);
-        if (sliced<T, KB>()) dx_finish<T>(p, d, a.dqpart, a, d->g_stride, a.dq, s);
+        if (sliced<KB>()) dx_finish<T>(p, d, a.dqpart, a, d->g_stride, a.dq, s);
     }
     const int elems = p.Spad * SROW;
     if (run_phase(d, RACE_PHASE_SCAN))
@@ -463,7 +472,7 @@ int gn_bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_beta, hip
             k_bwd_out<T, SP, true, KB, true, ALC><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_bwd_out<T, SP, true, KB, true><<<grid, threads_of(SP), 0, s>>>(a);
-        if (sliced<T, KB>()) {
+        if (sliced<KB>()) {
             dx_finish<T>(p, d, a.dkpart, a, d->g_stride, a.dk, s);
             slice_sum<T>(p, d, a.dvpart, d->g_stride, a.dv, s);
         }
@@ -477,8 +486,9 @@ int gn_bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_beta, hip
 #define RACE_FOR_COMBOS(X)                                                                                          \
     X(bf16, 32, 1) X(bf16, 64, 1) X(bf16, 32, 2) X(bf16, 64, 2) X(bf16, 32, 3) X(bf16, 64, 3) X(bf16, 128, 3)       \
     X(bf16, 32, 4) X(bf16, 64, 4) X(bf16, 128, 4) X(bf16, 128, 5) X(bf16, 128, 6) X(bf16, 128, 7) X(bf16, 128, 8)   \
-    X(float, 32, 1) X(float, 32, 2) X(float, 32, 3) X(float, 32, 4) X(float, 32, 5) X(float, 32, 6) X(float, 32, 7)  \
-    X(float, 32, 8)
+    X(float, 32, 1) X(float, 64, 1) X(float, 32, 2) X(float, 64, 2) X(float, 32, 3) X(float, 64, 3)                 \
+    X(float, 128, 3) X(float, 32, 4) X(float, 64, 4) X(float, 128, 4) X(float, 32, 5) X(float, 32, 6)               \
+    X(float, 32, 7) X(float, 32, 8)
 
 template <typename T> int fwd_dispatch(const race_desc *d, const Plan &p, const Args &a, hipStream_t s) {
 #define X(TT_, SP_, KB_)                                                                                             \
@@ -522,7 +532,7 @@ template <typename T, int SP, int KB> int probs_impl(const race_desc *d, const P
         return launched("race_probs");
     }
     k_probs<T, SP, KB, true><<<grid, threads_of(SP), 0, s>>>(a);
-    if (sliced<T, KB>()) dx_finish<T>(p, d, a.dqpart, a, d->g_stride, a.dq, s);
+    if (sliced<KB>()) dx_finish<T>(p, d, a.dqpart, a, d->g_stride, a.dq, s);
     if (grad_inv_temp) k_temp_sum<<<1, 256, 0, s>>>(a.tpart, p.N * p.nseg * p.nslice, grad_inv_temp);
     return launched("race_probs_bwd");
 }

@@ -95,15 +95,38 @@ struct Args {
     const float *dprobs;
 };
 
+// Occupancy.  The tile kernels are bound by each wave's chain of dependent LDS
+// reads, products and barriers, so what a CU gets done is set by the waves it
+// holds, and those by LDS (160 KiB) and registers.  LDS therefore holds only
+// what waves exchange: token rows, sigmoid rows of the columns in use, bucket
+// rows.  The planes' operands, the prefix / total / transpose / corner constants
+// and (bf16: transpose loads; fp32: column reads) the token-major operands need
+// none.  Against planes, constant tables and transposed tiles in LDS, and fp32
+// in slices of 32 buckets (2-wave workgroups, one per CU) with partial outputs
+// summed through HBM, one forward + backward on MI355X took:
+//   fp32 K=4 L=8, 8 x 8192 tokens, causal   1012 -> 437 us (8-wave workgroups)
+//   fp32 K=4 L=4, 8 x 16384, causal         1007 -> 390 us
+//   bf16 K=3 L=8, 48 x 4001, causal          363 -> 276 us
+//   bf16 K=4 L=4, 48 x 8192, global          614 -> 454 us
+//   bf16 K=2 L=5, 384 x 785, non-causal      321 -> 185 us (8 waves per CU, not 4)
+// The 128-bucket bf16 kernels keep their waves per CU (registers) and their time.
 constexpr int SROW = D + 1;  // state row: D values of B (or U) then A (or alpha)
 constexpr int WB = 16;       // buckets per wave
 __host__ __device__ constexpr int threads_of(int SP) { return 64 * (SP / WB); }
 
-// Instantiations that may run several bucket slices (fp32, and bf16 with more
-// than 4 hash bits) write partial outputs in the element type, summed in fp32
-// by k_slice_sum; the others write the outputs directly and run one slice.
-template <typename T, int KB> __host__ __device__ constexpr bool sliced() {
-    return !std::is_same<T, bf16>::value || KB > 4;
+// Instantiations that may run several bucket slices (more than 4 hash bits)
+// write partial outputs in the element type, summed in fp32 by k_slice_sum;
+// the others write the outputs directly and run one slice (at most 4 bits in
+// 32 projection columns are at most 128 buckets, one workgroup's).
+template <int KB> __host__ __device__ constexpr bool sliced() { return KB > 4; }
+
+// Projection columns that a workgroup's sigmoid rows hold: the L*K columns
+// an unsliced instantiation can have (L <= SP / 2^KB tables), in blocks of
+// 16; a slice's tables may be any of the 32 columns.  16-column rows are half
+// the LDS and half the projections of 32-column ones whose second half is
+// padding.
+template <int SP, int KB> __host__ __device__ constexpr int ncol_of() {
+    return !sliced<KB>() && (SP >> KB) * KB <= 16 ? 16 : NCOL;
 }
 
 // Row width (elements, a power of 2) of the sliced dX partials: the
@@ -267,9 +290,12 @@ template <typename P> __device__ __forceinline__ P *part_at(P *part, int64_t t0,
     return at_bytes(part + t0 * D, (uint32_t)(t * D + d) * (uint32_t)sizeof(P));
 }
 
+// Staging chunks are vector types: HIP's uint2 / uint4 structs can come out of
+// the optimiser as 64-bit integers joined from halves, an operation on a
+// prefetched register that waits for its load in the middle of a tile.
 template <int B> struct ChunkOf;
-template <> struct ChunkOf<16> { typedef uint4 type; };
-template <> struct ChunkOf<8> { typedef uint2 type; };
+template <> struct ChunkOf<16> { typedef u32x4 type; };
+template <> struct ChunkOf<8> { typedef u32x2 type; };
 
 // ---- swizzled LDS rows (bf16; race_layout.h): arrays read as 16-byte
 // operand pieces of 16 rows and written in 8-byte pieces.  fp32 keeps padded
@@ -335,7 +361,7 @@ template <typename T, bool SW> struct NatL {
 // fall on 32 distinct banks (the swizzled pi-order rows put them on 16).
 template <typename T> struct TrL {
     static constexpr bool P = false;
-    static constexpr int LD = D + 16;
+    static constexpr int LD = is_bf16<T>() ? D + 16 : ld_of<T>(D);  // fp32: column reads, conflict-free
     __device__ __forceinline__ static int off(int r, int k) { return r * LD + k; }
 };
 
@@ -384,55 +410,44 @@ template <typename T, int NTH, bool AL = false> struct Prefetch {
             if (idx < CHUNKS && t < rem) v[j] = ld_at<chunk_t>(base, tile_off(t, st, c * EPC, sizeof(T)));
         }
     }
-    template <class NL = NatL<T, false>> __device__ __forceinline__ void commit(T *nat, T *trn) const {
-        constexpr int LDT = ldp_of<T>(TT);
+    template <class NL = NatL<T, false>> __device__ __forceinline__ void commit(T *nat) const {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const int idx = threadIdx.x + j * NTH, t = idx / CPR, c = idx % CPR;
             if (!WHOLE && idx >= CHUNKS) continue;
-            if (nat) {
-                if constexpr (NL::P && CB == 16) {  // two runs of 4 elements
-                    *reinterpret_cast<uint2 *>(nat + NL::off(t, c * EPC)) = uint2{v[j].x, v[j].y};
-                    *reinterpret_cast<uint2 *>(nat + NL::off(t, c * EPC + 4)) = uint2{v[j].z, v[j].w};
-                } else {
-                    *reinterpret_cast<chunk_t *>(nat + NL::off(t, c * EPC)) = v[j];
-                }
-            }
-            if (trn) {
-                const T *e = reinterpret_cast<const T *>(&v[j]);
-#pragma unroll
-                for (int q = 0; q < EPC; ++q) trn[(c * EPC + q) * LDT + t] = e[q];
+            if constexpr (NL::P && CB == 16) {  // two runs of 4 elements
+                *reinterpret_cast<u32x2 *>(nat + NL::off(t, c * EPC)) = __builtin_shufflevector(v[j], v[j], 0, 1);
+                *reinterpret_cast<u32x2 *>(nat + NL::off(t, c * EPC + 4)) = __builtin_shufflevector(v[j], v[j], 2, 3);
+            } else {
+                *reinterpret_cast<chunk_t *>(nat + NL::off(t, c * EPC)) = v[j];
             }
         }
     }
 };
 
-// Staging of a tile that is also needed transposed ([D][TT], t contiguous):
-// each task is a pair of tokens (2tp, 2tp+1) times one 8-byte chunk of d.
-// Lanes of a wave cover 16 token pairs x 4 chunks, so the transposed rows are
-// written as packed token pairs to consecutive LDS words (few bank conflicts)
-// while each token row is still read in 32-byte runs.  NPART tensors share
-// the workgroup: this one uses threads [part*NTH/NPART, (part+1)*NTH/NPART).
-// TRN = false: natural rows only (bf16 reads the token operands from them
-// with LDS transpose loads, col_operand).
-template <typename T, int NTH, int NPART, bool AL = false, bool TRN = true> struct PrefetchT {
-    static constexpr int NT = NTH / NPART;
+// Staging of a tile as transposed rows ([D][TT], t contiguous): each task is a
+// pair of tokens (2tp, 2tp+1) times one 8-byte chunk of d.  Lanes of a wave
+// cover 16 token pairs x 4 chunks, so the transposed rows are written as packed
+// token pairs to consecutive LDS words (few bank conflicts) while each token
+// row is still read in 32-byte runs.  (bf16: the global normalisation's V.)
+template <typename T, int NTH, bool AL = false> struct PrefetchT {
+    static_assert(sizeof(T) == 2, "bf16 rows");
     static constexpr int EPC = 8 / sizeof(T), CPR = D / EPC, TASKS = (TT / 2) * CPR;
-    static constexpr int PER = (TASKS + NT - 1) / NT;
+    static constexpr int PER = (TASKS + NTH - 1) / NTH;
     uint2 v[PER][2];
-    __device__ __forceinline__ static bool task_of(int part, int j, int &tp, int &c) {
-        const int local = (int)threadIdx.x - part * NT, task = local + j * NT;
+    __device__ __forceinline__ static bool task_of(int j, int &tp, int &c) {
+        const int task = (int)threadIdx.x + j * NTH;
         tp = (task >> 2) & 15;
         c = (task & 3) + 4 * (task >> 6);
-        return local >= 0 && local < NT && task < TASKS;
+        return task < TASKS;
     }
-    __device__ __forceinline__ void issue(int part, const T *__restrict__ src, int64_t st, int64_t t0, int64_t Tn) {
+    __device__ __forceinline__ void issue(const T *__restrict__ src, int64_t st, int64_t t0, int64_t Tn) {
         const T *base = tile_ptr(src, st, t0);
         const int rem = AL ? TT : tile_rows(t0, Tn);
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             int tp, c;
-            const bool ok = task_of(part, j, tp, c);
+            const bool ok = task_of(j, tp, c);
             const uint32_t off = tile_off(2 * tp, st, c * EPC, sizeof(T));
             v[j][0] = uint2{0, 0};
             v[j][1] = uint2{0, 0};
@@ -440,46 +455,33 @@ template <typename T, int NTH, int NPART, bool AL = false, bool TRN = true> stru
             if (ok && 2 * tp + 1 < rem) v[j][1] = ld_at<uint2>(base, off + (uint32_t)st * (uint32_t)sizeof(T));
         }
     }
-    template <class NL = NatL<T, false>> __device__ __forceinline__ void commit(int part, T *nat, T *trn) const {
+    __device__ __forceinline__ void commit(T *trn) const {
         constexpr int LDT = ldp_of<T>(TT);
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             int tp, c;
-            if (!task_of(part, j, tp, c)) continue;
-            if (nat) {
-                *reinterpret_cast<uint2 *>(nat + NL::off(2 * tp, c * EPC)) = v[j][0];
-                *reinterpret_cast<uint2 *>(nat + NL::off(2 * tp + 1, c * EPC)) = v[j][1];
-            }
-            if constexpr (!TRN) continue;
-            // element q of a chunk: bf16 -> 16-bit half q of the 64-bit chunk; fp32 -> word q
+            if (!task_of(j, tp, c)) continue;
+            // element q of a chunk is 16-bit half q of the 64-bit chunk
             const uint2 a = v[j][0], b = v[j][1];
             uint32_t *row = reinterpret_cast<uint32_t *>(trn + (c * EPC) * LDT + 2 * tp);
             constexpr int RW = LDT * (int)sizeof(T) / 4;  // words per transposed row
-            if constexpr (sizeof(T) == 2) {
-                row[0 * RW] = (a.x & 0xFFFFu) | (b.x << 16);
-                row[1 * RW] = (a.x >> 16) | (b.x & 0xFFFF0000u);
-                row[2 * RW] = (a.y & 0xFFFFu) | (b.y << 16);
-                row[3 * RW] = (a.y >> 16) | (b.y & 0xFFFF0000u);
-            } else {
-                *reinterpret_cast<uint2 *>(row) = uint2{a.x, b.x};
-                *reinterpret_cast<uint2 *>(row + RW) = uint2{a.y, b.y};
-            }
+            row[0 * RW] = (a.x & 0xFFFFu) | (b.x << 16);
+            row[1 * RW] = (a.x >> 16) | (b.x & 0xFFFF0000u);
+            row[2 * RW] = (a.y & 0xFFFFu) | (b.y << 16);
+            row[3 * RW] = (a.y >> 16) | (b.y & 0xFFFF0000u);
         }
     }
 };
 
-// Two token tiles staged like PrefetchT (natural and/or transposed), the
-// first by the workgroup's first half of waves and the second by the other
-// half.  The tensor is chosen per wave (scalar selects of the source and
+// Two token tiles staged as natural rows, pairs of tokens per task, the first
+// by the workgroup's first half of waves and the second by the other half.  The tensor is chosen per wave (scalar selects of the source and
 // destinations), so every lane takes part and no lane mask is needed.
-// TRN: also write the transposed rows (fp32; bf16 reads its token operands
-// from the natural rows with LDS transpose loads, col_operand).
-template <typename T, int NTH, bool AL = false, bool TRN = true> struct PrefetchT2 {
+template <typename T, int NTH, bool AL = false> struct Prefetch2 {
     static constexpr int NT = NTH / 2;
     static constexpr int EPC = 8 / sizeof(T), CPR = D / EPC, TASKS = (TT / 2) * CPR;
     static_assert(NT % 64 == 0 && TASKS % NT == 0, "whole waves per tensor, whole tasks per lane");
     static constexpr int PER = TASKS / NT;
-    uint2 v[PER][2];
+    u32x2 v[PER][2];
     __device__ __forceinline__ static bool second() { return wave_id() >= NT / 64; }
     __device__ __forceinline__ static void task_of(int j, int &tp, int &c) {
         const int task = ((int)threadIdx.x & (NT - 1)) + j * NT;
@@ -498,40 +500,25 @@ template <typename T, int NTH, bool AL = false, bool TRN = true> struct Prefetch
             task_of(j, tp, c);
             const uint32_t off = tile_off(2 * tp, st, c * EPC, sizeof(T));
             if constexpr (AL) {
-                v[j][0] = ld_at<uint2>(base, off);
-                v[j][1] = ld_at<uint2>(base, off + (uint32_t)st * (uint32_t)sizeof(T));
+                v[j][0] = ld_at<u32x2>(base, off);
+                v[j][1] = ld_at<u32x2>(base, off + (uint32_t)st * (uint32_t)sizeof(T));
             } else {
-                v[j][0] = uint2{0, 0};
-                v[j][1] = uint2{0, 0};
-                if (2 * tp < rem) v[j][0] = ld_at<uint2>(base, off);
-                if (2 * tp + 1 < rem) v[j][1] = ld_at<uint2>(base, off + (uint32_t)st * (uint32_t)sizeof(T));
+                v[j][0] = u32x2{0, 0};
+                v[j][1] = u32x2{0, 0};
+                if (2 * tp < rem) v[j][0] = ld_at<u32x2>(base, off);
+                if (2 * tp + 1 < rem) v[j][1] = ld_at<u32x2>(base, off + (uint32_t)st * (uint32_t)sizeof(T));
             }
         }
     }
     template <class NL = NatL<T, false>>
-    __device__ __forceinline__ void commit(T *nat0, T *trn0, T *nat1, T *trn1) const {
-        constexpr int LDT = ldp_of<T>(TT);
-        const bool sc = second();
-        T *nat = sc ? nat1 : nat0, *trn = sc ? trn1 : trn0;
+    __device__ __forceinline__ void commit(T *nat0, T *nat1) const {
+        T *nat = second() ? nat1 : nat0;
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             int tp, c;
             task_of(j, tp, c);
-            *reinterpret_cast<uint2 *>(nat + NL::off(2 * tp, c * EPC)) = v[j][0];
-            *reinterpret_cast<uint2 *>(nat + NL::off(2 * tp + 1, c * EPC)) = v[j][1];
-            if constexpr (!TRN) continue;
-            const uint2 a = v[j][0], b = v[j][1];
-            uint32_t *row = reinterpret_cast<uint32_t *>(trn + (c * EPC) * LDT + 2 * tp);
-            constexpr int RW = LDT * (int)sizeof(T) / 4;
-            if constexpr (sizeof(T) == 2) {
-                row[0 * RW] = (a.x & 0xFFFFu) | (b.x << 16);
-                row[1 * RW] = (a.x >> 16) | (b.x & 0xFFFF0000u);
-                row[2 * RW] = (a.y & 0xFFFFu) | (b.y << 16);
-                row[3 * RW] = (a.y >> 16) | (b.y & 0xFFFF0000u);
-            } else {
-                *reinterpret_cast<uint2 *>(row) = uint2{a.x, b.x};
-                *reinterpret_cast<uint2 *>(row + RW) = uint2{a.y, b.y};
-            }
+            *reinterpret_cast<u32x2 *>(nat + NL::off(2 * tp, c * EPC)) = v[j][0];
+            *reinterpret_cast<u32x2 *>(nat + NL::off(2 * tp + 1, c * EPC)) = v[j][1];
         }
     }
 };
@@ -556,54 +543,124 @@ struct TokPre {
     }
 };
 
-// Planes [L*K][D] fp32 -> LDS.  pl/pllo: [NCOL][ld_of<T>(D)] (bf16 keeps a
-// hi/lo split so the projection is close to fp32), plt: [D][ld_of<T>(NCOL)].
-template <typename T, int NTH, class NL = NatL<T, false>>
-__device__ void load_planes(const float *__restrict__ planes, int LK, T *pl, T *pllo, T *plt) {
+// Operand of 8 consecutive k values (k = 8g .. 8g+7 of lane (g, i)), the
+// layout ld_frag reads from k-contiguous rows, from registers.
+template <typename T> __device__ __forceinline__ Frag<T> frag_seq(const float (&v)[8]);
+template <> __device__ __forceinline__ Frag<bf16> frag_seq<bf16>(const float (&v)[8]) {
+    Frag<bf16> f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f.v[j] = (bf16)v[j];
+    return f;
+}
+template <> __device__ __forceinline__ Frag<float> frag_seq<float>(const float (&v)[8]) {
+    Frag<float> f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        f.lo[j] = v[j];
+        f.hi[j] = v[4 + j];
+    }
+    return f;
+}
+
+// planes^T [D][NCOL] (the dX product's operand rows) -> LDS
+template <typename T, int NTH> __device__ void load_planes_t(const float *__restrict__ planes, int LK, T *plt) {
     for (int idx = threadIdx.x; idx < NCOL * D; idx += NTH) {
         const int c = idx / D, d = idx % D;
-        const float w = c < LK ? planes[c * D + d] : 0.f;
-        const T hi = from_f32<T>(w);
-        if (pl) pl[NL::off(c, d)] = hi;
-        if (pllo) pllo[NL::off(c, d)] = from_f32<T>(w - to_f32(hi));
-        if (plt) plt[sw_off<T, NCOL>(d, c)] = hi;
+        plt[sw_off<T, NCOL>(d, c)] = from_f32<T>(c < LK ? planes[c * D + d] : 0.f);
     }
 }
 
-// One 16x16 tile (rows c = 16mc.., columns t = 16nt..) of planes . X^T, then
-// th = tanh and the sigmoid pair of 2*th*inv_temp, stored as sp/sm/sth
-// [TT][ld_of<float>(NCOL)] (lane writes its 4 consecutive c of token t).
-// The planes operands of one 16-column block (rows 16 mc.. of pl / pllo),
-// held in registers by a wave whose projection task keeps that block on
-// every tile.
+// The planes operand of a wave's projection tasks (rows 16 mc + i of
+// planes [L*K][D], in NL's k order), in registers: PlaneBlocks gives every
+// wave one column block for all of its tasks, so the planes are read from
+// memory once per workgroup and take no LDS.  bf16 keeps a hi/lo split, so the
+// projection is close to fp32.
 template <typename T> struct PlaneOps {
-    Frag<T> hi[D / 32], lo[D / 32];
-    template <class NL> __device__ __forceinline__ void load(const T *pl, const T *pllo, int mc) {
+    Frag<T> hi[D / 32], lo[is_bf16<T>() ? D / 32 : 1];
+    template <class NL> __device__ __forceinline__ void load(const float *__restrict__ planes, int LK, int mc) {
+        // rows past L*K read the last one (every lane loads: no branch per load) and are cleared
+        const int c = 16 * mc + li();
+        const bool live = c < LK;
+        const float *row = planes + (live ? c : LK - 1) * D;
 #pragma unroll
         for (int kp = 0; kp < D / 32; ++kp) {
-            hi[kp] = NL::frag(pl, 16 * mc + li(), kp);
-            if constexpr (is_bf16<T>()) lo[kp] = NL::frag(pllo, 16 * mc + li(), kp);
+            // slots 0..3 and 4..7 of the lane's operand: pi order, or (padded natural rows) 8 consecutive k
+            const float *p0 = row + 32 * kp + (NL::P ? 4 : 8) * lg(), *p1 = p0 + (NL::P ? 16 : 4);
+            float v[8], r[8];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] = p0[j];
+                v[j + 4] = p1[j];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                v[j] = live ? v[j] : 0.f;
+                if constexpr (is_bf16<T>()) r[j] = v[j] - to_f32(from_f32<T>(v[j]));
+            }
+            hi[kp] = frag_seq<T>(v);
+            if constexpr (is_bf16<T>()) lo[kp] = frag_seq<T>(r);
         }
     }
 };
 
-// pc: the block's operands in registers (mc is then that block), or null.
+// Where a tile kernel keeps its planes: in registers, or (the 128-bucket bf16
+// instantiations that guard their tiles, whose registers are at the limit of
+// their waves per SIMD: 16 more spill) as hi and lo rows in LDS.
+template <typename T, int SP, bool AL> __host__ __device__ constexpr bool planes_reg() {
+    return !is_bf16<T>() || SP < 128 || AL;
+}
+template <typename T, class NL, bool REG> struct PlaneSrc {
+    static constexpr size_t lds_bytes = REG ? 0 : 2 * sizeof(T) * NCOL * NL::LD;
+    PlaneOps<T> ops;  // REG
+    const T *rows;    // !REG: hi rows [NCOL][LD], then lo rows
+    // one block mcw per wave (REG); visible to all waves after the next barrier (LDS)
+    template <int NTH> __device__ __forceinline__ void init(const float *__restrict__ planes, int LK, int mcw, T *lds) {
+        if constexpr (REG) {
+            ops.template load<NL>(planes, LK, mcw);
+        } else {
+            for (int idx = threadIdx.x; idx < NCOL * D; idx += NTH) {
+                const int c = idx / D, d = idx % D;
+                const float x = c < LK ? planes[c * D + d] : 0.f;
+                const T hi = from_f32<T>(x);
+                lds[NL::off(c, d)] = hi;
+                lds[NCOL * NL::LD + NL::off(c, d)] = from_f32<T>(x - to_f32(hi));
+            }
+            rows = lds;
+        }
+    }
+    __device__ __forceinline__ Frag<T> hi(int mc, int kp) const {
+        if constexpr (REG)
+            return ops.hi[kp];
+        else
+            return NL::frag(rows, 16 * mc + li(), kp);
+    }
+    __device__ __forceinline__ Frag<T> lo(int mc, int kp) const {
+        if constexpr (REG)
+            return ops.lo[kp];
+        else
+            return NL::frag(rows + NCOL * NL::LD, 16 * mc + li(), kp);
+    }
+};
+
+// One 16x16 tile (columns c = 16mc.. of the planes pc, tokens t = 16nt..) of planes . X^T, then th = tanh and the sigmoid pair of
+// 2*th*inv_temp, stored as sp/sm/sth [TT][ld_of<float>(NC)] (lane writes its 4
+// consecutive c of token t).
 // PAIR: instead of the corner pair of each column, write the products of
 // corner pairs of the lane's 4 columns (a nibble: columns c0 .. c0+3, c0 = 4q;
 // 8- and 4-bit tables are whole nibbles), the index's high bit choosing the
 // first column's factor (1: sigmoid(2u)):
 //   sp[c0 + j] = f(c0, j >> 1) f(c0 + 1, j & 1),  sm[c0 + j] = f(c0 + 2, j >> 1) f(c0 + 3, j & 1),
 // so probs_st_ forms a bucket probability from two or four products.
-template <typename T, class NL = NatL<T, false>, bool PAIR = false>
-__device__ void project_tile(const T *sx, const T *pl, const T *pllo, int mc, int nt, float inv_temp, float *sp,
-                             float *sm, float *sth, const PlaneOps<T> *pc = nullptr) {
-    constexpr int LDC = ld_of<float>(NCOL);
+template <typename T, class NL, bool PAIR, int NC, class PS>
+__device__ void project_tile(const T *sx, const PS &pc, int mc, int nt, float inv_temp, float *sp, float *sm,
+                             float *sth) {
+    constexpr int LDC = ld_of<float>(NC);
     f32x4 acc = zero4();
 #pragma unroll
     for (int kp = 0; kp < D / 32; ++kp) {
         const Frag<T> x = NL::frag(sx, 16 * nt + li(), kp);
-        mma(acc, pc ? pc->hi[kp] : NL::frag(pl, 16 * mc + li(), kp), x);
-        if constexpr (is_bf16<T>()) mma(acc, pc ? pc->lo[kp] : NL::frag(pllo, 16 * mc + li(), kp), x);
+        mma(acc, pc.hi(mc, kp), x);
+        if constexpr (is_bf16<T>()) mma(acc, pc.lo(mc, kp), x);
     }
     const int t = 16 * nt + li(), c0 = 16 * mc + 4 * lg();
     // the corner pair (sigmoid(2u), sigmoid(-2u)), u = th inv_temp, from
@@ -641,9 +698,9 @@ template <int KB> constexpr bool pair_tables() { return KB == 4 || KB == 8; }
 // corner pair (sp - sm), or (PAIR) from the nibble's pair products, whose
 // halves sum to one column's factor times (sigmoid(2u') + sigmoid(-2u')) = 1
 // of the other column in the pair.
-template <bool PAIR>
+template <bool PAIR, int NC>
 __device__ __forceinline__ float corner_tanh(const float *sp, const float *sm, int t, int c) {
-    constexpr int LDC = ld_of<float>(NCOL);
+    constexpr int LDC = ld_of<float>(NC);
     if constexpr (PAIR) {
         const int m = c & 3;
         const f32x4 h = *reinterpret_cast<const f32x4 *>((m < 2 ? sp : sm) + t * LDC + (c & ~3));
@@ -653,19 +710,21 @@ __device__ __forceinline__ float corner_tanh(const float *sp, const float *sm, i
     }
 }
 
-// Projection columns a workgroup needs: the K columns of every table its
-// bucket slice [z SP, (z+1) SP) touches, as 16-column blocks pb0 .. pb0+nb-1
-// (one task per block and 16-token half).  A slice of part of a table (bf16
-// with K >= 5) or of a few tables (fp32) projects one block instead of all
-// of them; C4's single slice of 8 tables of 4 bits needs both.
-struct PlaneBlocks {
+// Projection columns a workgroup of NW waves needs: the K columns of every
+// table its bucket slice [z SP, (z+1) SP) touches, as 16-column blocks
+// pb0 .. pb0+nb-1 (one task per block and 16-token half).  A slice of part of a
+// table (bf16 with K >= 5) or of a few tables (fp32) projects one block instead
+// of both; unsliced instantiations project all of their NC columns (compile-time
+// constants, so their task loops specialise per iteration).
+// A wave takes tasks w, w + NW, ...; their order gives all of them one column
+// block (with two waves the block is the task's low bit), the wave's plane
+// operand (PlaneOps).
+template <int NW> struct PlaneBlocks {
     int pb0, lg;  // first block; log2 of the tasks per projected tensor (1: one block, 2: both)
-    // full: every column block (compile-time constants; the unsliced
-    // instantiations, whose task loops then specialise per iteration)
-    __device__ __forceinline__ PlaneBlocks(int z, int SP, int KB, int L, bool full) {
+    __device__ __forceinline__ PlaneBlocks(int z, int SP, int KB, int L, bool full, int NC) {
         if (full) {
             pb0 = 0;
-            lg = 2;
+            lg = NC / 16;
             return;
         }
         const int l0 = (z * SP) >> KB;
@@ -676,8 +735,10 @@ struct PlaneBlocks {
     __device__ __forceinline__ int tasks() const { return 2 << (lg - 1); }  // per projected tensor
     __device__ __forceinline__ int task(int q) const { return q & (tasks() - 1); }   // task within its tensor
     __device__ __forceinline__ int tensor(int q) const { return q >> lg; }          // which tensor
-    // column block of task r < tasks() (token half r & 1)
-    __device__ __forceinline__ int mc(int r) const { return pb0 + (r >> 1); }
+    // column block and token half of task r < tasks()
+    // (one block: r < 2, so r >> 1 is 0)
+    __device__ __forceinline__ int mc(int r) const { return pb0 + (NW == 2 && lg == 2 ? r & 1 : r >> 1); }
+    __device__ __forceinline__ int half(int r) const { return NW == 2 && lg == 2 ? r >> 1 : r & 1; }
 };
 
 // Bucket probabilities of the wave's 16 buckets in bucket-row layout:
@@ -692,9 +753,9 @@ struct PlaneBlocks {
 // nibble's two low bits: P = sp[n + (r >> 2 & 3)] sm[n + (r & 3)] over the
 // table's last nibble n, times (8 bits) the first nibble's two products,
 // which the wave's buckets share.
-template <int KB, bool FULL, bool PAIR = false>
+template <int KB, bool FULL, bool PAIR, int NC>
 __device__ __forceinline__ void probs_st_(const float *sp, const float *sm, int sw, int S, int nv, f32x4 (&P)[2]) {
-    constexpr int LDC = ld_of<float>(NCOL);
+    constexpr int LDC = ld_of<float>(NC);
     constexpr int R = 1 << KB;
     const int g = lg(), i = li();
     const int s0 = sw + 4 * g;
@@ -758,28 +819,9 @@ __device__ __forceinline__ void probs_st_(const float *sp, const float *sm, int 
         }
     }
 }
-template <int KB, bool AL = false, bool PAIR = false>
+template <int KB, bool AL, bool PAIR, int NC>
 __device__ __forceinline__ void probs_st(const float *sp, const float *sm, int sw, int S, int nv, f32x4 (&P)[2]) {
-    probs_st_<KB, AL, PAIR>(sp, sm, sw, S, nv, P);
-}
-
-// Operand of 8 consecutive k values (k = 8g .. 8g+7 of lane (g, i)), the
-// layout ld_frag reads from k-contiguous rows, from registers.
-template <typename T> __device__ __forceinline__ Frag<T> frag_seq(const float (&v)[8]);
-template <> __device__ __forceinline__ Frag<bf16> frag_seq<bf16>(const float (&v)[8]) {
-    Frag<bf16> f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f.v[j] = (bf16)v[j];
-    return f;
-}
-template <> __device__ __forceinline__ Frag<float> frag_seq<float>(const float (&v)[8]) {
-    Frag<float> f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        f.lo[j] = v[j];
-        f.hi[j] = v[4 + j];
-    }
-    return f;
+    probs_st_<KB, AL, PAIR, NC>(sp, sm, sw, S, nv, P);
 }
 
 // ------------------------------------------------------------ constant operands
@@ -802,67 +844,75 @@ template <> __device__ __forceinline__ Frag<float> frag_pi_from<float>(const flo
     return f;
 }
 
+// Keep a constant operand in registers: without this the compiler may
+// rebuild it from the lane index at every use.
+__device__ __forceinline__ void pin(Frag<bf16> &f) { asm volatile("" : "+v"(f.v)); }
+__device__ __forceinline__ void pin(Frag<float> &f) { asm volatile("" : "+v"(f.lo), "+v"(f.hi)); }
+__device__ __forceinline__ void pin(Frag4<bf16> &f) { asm volatile("" : "+v"(f.v)); }
+__device__ __forceinline__ void pin(Frag4<float> &f) { asm volatile("" : "+v"(f.v)); }
+
 // B operands that turn token contractions into prefix sums, totals and
-// transposes on the matrix cores, read from small LDS tables:
-//   tri[t][tau] = (tau <= t): column t = 16nt + i of the prefix (row 31 is
-//                 all ones: token totals, replicated over the columns)
-//   id[s][s']   = (s == s'): 16-deep identity for transposes
+// transposes on the matrix cores, built in registers from the lane index:
+//   tri[t][tau] = (tau <= t): column t = 16nt + i of the prefix
+//   ones        : token totals, replicated over the columns
+//   ident[s][s'] = (s == s'): 16-deep identity for transposes
+// (fp32 rebuilds the triangle and the ones at each use: 24 registers for a few
+// compares beside products of 256 cycles.)
 template <typename T> struct Consts {
-    static constexpr int LDT = ldp_of<T>(TT), LDI = ldp_of<T>(16);
-    static constexpr size_t bytes = sizeof(T) * (TT * LDT + 16 * LDI);
-    const T *tri, *id;
-    // bf16: the prefix and total operands in registers (cache(), once the
-    // table is visible), so the tile loops do not read them from LDS
     Frag<T> tri0_, tri1_, ones_;
-    __device__ __forceinline__ void init(T *buf, int nth) {
-        T *t = buf, *d = buf + TT * LDT;
-        for (int idx = threadIdx.x; idx < TT * LDT; idx += nth)
-            t[idx] = from_f32<T>(idx % LDT <= idx / LDT ? 1.f : 0.f);
-        for (int idx = threadIdx.x; idx < 16 * LDI; idx += nth)
-            d[idx] = from_f32<T>(idx % LDI == idx / LDI ? 1.f : 0.f);
-        tri = t;
-        id = d;
+    Frag4<T> id_;
+    __device__ __forceinline__ static Frag<T> tri(int t) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (j < 4 ? 4 * lg() + j : 12 + 4 * lg() + j) <= t ? 1.f : 0.f;
+        return frag_pi_from<T>(v);
     }
-    __device__ __forceinline__ void cache() {
+    __device__ __forceinline__ void init() {
+        f32x4 d;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[j] = 4 * lg() + j == li() ? 1.f : 0.f;
+        id_ = frag16_acc<T>(d);
         if constexpr (is_bf16<T>()) {
-            tri0_ = ld_frag_pi(tri + li() * LDT);
-            tri1_ = ld_frag_pi(tri + (16 + li()) * LDT);
-            ones_ = ld_frag_pi(tri + (TT - 1) * LDT);
+            tri0_ = tri(li());
+            tri1_ = tri(16 + li());
+            ones_ = tri(TT);
+            pin(tri0_);
+            pin(tri1_);
+            pin(ones_);
+            pin(id_);
         }
     }
     __device__ __forceinline__ Frag<T> tri_op(int nt) const {
         if constexpr (is_bf16<T>())
             return nt ? tri1_ : tri0_;
         else
-            return ld_frag_pi(tri + (16 * nt + li()) * LDT);
+            return tri(16 * nt + li());
     }
     __device__ __forceinline__ Frag<T> ones() const {
         if constexpr (is_bf16<T>())
             return ones_;
         else
-            return ld_frag_pi(tri + (TT - 1) * LDT);
+            return tri(TT);
     }
-    __device__ __forceinline__ Frag4<T> ident() const { return ld_frag16(id + li() * LDI); }
+    __device__ __forceinline__ Frag4<T> ident() const { return id_; }
 };
 // bf16 pairwise transposes: id[n][k] = (k == n), 32 x 32.  With the pair
 // operand A = frag_acc(X0, X1) of two bucket-row tiles, A . lo() = X0^T and
 // A . hi() = X1^T: every k slot holds data, none is zero padding.
 template <typename T> struct PairOps {
-    static constexpr int LDT = ldp_of<T>(TT);
-    static constexpr size_t bytes = is_bf16<T>() ? sizeof(T) * TT * LDT : 0;
-    const T *id = nullptr;
-    Frag<T> lo_, hi_;  // in registers after cache()
-    __device__ __forceinline__ void init(T *buf, int nth) {
+    Frag<T> lo_, hi_;
+    __device__ __forceinline__ void init() {
         if constexpr (is_bf16<T>()) {
-            for (int idx = threadIdx.x; idx < TT * LDT; idx += nth)
-                buf[idx] = from_f32<T>(idx % LDT == idx / LDT ? 1.f : 0.f);
-            id = buf;
-        }
-    }
-    __device__ __forceinline__ void cache() {
-        if constexpr (is_bf16<T>()) {
-            lo_ = ld_frag_pi(id + li() * LDT);
-            hi_ = ld_frag_pi(id + (16 + li()) * LDT);
+            float l[8], h[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                l[j] = j < 4 && 4 * lg() + j == li() ? 1.f : 0.f;
+                h[j] = j >= 4 && 4 * lg() + j - 4 == li() ? 1.f : 0.f;
+            }
+            lo_ = frag_pi_from<T>(l);
+            hi_ = frag_pi_from<T>(h);
+            pin(lo_);
+            pin(hi_);
         }
     }
     __device__ __forceinline__ Frag<T> lo() const { return lo_; }
@@ -885,10 +935,6 @@ template <> struct OpX<float> { Frag4<float> f; };
 //   KB=4: g0 = c0 c1 c2 sum, g1 = c3 sum;  KB=3: g = table g: c0 c1 c2 sum;
 //   KB=2: g = table g: c0 c1 sum;          KB=1: g = tables 2g, 2g+1: (c0 sum) x 2.
 template <typename T, int KB> struct HashOps {
-    static constexpr int W_ = is_bf16<T>() ? TT : 16;  // bf16: 16 k values, then the same 16 again
-    static constexpr int LDI = ldp_of<T>(W_);
-    static constexpr size_t bytes = sizeof(T) * 16 * LDI;
-    const T *a;
     // row r = 4g + e (lane group g, slot e of the product's accumulator):
     // 1 = corner k of local table tl, 2 = sum of tl, 0 = unused; de = slot of
     // tl's sum row in the row's lane group.  The corners are spread over the
@@ -919,23 +965,23 @@ template <typename T, int KB> struct HashOps {
             return (e & 1) ? 2 : 1;
         }
     }
-    __device__ __forceinline__ void init(T *buf, int nth) {
-        for (int idx = threadIdx.x; idx < 16 * LDI; idx += nth) {
-            const int r = idx / LDI, kk = idx % LDI, sb = kk & 15;
-            int k = 0, tl = 0, de = 0;
-            const int kind = kind_of(r, k, tl, de);
-            float v = 0.f;
-            if (kk < W_ && (sb >> KB) == tl) v = kind == 2 ? 1.f : (kind == 1 ? (((sb >> (KB - 1 - k)) & 1) ? 1.f : -1.f) : 0.f);
-            buf[idx] = from_f32<T>(v);
+    OpX<T> op_;  // row li() of the operand, local buckets 4g + j (bf16: twice, OpX)
+    __device__ __forceinline__ void init() {
+        int k = 0, tl = 0, de = 0;
+        const int kind = kind_of(li(), k, tl, de);
+        float v[8];
+        f32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int sb = 4 * lg() + j;
+            const float c = kind == 2 ? 1.f : (kind == 1 ? (((sb >> (KB - 1 - k)) & 1) ? 1.f : -1.f) : 0.f);
+            v[j] = v[j + 4] = w[j] = (sb >> KB) == tl ? c : 0.f;
         }
-        a = buf;
-    }
-    OpX<T> op_;  // in registers after cache()
-    __device__ __forceinline__ void cache() {
         if constexpr (is_bf16<T>())
-            op_.f = ld_frag_pi(a + li() * LDI);
+            op_.f = frag_pi_from<T>(v);
         else
-            op_.f = ld_frag16(a + li() * LDI);
+            op_.f = frag16_acc<T>(w);
+        pin(op_.f);
     }
     __device__ __forceinline__ OpX<T> op() const { return op_; }
 };
@@ -1122,10 +1168,10 @@ __device__ void softhash_share(const f32x4 (&P)[2], const f32x4 (&dP)[2], const 
 // the table's waves is split between two neighbouring lanes (half the waves
 // each, in order) and joined with a DPP swap, so every wave of the workgroup
 // takes part and the dependent chain of LDS reads is half as long.
-template <int KB, typename T, int SP, int NTH, bool PAIR = false>
+template <int KB, typename T, int SP, int NTH, bool PAIR = false, int NC = NCOL>
 __device__ float softhash_combine(const float *share, const float *sp, const float *sm, const float *sth, int z, int L,
                                   float inv_temp, T *dproj) {
-    constexpr int LDC = ld_of<float>(NCOL), R = 1 << KB, NW_ = SP / WB;
+    constexpr int LDC = ld_of<float>(NC), R = 1 << KB, NW_ = SP / WB;
     constexpr int NTAB = SP >= R ? SP / R : 1;          // tables (or one table part) in the slice
     constexpr int WPT = (R / WB) < NW_ ? R / WB : NW_;  // waves per table in the slice
     constexpr int SPLIT = WPT % 2 == 0 ? 2 : 1, WPL = WPT / SPLIT, ITEMS = TT * NTAB * KB;
@@ -1149,7 +1195,7 @@ __device__ float softhash_combine(const float *share, const float *sp, const flo
         if (live && half == 0) {
             const int col = (l0 + tl) * KB + k;
             const float th = sth[t * LDC + col];
-            const float du = sx - sd * corner_tanh<PAIR>(sp, sm, t, col);
+            const float du = sx - sd * corner_tanh<PAIR, NC>(sp, sm, t, col);
             tsum += du * th;
             const float dp = du * inv_temp * (1.f - th * th);
             if constexpr (xpart_f32(is_bf16<T>(), SP, KB))
@@ -1189,10 +1235,10 @@ __device__ __forceinline__ void totals_of(const f32x4 (&X)[2], f32x4 &tot) {
 //        = sum_table pd c_k - (sum_table pd) tanh(u_k),  pd = P dP,
 // since sum_table P c_k = sigmoid(2u_k) - sigmoid(-2u_k) = tanh(u_k) (= sp - sm);
 //   dproj = du * inv_temp * (1 - th^2).
-template <int KB, typename T, bool PAIR = false>
+template <int KB, typename T, bool PAIR, int NC>
 __device__ float softhash_bwd(const f32x4 (&P)[2], const f32x4 (&dP)[2], const float *sp, const float *sm,
                               const float *sth, int sw, int L, float inv_temp, T *dproj, const HashOps<T, KB> &ho) {
-    constexpr int LDC = ld_of<float>(NCOL);
+    constexpr int LDC = ld_of<float>(NC);
     const int g = lg(), i = li(), l0 = sw >> KB;
     const OpX<T> A = ho.op();
     // the corner rows' tanh(u) = sp - sm and th, read ahead of the products
@@ -1207,7 +1253,7 @@ __device__ float softhash_bwd(const f32x4 (&P)[2], const f32x4 (&dP)[2], const f
             const int l = l0 + tl, c = l < L ? l * KB + k : 0, t = 16 * nt + i;
             tu[nt][e] = th[nt][e] = 0.f;
             if (kind == 1) {
-                tu[nt][e] = corner_tanh<PAIR>(sp, sm, t, c);
+                tu[nt][e] = corner_tanh<PAIR, NC>(sp, sm, t, c);
                 th[nt][e] = sth[t * LDC + c];
             }
         }
@@ -1276,11 +1322,21 @@ template <int N> __device__ __forceinline__ Frag<bf16> ts_operand_tr(const bf16 
 // transposed [D][TT] tile's row d.  bf16 reads it from the natural rows with
 // two LDS transpose loads: lane (g, p) reads columns 16 md + 4(p & 3) .. +3 of
 // row 4g + (p >> 2) (and row 16 + ...), runs of 4 columns that the natural
-// layout keeps contiguous; fp32 reads the transposed rows trn.
-template <typename T, class NL, bool NAT = is_bf16<T>()>
-__device__ __forceinline__ Frag<T> col_operand(const T *nat, const T *trn, int md) {
-    if constexpr (NAT) {
-        static_assert(is_bf16<T>(), "transpose loads of 16-bit elements");
+// layout keeps contiguous; fp32 reads the column's 8 elements one by one (rows
+// of D + 4 floats: conflict-free).  NAT = false: nat holds transposed rows (row
+// d at d * ldp_of(TT)).
+template <typename T, class NL, bool NAT = true>
+__device__ __forceinline__ Frag<T> col_operand(const T *nat, int md) {
+    if constexpr (NAT && !is_bf16<T>()) {
+        const T *p = nat + NL::off(4 * lg(), 16 * md + li());
+        Frag<T> f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f.lo[j] = p[j * NL::LD];
+            f.hi[j] = p[(16 + j) * NL::LD];
+        }
+        return f;
+    } else if constexpr (NAT) {
         typedef short v4s __attribute__((ext_vector_type(4)));
         typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
         const int g = lg(), p = li(), d0 = 16 * md + 4 * (p & 3);
@@ -1297,7 +1353,7 @@ __device__ __forceinline__ Frag<T> col_operand(const T *nat, const T *trn, int m
         }
         return f;
     } else {
-        return ld_frag_pi(trn + (16 * md + li()) * ldp_of<T>(TT));
+        return ld_frag_pi(nat + (16 * md + li()) * ldp_of<T>(TT));
     }
 }
 // token operand of a bucket-row tile pair X that the wave also stores to its
@@ -1463,6 +1519,11 @@ __device__ void dx_store(const T *dproj, const T *plt, T *dst, int64_t st, int64
     }
 }
 
+// Waves per SIMD the backward tile kernels are scheduled for: the causal
+// 128-bucket workgroups run one per CU (2 waves per SIMD, whatever their LDS
+// would allow, at more than 128 registers).
+__host__ __device__ constexpr int bwd_max_waves(int SP, bool causal) { return causal && SP == 128 ? 2 : 8; }
+
 // Workgroups per CU of a backward tile kernel with nw waves and `bytes` of
 // LDS: the kernels need more than 128 VGPRs, so at most 2 waves per SIMD
 // (8 per CU) run, whatever the LDS allows.
@@ -1489,6 +1550,10 @@ template <int NTH> __device__ double block_sum_f64(double v, float *scratch) {
 // state row index of (bucket s, column d)
 __device__ __forceinline__ int64_t sidx(int s, int d) { return (int64_t)s * SROW + d; }
 
+// Waves per SIMD that the forward tile kernels are compiled for: their LDS
+// allows this many and more, so the register bound is what decides.
+__host__ __device__ constexpr int fwd_waves(bool bf, int SP) { return bf ? (SP == 128 ? 4 : 3) : 2; }
+
 // =====================================================================
 // k_fwd_reduce: per-segment (A, B) sums (fp64 over fp32 tile sums).
 // =====================================================================
@@ -1496,20 +1561,21 @@ __device__ __forceinline__ int64_t sidx(int s, int d) { return (int64_t)s * SROW
 // committed (the 4 GT projection tasks then spread over the waves) and one
 // after the projections; V^T and the key weights alternate between two
 // buffers so the next group's commit can start while waves still read them.
-template <typename T, int SP> struct FwdReduceL {
+template <typename T, int SP, int KB, bool AL> struct FwdReduceL {
+    using PS = PlaneSrc<T, NatL<T, true>, planes_reg<T, SP, AL>()>;
     static constexpr int NW_ = SP / WB;
-    static constexpr int GT = 2;  // tiles per barrier group
-    static constexpr int LDN = NatL<T, true>::LD, LDT = ldp_of<T>(TT), LDC = ld_of<float>(NCOL);
-    static constexpr size_t oK = 0;                                          // [GT][TT][LDN]
-    // V tiles [2][GT]: bf16 natural rows (token operands by transpose loads,
-    // col_operand), fp32 transposed [D][LDT]
-    static constexpr int VTE = is_bf16<T>() ? TT * LDN : D * LDT;  // elements per tile
+    // tiles per barrier group: two for the 8-wave bf16 workgroups; the small
+    // workgroups take one, half the LDS, and run more workgroups per CU
+    static constexpr int GT = is_bf16<T>() && SP == 128 ? 2 : 1;
+    static constexpr int NC = ncol_of<SP, KB>();
+    static constexpr int LDN = NatL<T, true>::LD, LDC = ld_of<float>(NC);
+    static constexpr size_t oK = 0;  // [GT][TT][LDN]
+    // V tiles [2][GT], natural rows (col_operand)
+    static constexpr int VTE = TT * LDN;  // elements per tile
     static constexpr size_t oVt = align16(oK + sizeof(T) * GT * TT * LDN);
-    static constexpr size_t oPl = align16(oVt + sizeof(T) * 2 * GT * VTE);
-    static constexpr size_t oPlLo = align16(oPl + sizeof(T) * NCOL * LDN);
-    static constexpr size_t oSig = align16(oPlLo + sizeof(T) * NCOL * LDN);  // [GT][sp, sm][TT][LDC]
-    static constexpr size_t oCst = align16(oSig + sizeof(float) * GT * 2 * TT * LDC);
-    static constexpr size_t oTok = align16(oCst + Consts<T>::bytes);  // key weights [2][GT][2 * TT]
+    static constexpr size_t oSig = align16(oVt + sizeof(T) * 2 * GT * VTE);  // [GT][sp, sm][TT][LDC]
+    static constexpr size_t oPl = align16(oSig + sizeof(float) * GT * 2 * TT * LDC);
+    static constexpr size_t oTok = align16(oPl + PS::lds_bytes);  // key weights [2][GT][2 * TT]
     static constexpr size_t bytes = align16(oTok + sizeof(float) * 2 * GT * 2 * TT);
 };
 
@@ -1518,29 +1584,17 @@ template <typename T, int SP> struct FwdReduceL {
 // subtracts exactly these values (same operands, same instructions) from the
 // fp64 state to walk it backwards; bf16 accumulates B in fp32 MFMA
 // accumulators instead (k_fwd_reduce adds, k_bwd_out subtracts).
-template <typename T>
-__device__ __forceinline__ void tile_sums(const Frag<T> &Pf, const Consts<T> &cst, const T *sVt, f32x4 &tot,
-                                          f32x4 (&dB)[4]) {
-    constexpr int LDT = ldp_of<T>(TT);
-    tot = zero4();
-    mma(tot, Pf, cst.ones());
-#pragma unroll
-    for (int md = 0; md < 4; ++md) {
-        dB[md] = zero4();
-        mma(dB[md], ld_frag_pi(sVt + (16 * md + li()) * LDT), Pf);
-    }
-}
-// bf16: the same sums from a V tile that col_operand reads (natural rows nat
-// or transposed rows trn, per VL), with HL the lo part Pl of P_K added
-template <class VL, bool HL>
-__device__ __forceinline__ void tile_sums_bf(const Frag<bf16> &Pf, const Frag<bf16> &Pl, const Consts<bf16> &cst,
-                                             const bf16 *nat, const bf16 *trn, f32x4 &tot, f32x4 (&dB)[4]) {
+// V is a tile that col_operand reads (rows per VL); HL adds the lo part Pl of
+// P_K (bf16).
+template <class VL, bool HL, typename T>
+__device__ __forceinline__ void tile_sums(const Frag<T> &Pf, const Frag<T> &Pl, const Consts<T> &cst, const T *sV,
+                                          f32x4 &tot, f32x4 (&dB)[4]) {
     tot = zero4();
     mma(tot, Pf, cst.ones());
     if constexpr (HL) mma(tot, Pl, cst.ones());
 #pragma unroll
     for (int md = 0; md < 4; ++md) {
-        const Frag<bf16> vo = col_operand<bf16, VL>(nat, trn, md);
+        const Frag<T> vo = col_operand<T, VL>(sV, md);
         dB[md] = zero4();
         mma(dB[md], vo, Pf);
         if constexpr (HL) mma(dB[md], vo, Pl);
@@ -1548,23 +1602,22 @@ __device__ __forceinline__ void tile_sums_bf(const Frag<bf16> &Pf, const Frag<bf
 }
 
 template <typename T, int SP, int KB, bool AL = false>
-__global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
+__global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k_fwd_reduce(Args a) {
     if (a.inv_temp_ptr) a.inv_temp = *a.inv_temp_ptr;  // uniform scalar load
-    using Ly = FwdReduceL<T, SP>;
+    using Ly = FwdReduceL<T, SP, KB, AL>;
     using NL = NatL<T, true>;
     constexpr bool PR = pair_tables<KB>();  // K's sigmoid rows as pair products
     using VL = TrL<T>;                      // V rows: read only by transpose loads
-    static_assert(!is_bf16<T>() || TrL<T>::LD <= NatL<T, true>::LD, "V rows within the tile buffer");
-    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDC = Ly::LDC, LDT = ldp_of<T>(TT), LDN = Ly::LDN, GT = Ly::GT;
+    static_assert(TrL<T>::LD <= NatL<T, true>::LD, "V rows within the tile buffer");
+    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDC = Ly::LDC, LDN = Ly::LDN, GT = Ly::GT, NC = Ly::NC;
     __shared__ __align__(16) unsigned char smem[Ly::bytes];
     T *sK = (T *)(smem + Ly::oK), *sVt0 = (T *)(smem + Ly::oVt);
-    T *sPl = (T *)(smem + Ly::oPl), *sPlLo = (T *)(smem + Ly::oPlLo);
     float *sSig = (float *)(smem + Ly::oSig), *sTok0 = (float *)(smem + Ly::oTok);
-    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<T, KB>());
+    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<KB>());
     if (!wp.live) return;
     const int w = wave_id(), i = li(), g = lg(), sw = WB * w, z = wp.z,
               sg = z * SP + sw;
-    const PlaneBlocks pbk(z, SP, KB, a.L, !sliced<T, KB>());  // projection columns of this slice
+    const PlaneBlocks<NW_> pbk(z, SP, KB, a.L, !sliced<KB>(), NC);  // projection columns of this slice
 
     const int n = wp.n, seg = wp.seg;
     const int m = n / (a.B * a.H);
@@ -1576,14 +1629,9 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
     const float *kwp = a.kw ? a.kw + (int64_t)((n / a.H) % a.B) * a.T : nullptr;  // batch row's key weights
 
     Consts<T> cst;
-    cst.init((T *)(smem + Ly::oCst), NTH);
-    load_planes<T, NTH, NL>(a.planes + m * a.planes_m_stride, a.L * a.K, sPl, is_bf16<T>() ? sPlLo : nullptr, nullptr);
-    __syncthreads();  // the constant tables in LDS; their operands to registers
-    cst.cache();
-    // whole-tile instantiations: each wave has at most one projection task,
-    // the same column block on every tile, whose planes stay in registers
-    PlaneOps<T> pcw;
-    if constexpr (AL) pcw.template load<NL>(sPl, sPlLo, pbk.mc(pbk.task(w)));
+    cst.init();
+    typename Ly::PS pcw;
+    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), (T *)(smem + Ly::oPl));
     // segment sums: A in fp64; B in fp64, except in the whole-tile bf16
     // instantiations' fp32 MFMA accumulators (walk_f64).  Tile sums are added
     // tile by tile in token order.
@@ -1608,8 +1656,8 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
         for (int q = w; q < pbk.tasks() * GT; q += NW_) {
             const int u = pbk.tensor(q), r = pbk.task(q);
             float *sp = sSig + u * 2 * TT * LDC;
-            project_tile<T, NL, PR>(sK + u * TT * LDN, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sp, sp + TT * LDC,
-                                nullptr, (AL && q == w) ? &pcw : nullptr);
+            project_tile<T, NL, PR, NC>(sK + u * TT * LDN, pcw, pbk.mc(r), pbk.half(r), a.inv_temp, sp, sp + TT * LDC,
+                                        nullptr);
         }
         __syncthreads();  // sigmoid rows in LDS
 #pragma unroll
@@ -1619,7 +1667,7 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
             const float *sp = sSig + u * 2 * TT * LDC;
             const T *vt = sVt + u * Ly::VTE;
             f32x4 PK[2];
-            probs_st<KB, AL, PR>(sp, sp + TT * LDC, sg, a.S, tile_rows((int64_t)jt * TT, a.T), PK);
+            probs_st<KB, AL, PR, NC>(sp, sp + TT * LDC, sg, a.S, tile_rows((int64_t)jt * TT, a.T), PK);
             if (kwp)  // P_K' = w_t P_K
                 for (int nt = 0; nt < 2; ++nt) {
                     const float wt = sTok[u * 2 * TT + 16 * nt + i];
@@ -1637,17 +1685,14 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
                 mma(tot, Pf, cst.ones());
                 if constexpr (HL) mma(tot, Pl, cst.ones());
                 for (int md = 0; md < 4; ++md) {
-                    const Frag<T> vo = col_operand<T, VL>(vt, vt, md);
+                    const Frag<T> vo = col_operand<T, VL>(vt, md);
                     mma(accBm[md], vo, Pf);
                     if constexpr (HL) mma(accBm[md], vo, Pl);
                 }
                 for (int e = 0; e < 4; ++e) accA[e] += (double)tot[e];
             } else {
                 f32x4 tot, dB[4];
-                if constexpr (is_bf16<T>())
-                    tile_sums_bf<VL, HL>(Pf, Pl, cst, vt, vt, tot, dB);
-                else
-                    tile_sums<T>(Pf, cst, vt, tot, dB);
+                tile_sums<VL, HL>(Pf, Pl, cst, vt, tot, dB);
                 for (int e = 0; e < 4; ++e) {
                     accA[e] += (double)tot[e];
                     for (int md = 0; md < 4; ++md) accB[md][e] += (double)dB[md][e];
@@ -1681,8 +1726,8 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
             T *sVt = sVt0 + b * GT * Ly::VTE;
 #pragma unroll
             for (int u = 0; u < GT; ++u) {
-                pk[u].template commit<NL>(sK + u * TT * LDN, nullptr);
-                pv[u].template commit<VL>(sVt + u * Ly::VTE, nullptr);
+                pk[u].template commit<NL>(sK + u * TT * LDN);
+                pv[u].template commit<VL>(sVt + u * Ly::VTE);
             }
         };
         if (j0 < j1) {
@@ -1699,7 +1744,7 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
         }
     } else {
         Prefetch<T, NTH, AL> pk_[GT];
-        PrefetchT<T, NTH, 1, AL, !is_bf16<T>()> pv_[GT];
+        Prefetch<T, NTH, AL> pv_[GT];
         TokPre pt_[GT];
         auto issue = [&](int jg) {
 #pragma unroll
@@ -1708,7 +1753,7 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
                 // the segment reloads the segment's last tile (unused)
                 const int64_t t0 = (int64_t)(AL ? min(jg + u, j1 - 1) : jg + u) * TT;
                 pk_[u].issue(kp, a.sk.t, t0, send);
-                pv_[u].issue(0, vp, a.sv.t, t0, send);
+                pv_[u].issue(vp, a.sv.t, t0, send);
                 if (kwp) pt_[u].issue(kwp, nullptr, t0, send);
             }
         };
@@ -1723,9 +1768,8 @@ __global__ __launch_bounds__(threads_of(SP)) void k_fwd_reduce(Args a) {
             wait_vmem();
 #pragma unroll
             for (int u = 0; u < GT; ++u) {
-                pk_[u].template commit<NL>(sK + u * TT * LDN, nullptr);
-                pv_[u].template commit<VL>(0, is_bf16<T>() ? sVt + u * Ly::VTE : nullptr,
-                                           is_bf16<T>() ? nullptr : sVt + u * Ly::VTE);
+                pk_[u].template commit<NL>(sK + u * TT * LDN);
+                pv_[u].template commit<VL>(sVt + u * Ly::VTE);
                 if (kwp) pt_[u].commit(sTok + u * 2 * TT);
             }
             if (jg + GT < j1) issue(jg + GT);
@@ -1777,19 +1821,19 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_fwd_scan(double *fstate, const
 // P_K and B (tile start) to LDS as [.][s] arrays, then computes output tiles
 // over all buckets; the B carry of its buckets stays in registers.
 // =====================================================================
-template <typename T, int SP, bool CAUSAL, bool GN> struct FwdOutL {
-    static constexpr int NW_ = SP / WB;
+template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL> struct FwdOutL {
+    static constexpr int NW_ = SP / WB, NC = ncol_of<SP, KB>();
     // The Q and K tiles live inside the P_K / W region when they fit: they
     // are dead from the projection until the next tile's commit, P_K and W
     // are written after the projection and read before that commit (barriers
     // separate all four steps).  Then they also take the swizzled layout.
     static constexpr bool ALIAS = sw_ld<T, SP>() >= NatL<T, true>::LD;
     using NL = NatL<T, ALIAS>;
-    static constexpr int LDN = NL::LD, LDT = ldp_of<T>(TT), LDC = ld_of<float>(NCOL), LDS_ = sw_ld<T, SP>();
-    // the V tile: natural rows, its token operands read with transpose loads
-    // (bf16 F1), or transposed (fp32, and the global normalisation, whose
-    // registers are at the 4-waves-per-SIMD limit)
-    static constexpr bool VNAT = is_bf16<T>() && !GN;
+    using PS = PlaneSrc<T, NL, planes_reg<T, SP, AL>()>;
+    static constexpr int LDN = NL::LD, LDT = ldp_of<T>(TT), LDC = ld_of<float>(NC), LDS_ = sw_ld<T, SP>();
+    // the V tile: natural rows (col_operand), or transposed (bf16 global
+    // normalisation, whose registers are at the 4-waves-per-SIMD limit)
+    static constexpr bool VNAT = !is_bf16<T>() || !GN;
     static constexpr size_t VTB = VNAT ? sizeof(T) * TT * TrL<T>::LD : sizeof(T) * D * LDT;
     static constexpr size_t oVt = 0;
     static constexpr size_t oSig = align16(oVt + (CAUSAL ? VTB : 0));  // Q sp, Q sm, K sp, K sm
@@ -1801,11 +1845,14 @@ template <typename T, int SP, bool CAUSAL, bool GN> struct FwdOutL {
     static constexpr size_t oK = align16(oQ + sizeof(T) * TT * LDN);
     static constexpr size_t oKEnd = align16(oK + (CAUSAL ? sizeof(T) * TT * LDN : 0));
     static_assert(!ALIAS || oKEnd <= oBT, "Q/K tiles must fit in the P_K / W region");
-    static constexpr size_t oPl = ALIAS ? oEnd : oKEnd;
-    static constexpr size_t oPlLo = align16(oPl + sizeof(T) * NCOL * LDN);
-    static constexpr size_t oCst = align16(oPlLo + sizeof(T) * NCOL * LDN);
+    // Whole 4-bit tiles (QKP in the kernel) keep the Q and K rows apart from the
+    // P_K / W rows all the same, so the next tile's can be committed early
+    static constexpr bool QKP = AL && KB == 4;
+    static constexpr size_t oQ2 = ALIAS ? oEnd : oKEnd;
+    static constexpr size_t oK2 = align16(oQ2 + (QKP ? sizeof(T) * TT * LDN : 0));
     // [NW_][TT] per-wave den shares (GN; non-causal F1 when den is requested)
-    static constexpr size_t oDen = align16(oCst + Consts<T>::bytes);
+    static constexpr size_t oPl = align16(oK2 + (QKP ? sizeof(T) * TT * LDN : 0));
+    static constexpr size_t oDen = align16(oPl + PS::lds_bytes);
     static constexpr size_t bytes1 = align16(oDen + (GN || !CAUSAL ? sizeof(float) * NW_ * TT : 0));
     // causal, when it costs no workgroup per CU (160 KiB of LDS): a second
     // transposed V tile and the tile's Sc^T [t][t'] blocks, computed once
@@ -1822,7 +1869,7 @@ template <typename T, int SP, bool CAUSAL, bool GN> struct FwdOutL {
 // instantiations: this slice's den share, a partial).  GN also divides the
 // tile's numerator by max(den, eps) (sliced: the numerator is the partial).
 template <typename T, int SP, bool CAUSAL, bool GN = false, bool AL = false, class NL = NatL<T, true>,
-          bool VNAT = is_bf16<T>()>
+          bool VNAT = true>
 __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T *Wts, const T *sVt, T *op,
                              int64_t st, int64_t t0, int64_t Tn, T *part, const float *sDen = nullptr,
                              float *den = nullptr, float eps = 0.f) {
@@ -1846,7 +1893,7 @@ __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T
                     if (16 * mt + 4 * g + e > 16 * nt + i) Sc[mt][e] = 0.f;  // keep t' <= t
             }
         }
-        mma(O, col_operand<T, NL, VNAT>(sVt, sVt, md), frag_acc<T>(Sc[0], Sc[1]));
+        mma(O, col_operand<T, NL, VNAT>(sVt, md), frag_acc<T>(Sc[0], Sc[1]));
     }
     const int t = 16 * nt + i;
     if (GN || !CAUSAL ? sDen != nullptr : false) {
@@ -1910,12 +1957,12 @@ template <typename T, int SP> __device__ void fwd_out_partial2(int md, const T *
         mma(O[1], b, ld_frag(pw1 + 32 * kp));
     }
 }
-template <typename T, int SP, bool GN, bool AL = false, class NL = NatL<T, true>, bool VNAT = is_bf16<T>()>
+template <typename T, int SP, bool GN, bool AL = false, class NL = NatL<T, true>, bool VNAT = true>
 __device__ void fwd_out_final(int md, int nt, f32x4 O, const T *sVt, const T *sc, T *op, int64_t st, int64_t t0,
                               int64_t Tn, T *part, const float *sDen, float *den, float eps) {
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li();
-    mma(O, col_operand<T, NL, VNAT>(sVt, sVt, md), ld_frag_pi(sc + (16 * nt + i) * LDT));
+    mma(O, col_operand<T, NL, VNAT>(sVt, md), ld_frag_pi(sc + (16 * nt + i) * LDT));
     const int t = 16 * nt + i;
     if (GN && sDen != nullptr) {
         constexpr int NW_ = SP / WB;
@@ -1940,27 +1987,26 @@ __device__ void fwd_out_final(int md, int nt, f32x4 O, const T *sVt, const T *sc
 // GN: global normalisation (causal only) -- W = P_Q, and the output is
 // divided by den(t) = sum over all buckets of P_Q A_s(t), clamped below at eps.
 template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL = false>
-__global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(Args a) {
+__global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k_fwd_out(Args a) {
     if (a.inv_temp_ptr) a.inv_temp = *a.inv_temp_ptr;  // uniform scalar load
     static_assert(CAUSAL || !GN, "global normalisation is causal only");
-    using Ly = FwdOutL<T, SP, CAUSAL, GN>;
+    using Ly = FwdOutL<T, SP, CAUSAL, KB, GN, AL>;
     using NL = typename Ly::NL;
     constexpr bool VNAT = Ly::VNAT;
     constexpr bool PR = pair_tables<KB>();  // Q's and K's sigmoid rows as pair products
     constexpr bool HL = hl_ops<T, SP, KB>();  // P_K as a hi + lo pair
     using VL = TrL<T>;                      // V rows (VNAT): read only by transpose loads
-    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDT = Ly::LDT, LDC = Ly::LDC, LDS_ = Ly::LDS_;
+    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDT = Ly::LDT, LDC = Ly::LDC, NC = Ly::NC;
     __shared__ __align__(16) unsigned char smem[Ly::bytes];
     T *sQ = (T *)(smem + Ly::oQ), *sK = (T *)(smem + Ly::oK), *sVt = (T *)(smem + Ly::oVt);
     T *sPts = (T *)(smem + Ly::oPts), *sWts = (T *)(smem + Ly::oWts), *sBT = (T *)(smem + Ly::oBT);
-    T *sPl = (T *)(smem + Ly::oPl), *sPlLo = (T *)(smem + Ly::oPlLo);
     float *sSig = (float *)(smem + Ly::oSig);
     float *sSpQ = sSig, *sSmQ = sSig + TT * LDC, *sSpK = sSig + 2 * TT * LDC, *sSmK = sSig + 3 * TT * LDC;
-    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<T, KB>());
+    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<KB>());
     if (!wp.live) return;
     const int w = wave_id(), g = lg(), i = li(), sw = WB * w, z = wp.z,
               sg = z * SP + sw;
-    const PlaneBlocks pbk(z, SP, KB, a.L, !sliced<T, KB>());  // projection columns of this slice
+    const PlaneBlocks<NW_> pbk(z, SP, KB, a.L, !sliced<KB>(), NC);  // projection columns of this slice
 
     const int n = wp.n, seg = wp.seg;
     const int m = n / (a.B * a.H);
@@ -1971,22 +2017,17 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
     const T *kp = (const T *)a.k + stream_off(a.sk, n, a.B, a.H);
     const T *vp = (const T *)a.v + stream_off(a.sv, n, a.B, a.H);
     T *op = (T *)a.out + stream_off(a.so, n, a.B, a.H);
-    T *opart = sliced<T, KB>() ? (T *)a.opart + ((int64_t)z * a.M * a.B * a.H + n) * a.T * D : nullptr;
+    T *opart = sliced<KB>() ? (T *)a.opart + ((int64_t)z * a.M * a.B * a.H + n) * a.T * D : nullptr;
     const bool want_den = GN || (!CAUSAL && a.den);
     float *sDen = want_den ? (float *)(smem + Ly::oDen) : nullptr;
     float *denp = !want_den       ? nullptr
-                  : sliced<T, KB>() ? a.denpart + ((int64_t)z * a.M * a.B * a.H + n) * a.T
+                  : sliced<KB>() ? a.denpart + ((int64_t)z * a.M * a.B * a.H + n) * a.T
                                     : a.den + (int64_t)n * a.T;
 
     Consts<T> cst;
-    cst.init((T *)(smem + Ly::oCst), NTH);
-    load_planes<T, NTH, NL>(a.planes + m * a.planes_m_stride, a.L * a.K, sPl, is_bf16<T>() ? sPlLo : nullptr, nullptr);
-    __syncthreads();  // the constant tables in LDS; their operands to registers
-    cst.cache();
-    // whole-tile instantiations: each wave has at most one projection task,
-    // the same column block on every tile, whose planes stay in registers
-    PlaneOps<T> pcw;
-    if constexpr (AL) pcw.template load<NL>(sPl, sPlLo, pbk.mc(pbk.task(w)));
+    cst.init();
+    typename Ly::PS pcw;
+    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), (T *)(smem + Ly::oPl));
     // carried state: causal = prefix at the segment start, non-causal = totals.
     // B in bucket-row layout: lane holds B[s = sw + 4g + e][d = 16md + i]
     const double *st = a.fstate + ((int64_t)n * (a.fnseg + 1) + (CAUSAL ? seg * a.fmul : a.fnseg)) * a.Spad * SROW;
@@ -2002,18 +2043,13 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
     Prefetch<T, NTH, AL> pq_, pk_;
     // V: plain rows read by transpose loads (VNAT; staged row by row, 16
     // lanes per row, conflict-free) or transposed rows
-    std::conditional_t<VNAT, Prefetch<T, NTH, AL>, PrefetchT<T, NTH, 1, AL, true>> pv_;
-    auto v_issue = [&](int64_t t0) {
-        if constexpr (VNAT)
-            pv_.issue(vp, a.sv.t, t0, a.T);
-        else
-            pv_.issue(0, vp, a.sv.t, t0, a.T);
-    };
+    std::conditional_t<VNAT, Prefetch<T, NTH, AL>, PrefetchT<bf16, NTH, AL>> pv_;
+    auto v_issue = [&](int64_t t0) { pv_.issue(vp, a.sv.t, t0, a.T); };
     auto v_commit = [&](T *buf) {
         if constexpr (VNAT)
-            pv_.template commit<VL>(buf, nullptr);
+            pv_.template commit<VL>(buf);
         else
-            pv_.template commit<NL>(0, nullptr, buf);
+            pv_.commit(buf);
     };
     if (j0 < j1) {
         pq_.issue(qp, a.sq.t, (int64_t)j0 * TT, a.T);
@@ -2027,28 +2063,25 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
         // rows, barrier, Sc blocks and the carried-state part of O, barrier,
         // then the next tile's rows (Q/K alias the P_K / W rows, now read;
         // V^T goes to the other buffer) and the rest of O.
-        // Whole 4-bit tiles (QKP; F1 and the global normalisation): every
-        // wave's planes are in registers, so Q and K take the planes' rows
-        // instead (same layout and size: NCOL = TT rows).  The next tile's rows are then committed in the third
+        // Whole 4-bit tiles (QKP; F1 and the global normalisation): Q and K
+        // have rows of their own.  The next tile's rows are then committed in the third
         // phase (this tile's projections are done by then), and the next
         // tile's projections run at the end of the last phase, after the
         // output tiles: three barriers per tile (probabilities and rows,
         // barrier, Sc blocks, carried-state part of O and the next rows'
         // commit, barrier, the rest of O and the next projections, barrier).
-        constexpr bool QKP = AL && KB == 4;
-        static_assert(NCOL == TT, "Q and K rows in the planes' rows");
+        constexpr bool QKP = Ly::QKP;
         if constexpr (QKP) {
-            sQ = sPl;
-            sK = sPlLo;
-            __syncthreads();  // every wave has read its planes
+            sQ = (T *)(smem + Ly::oQ2);
+            sK = (T *)(smem + Ly::oK2);
         }
         T *sSc = (T *)(smem + Ly::oSc);
         zero_lds<T>(sSc, TT * LDT, NTH);  // its (t < 16 <= t') block stays zero
         auto vt_of = [&](int j) { return (T *)(smem + ((j & 1) ? Ly::oVt2 : Ly::oVt)); };
         auto commit = [&](int j) {  // the prefetched rows, V^T to the buffer of tile j
             wait_vmem();
-            pq_.template commit<NL>(sQ, nullptr);
-            pk_.template commit<NL>(sK, nullptr);
+            pq_.template commit<NL>(sQ);
+            pk_.template commit<NL>(sK);
             v_commit(vt_of(j));
         };
         // The rows of tile j + 1 are loaded from the commit of tile j on
@@ -2069,8 +2102,8 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
             if (2 * pbk.tasks() >= NW_ || w < 2 * pbk.tasks()) {
                 const bool isq = w < pbk.tasks();
                 const int r = pbk.task(w);
-                project_tile<T, NL, PR>(isq ? sQ : sK, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, isq ? sSpQ : sSpK,
-                                        isq ? sSmQ : sSmK, nullptr, &pcw);
+                project_tile<T, NL, PR, NC>(isq ? sQ : sK, pcw, pbk.mc(r), pbk.half(r), a.inv_temp, isq ? sSpQ : sSpK,
+                                            isq ? sSmQ : sSmK, nullptr);
             }
         };
         if constexpr (QKP) {
@@ -2093,20 +2126,17 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
                 __syncthreads();
                 for (int q = w; q < 2 * pbk.tasks(); q += NW_) {
                     const int r = pbk.task(q);
-                    if (q < pbk.tasks())
-                        project_tile<T, NL, PR>(sQ, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpQ, sSmQ, nullptr,
-                                                (AL && q == w) ? &pcw : nullptr);
-                    else
-                        project_tile<T, NL, PR>(sK, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpK, sSmK, nullptr,
-                                                (AL && q == w) ? &pcw : nullptr);
+                    const bool isq = q < pbk.tasks();
+                    project_tile<T, NL, PR, NC>(isq ? sQ : sK, pcw, pbk.mc(r), pbk.half(r), a.inv_temp,
+                                                isq ? sSpQ : sSpK, isq ? sSmQ : sSmK, nullptr);
                 }
             }
             __syncthreads();
             f32x4 PQ[2], PK[2], Acum[2], W[2], tot;
             Frag<T> Pf, Pl;  // Pl: the lo part of P_K (HL)
-            probs_st<KB, AL, PR>(sSpQ, sSmQ, sg, a.S, jt + 1 < ntiles ? TT : lastv, PQ);
+            probs_st<KB, AL, PR, NC>(sSpQ, sSmQ, sg, a.S, jt + 1 < ntiles ? TT : lastv, PQ);
             if constexpr (CAUSAL) {
-                probs_st<KB, AL, PR>(sSpK, sSmK, sg, a.S, jt + 1 < ntiles ? TT : lastv, PK);
+                probs_st<KB, AL, PR, NC>(sSpK, sSmK, sg, a.S, jt + 1 < ntiles ? TT : lastv, PK);
                 Pf = store_ts_operand<T, SP>(sPts, sw, PK, cst);
                 if constexpr (HL) {
                     f32x4 R[2];
@@ -2166,7 +2196,7 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
             }
             // carry: B[s][d] += sum_t P_K[t][s] V[t][d]
             for (int md = 0; md < 4; ++md) {
-                const Frag<T> vo = col_operand<T, VL, VNAT>(sVt, sVt, md);
+                const Frag<T> vo = col_operand<T, VL, VNAT>(sVt, md);
                 mma(Bc[md], Pf, vo);
                 if constexpr (HL) mma(Bc[md], Pl, vo);
             }
@@ -2198,9 +2228,9 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
     for (int jt = j0; jt < j1; ++jt) {
         const int64_t t0 = (int64_t)jt * TT;
         __syncthreads();  // previous tile's readers of sVt / sPts / sWts / sBT are done
-        pq_.template commit<NL>(sQ, nullptr);
+        pq_.template commit<NL>(sQ);
         if constexpr (CAUSAL) {
-            pk_.template commit<NL>(sK, nullptr);
+            pk_.template commit<NL>(sK);
             v_commit(sVt);
         }
         if (jt + 1 < j1) {
@@ -2213,19 +2243,16 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
         __syncthreads();
         for (int q = w; q < (CAUSAL ? 2 : 1) * pbk.tasks(); q += NW_) {
             const int r = pbk.task(q);
-            if (q < pbk.tasks())
-                project_tile<T, NL, PR>(sQ, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpQ, sSmQ, nullptr,
-                                    (AL && q == w) ? &pcw : nullptr);
-            else
-                project_tile<T, NL, PR>(sK, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpK, sSmK, nullptr,
-                                    (AL && q == w) ? &pcw : nullptr);
+            const bool isq = q < pbk.tasks();
+            project_tile<T, NL, PR, NC>(isq ? sQ : sK, pcw, pbk.mc(r), pbk.half(r), a.inv_temp, isq ? sSpQ : sSpK,
+                                        isq ? sSmQ : sSmK, nullptr);
         }
         __syncthreads();
         f32x4 PQ[2], PK[2], Acum[2], W[2], tot;
         Frag<T> Pf, Pl;  // Pl: the lo part of P_K (HL)
-        probs_st<KB, AL, PR>(sSpQ, sSmQ, sg, a.S, jt + 1 < ntiles ? TT : lastv, PQ);
+        probs_st<KB, AL, PR, NC>(sSpQ, sSmQ, sg, a.S, jt + 1 < ntiles ? TT : lastv, PQ);
         if constexpr (CAUSAL) {
-            probs_st<KB, AL, PR>(sSpK, sSmK, sg, a.S, jt + 1 < ntiles ? TT : lastv, PK);
+            probs_st<KB, AL, PR, NC>(sSpK, sSmK, sg, a.S, jt + 1 < ntiles ? TT : lastv, PK);
             if constexpr (HL) {
                 f32x4 R[2];
                 lo_rem(PK, R);
@@ -2282,7 +2309,7 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
         if constexpr (CAUSAL) {
             // carry: B[s][d] += sum_t P_K[t][s] V[t][d]
             for (int md = 0; md < 4; ++md) {
-                const Frag<T> vo = col_operand<T, VL, VNAT>(sVt, sVt, md);
+                const Frag<T> vo = col_operand<T, VL, VNAT>(sVt, md);
                 mma(Bc[md], Pf, vo);
                 if constexpr (HL) mma(Bc[md], Pl, vo);
             }
@@ -2311,35 +2338,30 @@ __global__ __launch_bounds__(threads_of(SP), SP == 128 ? 4 : 1) void k_fwd_out(A
 // (GS) take it from a pre-pass: the same kernel with GP set walks the tiles
 // as far as G and writes its slice's share of S_t; k_gn_terms adds the
 // shares and writes rd and gd per token for the second pass and k_bwd_out.
-template <typename T, int KB> __host__ __device__ constexpr bool gn_own_gd() { return !sliced<T, KB>(); }
+template <typename T, int KB> __host__ __device__ constexpr bool gn_own_gd() { return !sliced<KB>(); }
 
-template <typename T, int SP, bool CAUSAL, int KB, bool GN> struct BwdReduceL {
-    static constexpr int NW_ = SP / WB;
-    static constexpr int LDN = NatL<T, true>::LD, LDT = ldp_of<T>(TT), LDC = ld_of<float>(NCOL), LDDP = sw_ld<T, NCOL>();
+template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL> struct BwdReduceL {
+    using PS = PlaneSrc<T, NatL<T, true>, planes_reg<T, SP, AL>()>;
+    static constexpr int NW_ = SP / WB, NC = ncol_of<SP, KB>();
+    static constexpr int LDN = NatL<T, true>::LD, LDC = ld_of<float>(NC), LDDP = sw_ld<T, NCOL>();
     static constexpr bool GS = GN && !gn_own_gd<T, KB>();  // gd per token from k_gn_terms
     static constexpr bool GC = GN && gn_own_gd<T, KB>();   // gd from this kernel's own sums
-    // token block: one tile's staged rows (Q, K, V, dO natural; V, dO
-    // transposed; GN: (den, dden) [2][TT], GS (den, gd); non-causal: dden [TT])
+    // token block: one tile's staged rows (Q, K, V, dO; GN: (den, dden)
+    // [2][TT], GS (den, gd); non-causal: dden [TT])
     static constexpr size_t oQ = 0;
     static constexpr size_t oK = align16(oQ + sizeof(T) * TT * LDN);
     static constexpr size_t oV = align16(oK + (CAUSAL ? sizeof(T) * TT * LDN : 0));
     static constexpr size_t oG = align16(oV + (CAUSAL ? sizeof(T) * TT * LDN : 0));
-    static constexpr size_t oVt = align16(oG + sizeof(T) * TT * LDN);
-    static constexpr size_t oGt = align16(oVt + (CAUSAL ? sizeof(T) * D * LDT : 0));
-    static constexpr size_t oTokIn = align16(oGt + sizeof(T) * D * LDT);
+    static constexpr size_t oTokIn = align16(oG + sizeof(T) * TT * LDN);
     static constexpr size_t TB = align16(oTokIn + (GN || !CAUSAL ? sizeof(float) * 2 * TT : 0));
     // the rest, relative to its start
-    static constexpr size_t rX = 0;  // (the in-tile v.g^T blocks live in each wave's registers)
-    static constexpr size_t rDproj = rX;
-    static constexpr size_t rPl = align16(rDproj + sizeof(T) * TT * LDDP);
-    static constexpr size_t rPlLo = align16(rPl + sizeof(T) * NCOL * LDN);
-    static constexpr size_t rPlT = align16(rPlLo + sizeof(T) * NCOL * LDN);
-    static constexpr size_t rSig = align16(rPlT + sizeof(T) * D * LDDP);  // Q sp, Q sm, Q th, K sp, K sm
-    static constexpr size_t rRed = align16(rSig + sizeof(float) * 5 * TT * LDC);
-    static constexpr size_t rCst = align16(rRed + sizeof(float) * 64 * NW_);
-    static constexpr size_t rHash = align16(rCst + Consts<T>::bytes);
-    static constexpr size_t rPair = align16(rHash + HashOps<T, 4>::bytes);
-    static constexpr size_t rShare = align16(rPair + PairOps<T>::bytes);
+    static constexpr size_t rDproj = 0;
+    static constexpr size_t rPlT = align16(rDproj + sizeof(T) * TT * LDDP);
+    static constexpr size_t rPl = align16(rPlT + sizeof(T) * D * LDDP);
+    static constexpr size_t rSig = align16(rPl + PS::lds_bytes);  // Q sp, Q sm, Q th, K sp, K sm
+    // the end-of-kernel block sum's scratch reuses the sigmoid rows
+    static constexpr size_t rRed = rSig;
+    static constexpr size_t rShare = align16(rSig + sizeof(float) * (CAUSAL ? 5 : 3) * TT * LDC);
     static constexpr size_t rTok = align16(rShare + (KB > 4 ? WideHash<T, KB>::bytes(NW_) : 0));
     // GN (GC, and GS's pre-pass): the waves' shares of sum_s P_Q G [NW_][TT]
     static constexpr size_t rGs = rTok;
@@ -2350,8 +2372,7 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN> struct BwdReduceL {
     static constexpr size_t LDS_CU = 160 * 1024;
     static constexpr int NB = bwd_wgs_per_cu(NW_, 2 * TB + rEnd) >= bwd_wgs_per_cu(NW_, TB + rEnd) ? 2 : 1;
     static constexpr size_t R0 = NB * TB;
-    static constexpr size_t oX = R0 + rX, oDproj = R0 + rDproj, oPl = R0 + rPl, oPlLo = R0 + rPlLo, oPlT = R0 + rPlT,
-                            oSig = R0 + rSig, oRed = R0 + rRed, oCst = R0 + rCst, oHash = R0 + rHash, oPair = R0 + rPair,
+    static constexpr size_t oDproj = R0 + rDproj, oPlT = R0 + rPlT, oPl = R0 + rPl, oSig = R0 + rSig, oRed = R0 + rRed,
                             oShare = R0 + rShare, oGs = R0 + rGs;
     static constexpr size_t bytes = R0 + rEnd;
 };
@@ -2362,10 +2383,11 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN> struct BwdReduceL {
 // dA = gd P_Q.  GP: the GS pre-pass, which writes this slice's share of
 // sum_s P_Q G per token (gsum) and nothing else.
 template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL = false, bool GP = false>
-__global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
+__global__ __launch_bounds__(threads_of(SP)) __attribute__((amdgpu_waves_per_eu(2, bwd_max_waves(SP, CAUSAL))))
+void k_bwd_reduce(Args a) {
     if (a.inv_temp_ptr) a.inv_temp = *a.inv_temp_ptr;  // uniform scalar load
     static_assert(CAUSAL || !GN, "global normalisation is causal only");
-    using Ly = BwdReduceL<T, SP, CAUSAL, KB, GN>;
+    using Ly = BwdReduceL<T, SP, CAUSAL, KB, GN, AL>;
     using NL = NatL<T, true>;
     // K's sigmoid rows as pair products, as in the forward kernels (the walk of
     // the forward state needs the same P_K); Q's stay corner pairs, which its
@@ -2374,10 +2396,10 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
     constexpr bool HL = hl_ops<T, SP, KB>();  // P_K and W as hi + lo pairs
     constexpr bool GS = Ly::GS, GC = Ly::GC;   // GN: gd read per token / from this kernel's sums
     static_assert(!GP || GS, "the pre-pass is the bucket-slice instantiations'");
-    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDN = Ly::LDN, LDT = Ly::LDT, LDC = Ly::LDC, LDDP = Ly::LDDP;
+    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDC = Ly::LDC, LDDP = Ly::LDDP, NC = Ly::NC;
     __shared__ __align__(16) unsigned char smem[Ly::bytes];
     // this tile's token block (block jt & 1 of two; block 0 of one)
-    T *sQ, *sK, *sV, *sG, *sVt, *sGt;
+    T *sQ, *sK, *sV, *sG;
     float *sTokIn;
     auto use_block = [&](int b) {
         unsigned char *tb = smem + b * Ly::TB;
@@ -2385,20 +2407,17 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
         sK = (T *)(tb + Ly::oK);
         sV = (T *)(tb + Ly::oV);
         sG = (T *)(tb + Ly::oG);
-        sVt = (T *)(tb + Ly::oVt);
-        sGt = (T *)(tb + Ly::oGt);
         sTokIn = (float *)(tb + Ly::oTokIn);
     };
-    T *sDproj = (T *)(smem + Ly::oDproj);
-    T *sPl = (T *)(smem + Ly::oPl), *sPlLo = (T *)(smem + Ly::oPlLo), *sPlT = (T *)(smem + Ly::oPlT);
+    T *sDproj = (T *)(smem + Ly::oDproj), *sPlT = (T *)(smem + Ly::oPlT);
     float *sSig = (float *)(smem + Ly::oSig), *sRed = (float *)(smem + Ly::oRed);
     float *sSpQ = sSig, *sSmQ = sSig + TT * LDC, *sThQ = sSig + 2 * TT * LDC;
     float *sSpK = sSig + 3 * TT * LDC, *sSmK = sSig + 4 * TT * LDC;
-    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<T, KB>());
+    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<KB>());
     if (!wp.live) return;
     const int w = wave_id(), g = lg(), i = li(), sw = WB * w, z = wp.z,
               sg = z * SP + sw;
-    const PlaneBlocks pbk(z, SP, KB, a.L, !sliced<T, KB>());  // projection columns of this slice
+    const PlaneBlocks<NW_> pbk(z, SP, KB, a.L, !sliced<KB>(), NC);  // projection columns of this slice
 
     const int n = wp.n, seg = wp.seg;
     const int m = n / (a.B * a.H);
@@ -2412,7 +2431,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
     T *dqp = (T *)a.dq + stream_off(a.sg, n, a.B, a.H);
     constexpr int XC = xcols_of(SP, KB);
     constexpr bool XF = xpart_f32(is_bf16<T>(), SP, KB);
-    void *xpart = sliced<T, KB>() ? xpart_at<T, SP, KB>(a.dqpart, z, n, a) : nullptr;
+    void *xpart = sliced<KB>() ? xpart_at<T, SP, KB>(a.dqpart, z, n, a) : nullptr;
     const int xc0 = ((z * SP) >> KB) * KB;  // first projection column of the slice's tables
     float *sGs = (float *)(smem + Ly::oGs);
     const float *denp = GN ? a.den + (int64_t)n * a.T : nullptr;
@@ -2426,26 +2445,20 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
     float *gdw = GC ? a.gden + (int64_t)n * a.T : nullptr;
 
     Consts<T> cst;
-    cst.init((T *)(smem + Ly::oCst), NTH);
+    cst.init();
     HashOps<T, KB> ho;
     WideHash<T, KB> wh;
     float *sShare = (float *)(smem + Ly::oShare);
     if constexpr (KB <= 4)
-        ho.init((T *)(smem + Ly::oHash), NTH);
+        ho.init();
     else
         wh.init(sg);
     PairOps<T> po;
-    po.init((T *)(smem + Ly::oPair), NTH);
-    load_planes<T, NTH, NL>(a.planes + m * a.planes_m_stride, a.L * a.K, sPl, is_bf16<T>() ? sPlLo : nullptr, sPlT);
+    po.init();
+    typename Ly::PS pcw;
+    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), (T *)(smem + Ly::oPl));
+    load_planes_t<T, NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, sPlT);
     zero_lds<T>(sDproj, TT * LDDP, NTH);
-    __syncthreads();  // the constant tables in LDS; their operands to registers
-    cst.cache();
-    if constexpr (KB <= 4) ho.cache();
-    po.cache();
-    // whole-tile instantiations: each wave has at most one projection task,
-    // the same column block on every tile, whose planes stay in registers
-    PlaneOps<T> pcw;
-    if constexpr (AL) pcw.template load<NL>(sPl, sPlLo, pbk.mc(pbk.task(w)));
     // forward state in d-row layout: lane holds B^T[d = 16md + 4g + e][s = sw + i]
     const double *st = a.fstate + ((int64_t)n * (a.fnseg + 1) + (CAUSAL ? seg * a.fmul : a.fnseg)) * a.Spad * SROW;
     f32x4 Bt[4], Ut[4];
@@ -2462,22 +2475,20 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
     CarryA<T> tsum = 0;  // this thread's share of sum du * th
 
     wait_state_loads();
-    constexpr int NP = CAUSAL ? 2 : 1;  // transposed tiles: dO (and V)
-    Prefetch<T, NTH, AL> pq_, pk_;
-    PrefetchT<T, NTH, NP, AL> pg_;  // non-causal dO
-    PrefetchT2<T, NTH, AL, !is_bf16<T>()> pgv_;  // causal dO (first half of the waves) and V
+    Prefetch<T, NTH, AL> pq_, pk_, pg_;  // pg_: non-causal dO
+    Prefetch2<T, NTH, AL> pgv_;          // causal dO (first half of the waves) and V
     TokPre pt_;
     // Writes the prefetched rows to token block b.
     auto commit = [&](int b) {
         unsigned char *tb = smem + b * Ly::TB;
         float *tin = (float *)(tb + Ly::oTokIn);
         wait_vmem();
-        pq_.template commit<NL>((T *)(tb + Ly::oQ), nullptr);
+        pq_.template commit<NL>((T *)(tb + Ly::oQ));
         if constexpr (CAUSAL) {
-            pk_.template commit<NL>((T *)(tb + Ly::oK), nullptr);
-            pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oGt), (T *)(tb + Ly::oV), (T *)(tb + Ly::oVt));
+            pk_.template commit<NL>((T *)(tb + Ly::oK));
+            pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oV));
         } else {
-            pg_.template commit<NL>(0, (T *)(tb + Ly::oG), (T *)(tb + Ly::oGt));
+            pg_.template commit<NL>((T *)(tb + Ly::oG));
         }
         if constexpr (GN) {
             pt_.commit(tin);
@@ -2492,7 +2503,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
             pk_.issue(kp, a.sk.t, (int64_t)j0 * TT, a.T);
             pgv_.issue(gp, a.sdo.t, vp, a.sv.t, (int64_t)j0 * TT, a.T);
         } else {
-            pg_.issue(0, gp, a.sdo.t, (int64_t)j0 * TT, a.T);
+            pg_.issue(gp, a.sdo.t, (int64_t)j0 * TT, a.T);
         }
         if constexpr (GN) {
             pt_.issue(denp, ddp, (int64_t)j0 * TT, a.T);
@@ -2515,7 +2526,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
                 pk_.issue(kp, a.sk.t, tn, a.T);
                 pgv_.issue(gp, a.sdo.t, vp, a.sv.t, tn, a.T);
             } else {
-                pg_.issue(0, gp, a.sdo.t, tn, a.T);
+                pg_.issue(gp, a.sdo.t, tn, a.T);
             }
             if constexpr (GN) {
                 pt_.issue(denp, ddp, tn, a.T);
@@ -2536,11 +2547,10 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
         for (int q = w; q < (CAUSAL ? 2 : 1) * pbk.tasks(); q += NW_) {
             const int r = pbk.task(q);
             if (q < pbk.tasks())
-                project_tile<T, NL>(sQ, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpQ, sSmQ, GP ? nullptr : sThQ,
-                                    (AL && q == w) ? &pcw : nullptr);
+                project_tile<T, NL, false, NC>(sQ, pcw, pbk.mc(r), pbk.half(r), a.inv_temp, sSpQ, sSmQ,
+                                               GP ? nullptr : sThQ);
             else
-                project_tile<T, NL, PR>(sK, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpK, sSmK, nullptr,
-                                    (AL && q == w) ? &pcw : nullptr);
+                project_tile<T, NL, PR, NC>(sK, pcw, pbk.mc(r), pbk.half(r), a.inv_temp, sSpK, sSmK, nullptr);
         }
         // one token block: dQ of the previous tile, from the dproj rows its
         // softmax backward left in LDS, after the projections (they overlap);
@@ -2550,9 +2560,9 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
         __syncthreads();
         f32x4 PQ[2], PK[2], Acum[2], W[2], inv[2], tot;
         Frag<T> Pf, Pl;  // Pl: the lo part of P_K (HL)
-        probs_st<KB, AL>(sSpQ, sSmQ, sg, a.S, jt + 1 < ntiles ? TT : lastv, PQ);
+        probs_st<KB, AL, false, NC>(sSpQ, sSmQ, sg, a.S, jt + 1 < ntiles ? TT : lastv, PQ);
         if constexpr (CAUSAL) {
-            probs_st<KB, AL, PR>(sSpK, sSmK, sg, a.S, jt + 1 < ntiles ? TT : lastv, PK);
+            probs_st<KB, AL, PR, NC>(sSpK, sSmK, sg, a.S, jt + 1 < ntiles ? TT : lastv, PK);
             Pf = token_operand<T>(PK, cst, po);
             if constexpr (HL) {
                 f32x4 R[2];
@@ -2656,12 +2666,12 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
         // U^T[d][s] += sum_t g[t][d] W[t][s]; carry B^T[d][s] += sum_t V[t][d] P_K[t][s]
         for (int md = 0; md < 4; ++md) {
             if constexpr (!GP) {
-                const Frag<T> go = col_operand<T, NL>(sG, sGt, md);
+                const Frag<T> go = col_operand<T, NL>(sG, md);
                 mma(Ut[md], go, Wf);
                 if constexpr (HL) mma(Ut[md], go, Wl);
             }
             if constexpr (CAUSAL) {
-                const Frag<T> vo = col_operand<T, NL>(sV, sVt, md);
+                const Frag<T> vo = col_operand<T, NL>(sV, md);
                 mma(Bt[md], vo, Pf);
                 if constexpr (HL) mma(Bt[md], vo, Pl);
             }
@@ -2699,11 +2709,11 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_reduce(Args a) {
                     if (t < tile_rows(t0, a.T)) gsp[t0 + t] = sq;
                 }
         } else if constexpr (KB <= 4) {
-            tsum += softhash_bwd<KB, T>(PQ, dPQ, sSpQ, sSmQ, sThQ, sg, a.L, a.inv_temp, sDproj, ho);
+            tsum += softhash_bwd<KB, T, false, NC>(PQ, dPQ, sSpQ, sSmQ, sThQ, sg, a.L, a.inv_temp, sDproj, ho);
         } else {
             softhash_share<KB, T>(PQ, dPQ, wh, sShare);
             __syncthreads();
-            tsum += softhash_combine<KB, T, SP, NTH>(sShare, sSpQ, sSmQ, sThQ, z, a.L, a.inv_temp, sDproj);
+            tsum += softhash_combine<KB, T, SP, NTH, false, NC>(sShare, sSpQ, sSmQ, sThQ, z, a.L, a.inv_temp, sDproj);
         }
         // The next tile's rows go to the other token block (its last readers
         // finished before this tile's first barrier), or with one block to it
@@ -2764,28 +2774,26 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_bwd_scan(float *rstate, const 
 // Sc2[t][tau] = sum_s W[t][s] P_K[tau][s], computed as output tiles over all
 // buckets from the waves' [.][s] LDS arrays; dK through each wave's buckets.
 // =====================================================================
-template <typename T, int SP, bool CAUSAL, int KB, bool GN> struct BwdOutL {
-    static constexpr int NW_ = SP / WB;
+template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL> struct BwdOutL {
+    using PS = PlaneSrc<T, NatL<T, true>, planes_reg<T, SP, AL>()>;
+    static constexpr int NW_ = SP / WB, NC = ncol_of<SP, KB>();
     // the configuration of the whole-tile 4-bit instantiation (bf16, 128-bucket
     // slices, causal F1): it projects a tile in the previous tile's last phase,
-    // so K's sigmoid rows are double-buffered, and the transposed V / dO rows,
-    // which bf16 never reads, take no LDS.  (8-bit slices measured faster with
+    // so K's sigmoid rows are double-buffered.  (8-bit slices measured faster with
     // the projections in a phase of their own: only half of their waves have a
     // projection task, and their last phase already ends at the wide-table
     // barrier.)
     static constexpr bool P2L = is_bf16<T>() && SP == 128 && CAUSAL && !GN && KB == 4;
     static constexpr int NSIG = P2L ? 8 : (CAUSAL ? 5 : 3);  // sigmoid row arrays
-    static constexpr int LDN = NatL<T, true>::LD, LDT = ldp_of<T>(TT), LDC = ld_of<float>(NCOL), LDDP = sw_ld<T, NCOL>(),
+    static constexpr int LDN = NatL<T, true>::LD, LDT = ldp_of<T>(TT), LDC = ld_of<float>(NC), LDDP = sw_ld<T, NCOL>(),
                          LDS_ = sw_ld<T, SP>();
-    // token block: one tile's staged rows (K, Q, V, dO natural; V, dO
-    // transposed; GN: rden, gden [2][TT]; non-causal: key weights [TT])
+    // token block: one tile's staged rows (K, Q, V, dO; GN: rden, gden
+    // [2][TT]; non-causal: key weights [TT])
     static constexpr size_t oK = 0;
     static constexpr size_t oQ = align16(oK + sizeof(T) * TT * LDN);
     static constexpr size_t oV = align16(oQ + (CAUSAL ? sizeof(T) * TT * LDN : 0));
     static constexpr size_t oG = align16(oV + sizeof(T) * TT * LDN);
-    static constexpr size_t oVt = align16(oG + (CAUSAL ? sizeof(T) * TT * LDN : 0));
-    static constexpr size_t oGt = align16(oVt + (CAUSAL && !P2L ? sizeof(T) * D * LDT : 0));
-    static constexpr size_t oTok = align16(oGt + (CAUSAL && !P2L ? sizeof(T) * D * LDT : 0));
+    static constexpr size_t oTok = align16(oG + (CAUSAL ? sizeof(T) * TT * LDN : 0));
     static constexpr size_t TB = align16(oTok + (GN || !CAUSAL ? sizeof(float) * 2 * TT : 0));
     // the rest, relative to its start
     static constexpr size_t rX = 0;
@@ -2794,21 +2802,16 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN> struct BwdOutL {
     static constexpr size_t rWts = align16(rPts + sizeof(T) * TT * LDS_);
     static constexpr size_t rUT = align16(rWts + (CAUSAL ? sizeof(T) * TT * LDS_ : 0));
     static constexpr size_t rDproj = align16(rUT + sizeof(T) * D * LDS_);
-    static constexpr size_t rPl = align16(rDproj + sizeof(T) * TT * LDDP);
-    static constexpr size_t rPlLo = align16(rPl + sizeof(T) * NCOL * LDN);
-    static constexpr size_t rPlT = align16(rPlLo + sizeof(T) * NCOL * LDN);
+    static constexpr size_t rPlT = align16(rDproj + sizeof(T) * TT * LDDP);
+    static constexpr size_t rPl = align16(rPlT + sizeof(T) * D * LDDP);
     // K sp, K sm, K th, Q sp, Q sm (P2L: then K sp, K sm, K th of odd tiles)
-    static constexpr size_t rSig = align16(rPlT + sizeof(T) * D * LDDP);
+    static constexpr size_t rSig = align16(rPl + PS::lds_bytes);
     // the end-of-kernel block sum's scratch [64 * NW_] reuses the sigmoid rows
     static_assert(64 * NW_ <= (CAUSAL ? 5 : 3) * TT * LDC, "block-sum scratch inside the sigmoid rows");
     static constexpr size_t rRed = rSig;
-    static constexpr size_t rCst = align16(rSig + sizeof(float) * NSIG * TT * LDC);
-    static constexpr size_t rHash = align16(rCst + Consts<T>::bytes);
-    // causal: Sc2^T [tau][t] of the last tile, for the dV tiles of the next
-    // iteration (with two token blocks)
-    static constexpr size_t rSc2 = align16(rHash + HashOps<T, 4>::bytes);
-    static constexpr size_t rPair = align16(rSc2 + (CAUSAL ? sizeof(T) * TT * LDT : 0));
-    static constexpr size_t rShare = align16(rPair + PairOps<T>::bytes);
+    // causal: Sc2^T [tau][t] of the last tile, for its dV tiles
+    static constexpr size_t rSc2 = align16(rSig + sizeof(float) * NSIG * TT * LDC);
+    static constexpr size_t rShare = align16(rSc2 + (CAUSAL ? sizeof(T) * TT * LDT : 0));
     static constexpr size_t rEnd = align16(rShare + (KB > 4 ? WideHash<T, KB>::bytes(NW_) : 0));
     // two token blocks when they cost no workgroup per CU (160 KiB of LDS):
     // the next tile's rows then go to the other block while this tile still
@@ -2817,9 +2820,8 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN> struct BwdOutL {
     static constexpr int NB = bwd_wgs_per_cu(NW_, 2 * TB + rEnd) >= bwd_wgs_per_cu(NW_, TB + rEnd) ? 2 : 1;
     static constexpr size_t R0 = NB * TB;
     static constexpr size_t oX = R0 + rX, oY = R0 + rY, oPts = R0 + rPts, oWts = R0 + rWts, oUT = R0 + rUT,
-                            oDproj = R0 + rDproj, oPl = R0 + rPl, oPlLo = R0 + rPlLo, oPlT = R0 + rPlT,
-                            oSig = R0 + rSig, oRed = R0 + rRed, oCst = R0 + rCst, oHash = R0 + rHash,
-                            oPair = R0 + rPair, oShare = R0 + rShare, oSc2 = R0 + rSc2;
+                            oDproj = R0 + rDproj, oPlT = R0 + rPlT, oPl = R0 + rPl, oSig = R0 + rSig, oRed = R0 + rRed,
+                            oShare = R0 + rShare, oSc2 = R0 + rSc2;
     static constexpr size_t bytes = R0 + rEnd;
 };
 
@@ -2838,44 +2840,6 @@ template <typename T, int SP> __device__ void sc2_tile(int r, const T *Wts, cons
     store4<T>(sc2 + (16 * nt + i) * LDT + 16 * mt + 4 * g, acc);
 }
 
-template <typename T, int SP, bool CAUSAL, bool AL = false, class NL = NatL<T, true>>
-__device__ void dv_tile(int md, int nt, const T *sUT, const T *Pts, const T *Wts, const T *sG, const T *sGt, T *dvp,
-                        int64_t st,
-                        int64_t t0, int64_t Tn, T *part) {
-    constexpr int LDT = ldp_of<T>(TT);
-    const int g = lg(), i = li();
-    const T *pu = sw_frag_ptr<T, SP>(sUT, 16 * md + i), *pp = sw_frag_ptr<T, SP>(Pts, 16 * nt + i);
-    f32x4 acc = zero4();
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) mma(acc, ld_frag(pu + 32 * kp), ld_frag(pp + 32 * kp));
-    if constexpr (CAUSAL) {
-        f32x4 Sc2[2];
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            Sc2[mt] = zero4();
-            if (mt >= nt) {
-                const T *pw = sw_frag_ptr<T, SP>(Wts, 16 * mt + i);
-#pragma unroll
-                for (int kp = 0; kp < SP / 32; ++kp) mma(Sc2[mt], ld_frag(pw + 32 * kp), ld_frag(pp + 32 * kp));
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (16 * mt + 4 * g + e < 16 * nt + i) Sc2[mt][e] = 0.f;  // keep t >= tau
-            }
-        }
-        mma(acc, col_operand<T, NL>(sG, sGt, md), frag_acc<T>(Sc2[0], Sc2[1]));
-    }
-    const int t = 16 * nt + i;
-    if ((AL || t < tile_rows(t0, Tn))) {
-        if (part)
-            store4<T>(part_at(part, t0, t, 16 * md + 4 * g), acc);
-        else
-            store4<T>(at_bytes(tile_ptr(dvp, st, t0), tile_off(t, st, 16 * md + 4 * g, sizeof(T))), acc);
-    }
-}
-
-// dV tile (md, nt) in two steps: the carried part U P_K (over all buckets,
-// from the U and P_K rows), then, once the tile's Sc2 rows exist (sc2_tile),
-// the in-tile part g^T Sc2 and the store.
 // The d-row carry U^T (lane: [d = 16md + 4g + e][s = sw + i]) as the operand
 // of acc[s][tau] += sum_d U[s][d] v_tau[d]; with HL an fp32-accurate hi + lo
 // pair
@@ -2901,6 +2865,9 @@ template <typename T, bool HL> struct UOps {
         }
     }
 };
+// dV tile (md, nt) in two steps: the part U P_K (over all buckets, from the U
+// and P_K rows: the carried U, or the totals), then (causal) the in-tile part
+// g^T Sc2 once the tile's Sc2 rows exist (sc2_tile), and the store.
 template <typename T, int SP> __device__ f32x4 dv_part(int md, int nt, const T *sUT, const T *Pts) {
     const int i = li();
     const T *pu = sw_frag_ptr<T, SP>(sUT, 16 * md + i), *pp = sw_frag_ptr<T, SP>(Pts, 16 * nt + i);
@@ -2909,13 +2876,12 @@ template <typename T, int SP> __device__ f32x4 dv_part(int md, int nt, const T *
     for (int kp = 0; kp < SP / 32; ++kp) mma(acc, ld_frag(pu + 32 * kp), ld_frag(pp + 32 * kp));
     return acc;
 }
-template <typename T, bool AL = false, class NL = NatL<T, true>>
-__device__ void dv_finish(int md, int nt, f32x4 acc, const T *sG, const T *sGt, const T *sc2, T *dvp, int64_t st,
-                          int64_t t0,
+template <typename T, bool CAUSAL, bool AL = false, class NL = NatL<T, true>>
+__device__ void dv_finish(int md, int nt, f32x4 acc, const T *sG, const T *sc2, T *dvp, int64_t st, int64_t t0,
                           int64_t Tn, T *part) {
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li();
-    mma(acc, col_operand<T, NL>(sG, sGt, md), ld_frag_pi(sc2 + (16 * nt + i) * LDT));
+    if constexpr (CAUSAL) mma(acc, col_operand<T, NL>(sG, md), ld_frag_pi(sc2 + (16 * nt + i) * LDT));
     const int t = 16 * nt + i;
     if ((AL || t < tile_rows(t0, Tn))) {
         if (part)
@@ -2929,10 +2895,11 @@ __device__ void dv_finish(int md, int nt, f32x4 acc, const T *sG, const T *sGt, 
 // token (rd = 1/max(den, eps), gd = dL/d den), so the reverse walk needs
 // neither the forward state nor G.
 template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL = false, bool XW = walk_f64<T, AL>()>
-__global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
+__global__ __launch_bounds__(threads_of(SP)) __attribute__((amdgpu_waves_per_eu(2, bwd_max_waves(SP, CAUSAL))))
+void k_bwd_out(Args a) {
     if (a.inv_temp_ptr) a.inv_temp = *a.inv_temp_ptr;  // uniform scalar load
     static_assert(CAUSAL || !GN, "global normalisation is causal only");
-    using Ly = BwdOutL<T, SP, CAUSAL, KB, GN>;
+    using Ly = BwdOutL<T, SP, CAUSAL, KB, GN, AL>;
     using NL = NatL<T, true>;
     // Q's and K's sigmoid rows as pair products (K's as in the forward kernels:
     // the walk back of the forward state subtracts the same P_K)
@@ -2944,11 +2911,10 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
     // table's buckets share of it).  An 8-bit table's 256 buckets spread W, and
     // the single operand costs it no more than the other roundings do.
     constexpr bool WM = is_bf16<T>() && KB < 8;
-    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDN = Ly::LDN, LDT = Ly::LDT, LDC = Ly::LDC, LDDP = Ly::LDDP,
-                  LDS_ = Ly::LDS_;
+    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDT = Ly::LDT, LDC = Ly::LDC, LDDP = Ly::LDDP, NC = Ly::NC;
     __shared__ __align__(16) unsigned char smem[Ly::bytes];
     // this tile's token block (block jr & 1 of two; block 0 of one)
-    T *sQ, *sK, *sV, *sG, *sVt, *sGt;
+    T *sQ, *sK, *sV, *sG;
     float *sTok;
     auto use_block = [&](int b) {
         unsigned char *tb = smem + b * Ly::TB;
@@ -2956,22 +2922,20 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
         sQ = (T *)(tb + Ly::oQ);
         sV = (T *)(tb + Ly::oV);
         sG = (T *)(tb + Ly::oG);
-        sVt = (T *)(tb + Ly::oVt);
-        sGt = (T *)(tb + Ly::oGt);
         sTok = (float *)(tb + Ly::oTok);
     };
     T *sX = (T *)(smem + Ly::oX), *sY = (T *)(smem + Ly::oY);
     T *sPts = (T *)(smem + Ly::oPts), *sWts = (T *)(smem + Ly::oWts), *sUT = (T *)(smem + Ly::oUT);
     T *sDproj = (T *)(smem + Ly::oDproj), *sSc2 = (T *)(smem + Ly::oSc2);
-    T *sPl = (T *)(smem + Ly::oPl), *sPlLo = (T *)(smem + Ly::oPlLo), *sPlT = (T *)(smem + Ly::oPlT);
+    T *sPlT = (T *)(smem + Ly::oPlT);
     float *sSig = (float *)(smem + Ly::oSig), *sRed = (float *)(smem + Ly::oRed);
     float *sSpK = sSig, *sSmK = sSig + TT * LDC, *sThK = sSig + 2 * TT * LDC;
     float *sSpQ = sSig + 3 * TT * LDC, *sSmQ = sSig + 4 * TT * LDC;
-    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<T, KB>());
+    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<KB>());
     if (!wp.live) return;
     const int w = wave_id(), g = lg(), i = li(), sw = WB * w, z = wp.z,
               sg = z * SP + sw;
-    const PlaneBlocks pbk(z, SP, KB, a.L, !sliced<T, KB>());  // projection columns of this slice
+    const PlaneBlocks<NW_> pbk(z, SP, KB, a.L, !sliced<KB>(), NC);  // projection columns of this slice
 
     const int n = wp.n, seg = wp.seg;
     const int m = n / (a.B * a.H);
@@ -2986,38 +2950,32 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
     T *dvp = (T *)a.dv + stream_off(a.sg, n, a.B, a.H);
     constexpr int XC = xcols_of(SP, KB);
     constexpr bool XF = xpart_f32(is_bf16<T>(), SP, KB);
-    void *xpart = sliced<T, KB>() ? xpart_at<T, SP, KB>(a.dkpart, z, n, a) : nullptr;
+    void *xpart = sliced<KB>() ? xpart_at<T, SP, KB>(a.dkpart, z, n, a) : nullptr;
     const int xc0 = ((z * SP) >> KB) * KB;  // first projection column of the slice's tables
-    T *vpart = sliced<T, KB>() ? (T *)a.dvpart + ((int64_t)z * a.M * a.B * a.H + n) * a.T * D : nullptr;
+    T *vpart = sliced<KB>() ? (T *)a.dvpart + ((int64_t)z * a.M * a.B * a.H + n) * a.T * D : nullptr;
     const float *rdp = GN ? a.rden + (int64_t)n * a.T : nullptr, *gdp = GN ? a.gden + (int64_t)n * a.T : nullptr;
     const float *kwp = !CAUSAL && a.kw ? a.kw + (int64_t)((n / a.H) % a.B) * a.T : nullptr;
 
     Consts<T> cst;
-    cst.init((T *)(smem + Ly::oCst), NTH);
+    cst.init();
     HashOps<T, KB> ho;
     WideHash<T, KB> wh;
     float *sShare = (float *)(smem + Ly::oShare);
     if constexpr (KB <= 4)
-        ho.init((T *)(smem + Ly::oHash), NTH);
+        ho.init();
     else
         wh.init(sg);
     PairOps<T> po;
-    po.init((T *)(smem + Ly::oPair), NTH);
-    load_planes<T, NTH, NL>(a.planes + m * a.planes_m_stride, a.L * a.K, sPl, is_bf16<T>() ? sPlLo : nullptr, sPlT);
+    po.init();
+    typename Ly::PS pcw;
+    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), (T *)(smem + Ly::oPl));
+    load_planes_t<T, NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, sPlT);
     zero_lds<T>(sDproj, TT * LDDP, NTH);
     if constexpr (CAUSAL) {
         zero_lds<T>(sX, TT * LDT, NTH);
         zero_lds<T>(sY, TT * LDT, NTH);
         zero_lds<T>(sSc2, TT * LDT, NTH);  // its (t < 16 <= tau) block stays zero
     }
-    __syncthreads();  // the constant tables in LDS; their operands to registers
-    cst.cache();
-    if constexpr (KB <= 4) ho.cache();
-    po.cache();
-    // whole-tile instantiations: each wave has at most one projection task,
-    // the same column block on every tile, whose planes stay in registers
-    PlaneOps<T> pcw;
-    if constexpr (AL) pcw.template load<NL>(sPl, sPlLo, pbk.mc(pbk.task(w)));
     // reverse carries (U, alpha) after the segment; forward state at the segment end
     const float *rs = a.rstate + ((int64_t)n * a.nseg + seg) * a.Spad * SROW;
     const double *fs =
@@ -3051,19 +3009,19 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
 
     wait_state_loads();
     Prefetch<T, NTH, AL> pq_, pk_, pvn_;  // pvn_: non-causal V (natural only)
-    PrefetchT2<T, NTH, AL, !is_bf16<T>()> pgv_;  // causal dO (first half of the waves) and V
+    Prefetch2<T, NTH, AL> pgv_;                // causal dO (first half of the waves) and V
     TokPre pt_;
     // Writes the prefetched rows to token block b.
     auto commit = [&](int b) {
         unsigned char *tb = smem + b * Ly::TB;
         float *tok = (float *)(tb + Ly::oTok);
         wait_vmem();
-        pk_.template commit<NL>((T *)(tb + Ly::oK), nullptr);
+        pk_.template commit<NL>((T *)(tb + Ly::oK));
         if constexpr (CAUSAL) {
-            pq_.template commit<NL>((T *)(tb + Ly::oQ), nullptr);
-            pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oGt), (T *)(tb + Ly::oV), (T *)(tb + Ly::oVt));
+            pq_.template commit<NL>((T *)(tb + Ly::oQ));
+            pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oV));
         } else {
-            pvn_.template commit<NL>((T *)(tb + Ly::oV), nullptr);
+            pvn_.template commit<NL>((T *)(tb + Ly::oV));
             if (kwp) pt_.commit(tok);
         }
         if constexpr (GN) pt_.commit(tok);
@@ -3073,7 +3031,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
     // iteration, from Sc2 rows computed once in LDS
     constexpr bool SCN = CAUSAL && NB == 2;
     constexpr int NQD = (8 + NW_ - 1) / NW_;  // dV tiles per wave
-    f32x4 dvacc[NQD];                          // SCN: carried part of the last tile's dV tiles
+    f32x4 dvacc[NQD];                          // causal: carried part of the last tile's dV tiles
 #pragma unroll
     for (int k = 0; k < NQD; ++k) dvacc[k] = zero4();
     // Whole 4-bit tiles (P2): two barriers per tile instead of three.  The Q and K
@@ -3092,12 +3050,12 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
     static_assert(!Ly::P2L || !AL || SCN, "the 4-bit whole-tile instantiation runs the two-barrier walk");
     auto commit_qk = [&](int b) {
         unsigned char *tb = smem + b * Ly::TB;
-        pk_.template commit<NL>((T *)(tb + Ly::oK), nullptr);
-        pq_.template commit<NL>((T *)(tb + Ly::oQ), nullptr);
+        pk_.template commit<NL>((T *)(tb + Ly::oK));
+        pq_.template commit<NL>((T *)(tb + Ly::oQ));
     };
     auto commit_vg = [&](int b) {
         unsigned char *tb = smem + b * Ly::TB;
-        pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oGt), (T *)(tb + Ly::oV), (T *)(tb + Ly::oVt));
+        pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oV));
     };
     auto issue_qk = [&](int64_t tq) {
         pk_.issue(kp, a.sk.t, tq, a.T);
@@ -3112,9 +3070,9 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
             const bool isk = w < pbk.tasks();
             const int r = pbk.task(w);
             float *kr = sSig + (par ? 5 : 0) * TT * LDC;
-            project_tile<T, NL, PR>(isk ? (const T *)(tb + Ly::oK) : (const T *)(tb + Ly::oQ), sPl, sPlLo, pbk.mc(r),
-                                    r & 1, a.inv_temp, isk ? kr : sSpQ, isk ? kr + TT * LDC : sSmQ,
-                                    isk ? kr + 2 * TT * LDC : nullptr, &pcw);
+            project_tile<T, NL, PR, NC>(isk ? (const T *)(tb + Ly::oK) : (const T *)(tb + Ly::oQ), pcw, pbk.mc(r),
+                                        pbk.half(r), a.inv_temp, isk ? kr : sSpQ, isk ? kr + TT * LDC : sSmQ,
+                                        isk ? kr + 2 * TT * LDC : nullptr);
         }
     };
     if (P2 && j0 < j1) {
@@ -3173,18 +3131,16 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
                 if (w < 2 * pbk.tasks()) {
                     const bool isk = w < pbk.tasks();
                     const int r = pbk.task(w);
-                    project_tile<T, NL, PR>(isk ? sK : sQ, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp,
-                                            isk ? sSpK : sSpQ, isk ? sSmK : sSmQ, isk ? sThK : nullptr, &pcw);
+                    project_tile<T, NL, PR, NC>(isk ? sK : sQ, pcw, pbk.mc(r), pbk.half(r), a.inv_temp,
+                                                isk ? sSpK : sSpQ, isk ? sSmK : sSmQ, isk ? sThK : nullptr);
                 }
             } else {
                 for (int q = w; q < (CAUSAL ? 2 * pbk.tasks() + (MT2 ? 0 : 3) : pbk.tasks()); q += NW_) {
                     const int r = pbk.task(q);
-                    if (q < pbk.tasks())
-                        project_tile<T, NL, PR>(sK, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpK, sSmK, sThK,
-                                                (AL && q == w) ? &pcw : nullptr);
-                    else if (q < 2 * pbk.tasks())
-                        project_tile<T, NL, PR>(sQ, sPl, sPlLo, pbk.mc(r), r & 1, a.inv_temp, sSpQ, sSmQ, nullptr,
-                                                (AL && q == w) ? &pcw : nullptr);
+                    const bool isk = q < pbk.tasks();
+                    if (q < (CAUSAL ? 2 : 1) * pbk.tasks())
+                        project_tile<T, NL, PR, NC>(isk ? sK : sQ, pcw, pbk.mc(r), pbk.half(r), a.inv_temp,
+                                                    isk ? sSpK : sSpQ, isk ? sSmK : sSmQ, isk ? sThK : nullptr);
                     else
                         m_tile_xy<T, NL>(q - 2 * pbk.tasks(), sV, sG, sX, sY);
                 }
@@ -3201,12 +3157,11 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
             // tile's third barrier)
             if constexpr (SCN)
                 if (jr + 1 < j1) {
-                    const T *gtn = (const T *)(smem + ((jr + 1) & 1) * Ly::TB + Ly::oGt);
                     const T *gnn = (const T *)(smem + ((jr + 1) & 1) * Ly::TB + Ly::oG);
 #pragma unroll
                     for (int k = 0; k < NQD; ++k)
                         if (w + k * NW_ < 8)
-                            dv_finish<T, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], gnn, gtn, sSc2, dvp,
+                            dv_finish<T, CAUSAL, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], gnn, sSc2, dvp,
                                              a.sg.t, t0 + TT, a.T, vpart);
                 }
         }
@@ -3218,12 +3173,11 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
             commit_qk((jr + 1) & 1);
             issue_qk((int64_t)max(jr - 2, j0) * TT);
             if (jr + 1 < j1) {
-                const T *gtn = (const T *)(smem + ((jr + 1) & 1) * Ly::TB + Ly::oGt);
                 const T *gnn = (const T *)(smem + ((jr + 1) & 1) * Ly::TB + Ly::oG);
 #pragma unroll
                 for (int k = 0; k < NQD; ++k)
                     if (w + k * NW_ < 8)
-                        dv_finish<T, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], gnn, gtn, sSc2, dvp, a.sg.t,
+                        dv_finish<T, CAUSAL, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], gnn, sSc2, dvp, a.sg.t,
                                          t0 + TT, a.T, vpart);
             }
         }
@@ -3232,7 +3186,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
         if constexpr (MT2)  // X and Y are read after the next barrier
             for (int q = w; q < 3; q += NW_) m_tile_xy<T, NL>(q, sV, sG, sX, sY);
         f32x4 PKraw[2], PKr[2];  // fp32 P_K (kept for the softmax backward), operand-rounded P_K
-        probs_st<KB, AL, PR>(sSpK, sSmK, sg, a.S, jr + 1 < ntiles ? TT : lastv, PKraw);
+        probs_st<KB, AL, PR, NC>(sSpK, sSmK, sg, a.S, jr + 1 < ntiles ? TT : lastv, PKraw);
         PKr[0] = PKraw[0];
         PKr[1] = PKraw[1];
         float kwt[2] = {1.f, 1.f};  // non-causal key weights: P_K' = w_t P_K
@@ -3265,7 +3219,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
             };
             if constexpr (GN) {
                 f32x4 PQ[2], W[2];
-                probs_st<KB, AL, PR>(sSpQ, sSmQ, sg, a.S, jr + 1 < ntiles ? TT : lastv, PQ);
+                probs_st<KB, AL, PR, NC>(sSpQ, sSmQ, sg, a.S, jr + 1 < ntiles ? TT : lastv, PQ);
                 for (int nt = 0; nt < 2; ++nt) {
                     const float rd = sTok[16 * nt + i], gd = sTok[TT + 16 * nt + i];
                     for (int e = 0; e < 4; ++e) {
@@ -3276,7 +3230,7 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
                 w_operands(W);
             } else {
                 f32x4 PQ[2], Acum[2], W[2], tot, dB[4];
-                probs_st<KB, AL, PR>(sSpQ, sSmQ, sg, a.S, jr + 1 < ntiles ? TT : lastv, PQ);
+                probs_st<KB, AL, PR, NC>(sSpQ, sSmQ, sg, a.S, jr + 1 < ntiles ? TT : lastv, PQ);
                 // forward state at the tile start: end state minus this tile's sums
                 if constexpr (BM) {
                     tot = zero4();
@@ -3284,16 +3238,13 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
                     if constexpr (HL) mma(tot, Pl, cst.ones());
                     const Frag<T> Pn = neg_frag(Pf);
                     for (int md = 0; md < 4; ++md) {
-                        const Frag<T> vo = col_operand<T, NL>(sV, sVt, md);
+                        const Frag<T> vo = col_operand<T, NL>(sV, md);
                         mma(Bm[md], vo, Pn);
                         if constexpr (HL) mma(Bm[md], vo, neg_frag(Pl));
                     }
                     for (int e = 0; e < 4; ++e) Ae[e] -= (double)tot[e];
                 } else {
-                    if constexpr (is_bf16<T>())
-                        tile_sums_bf<NL, HL>(Pf, Pl, cst, sV, sVt, tot, dB);
-                    else
-                        tile_sums<T>(Pf, cst, sVt, tot, dB);
+                    tile_sums<NL, HL>(Pf, Pl, cst, sV, tot, dB);
                     for (int e = 0; e < 4; ++e) {
                         Ae[e] -= (double)tot[e];
                         for (int md = 0; md < 4; ++md) Be[md][e] -= (double)dB[md][e];
@@ -3367,28 +3318,27 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
             }
             // ---- U^T[d][s] += sum_t g[t][d] W[t][s]  (the dV tiles read the LDS copy of U)
             for (int md = 0; md < 4; ++md) {
-                const Frag<T> go = col_operand<T, NL>(sG, sGt, md);
+                const Frag<T> go = col_operand<T, NL>(sG, md);
                 mma(Ut[md], go, Wf);
                 if constexpr (HL) mma(Ut[md], go, Wl);
             }
-            if constexpr (SCN) {
-                // the tile's three Sc2 blocks, once each, for its dV tiles in
-                // the next iteration
-                for (int r = w; r < 3; r += NW_) sc2_tile<T, SP>(r, sWts, sPts, sSc2);
-                // and the carried part of its dV tiles (U and P_K rows of this tile)
+            // the tile's three Sc2 blocks, once each, for its dV tiles (stored in
+            // the next iteration, or with one token block at this tile's end),
+            // and the carried part of those (U and P_K rows of this tile)
+            for (int r = w; r < 3; r += NW_) sc2_tile<T, SP>(r, sWts, sPts, sSc2);
 #pragma unroll
-                for (int k = 0; k < NQD; ++k)
-                    if (w + k * NW_ < 8) dvacc[k] = dv_part<T, SP>((w + k * NW_) >> 1, (w + k * NW_) & 1, sUT, sPts);
-            } else {
-                for (int q = w; q < 8; q += NW_)
-                    dv_tile<T, SP, CAUSAL, AL>(q >> 1, q & 1, sUT, sPts, sWts, sG, sGt, dvp, a.sg.t, t0, a.T, vpart);
-            }
+            for (int k = 0; k < NQD; ++k)
+                if (w + k * NW_ < 8) dvacc[k] = dv_part<T, SP>((w + k * NW_) >> 1, (w + k * NW_) & 1, sUT, sPts);
         } else {
             __syncthreads();  // all waves' P_K rows in LDS
             if constexpr (NB == 2) commit((int)((jr + 1) & 1));
             // non-causal: dV^T = U^T P_K^T; dP_K = alpha + v . U (totals)
-            for (int q = w; q < 8; q += NW_)
-                dv_tile<T, SP, CAUSAL, AL>(q >> 1, q & 1, sUT, sPts, nullptr, nullptr, nullptr, dvp, a.sg.t, t0, a.T, vpart);
+#pragma unroll
+            for (int k = 0; k < NQD; ++k)
+                if (w + k * NW_ < 8)
+                    dv_finish<T, CAUSAL, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1,
+                                             dv_part<T, SP>((w + k * NW_) >> 1, (w + k * NW_) & 1, sUT, sPts), sG, sSc2,
+                                             dvp, a.sg.t, t0, a.T, vpart);
             const UOps<T, HL> uo(Ut);
             for (int nt = 0; nt < 2; ++nt) {
                 f32x4 c = zero4();
@@ -3398,21 +3348,29 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
         }
         {
             if constexpr (KB <= 4) {
-                tsum += softhash_bwd<KB, T, PR>(PKraw, dPK, sSpK, sSmK, sThK, sg, a.L, a.inv_temp, sDproj, ho);
+                tsum += softhash_bwd<KB, T, PR, NC>(PKraw, dPK, sSpK, sSmK, sThK, sg, a.L, a.inv_temp, sDproj, ho);
             } else {
                 softhash_share<KB, T>(PKraw, dPK, wh, sShare);
                 __syncthreads();
-                tsum += softhash_combine<KB, T, SP, NTH, PR>(sShare, sSpK, sSmK, sThK, z, a.L, a.inv_temp, sDproj);
+                tsum += softhash_combine<KB, T, SP, NTH, PR, NC>(sShare, sSpK, sSmK, sThK, z, a.L, a.inv_temp, sDproj);
             }
         }
         // P2: tile j - 1's projections (its Q and K rows arrived in the second
         // phase), for the next iteration
         if constexpr (P2) project2((jr + 1) & 1, (jr + 1) & 1);
         // one token block: the next tile's rows go to it after the tile's
-        // last barrier.  The tile's dK is stored in the next iteration (or
-        // after the loop).
+        // last barrier (causal: the dV tiles read its dO and Sc2 rows first).
+        // The tile's dK is stored in the next iteration (or after the loop).
         if constexpr (NB == 1) {
             __syncthreads();
+            if constexpr (CAUSAL) {
+#pragma unroll
+                for (int k = 0; k < NQD; ++k)
+                    if (w + k * NW_ < 8)
+                        dv_finish<T, CAUSAL, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], sG, sSc2, dvp,
+                                                 a.sg.t, t0, a.T, vpart);
+                __syncthreads();
+            }
             commit(0);
         }
     }
@@ -3420,12 +3378,11 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
         if constexpr (NB == 2) __syncthreads();  // every wave's dproj (and Sc2) rows of the last tile
         dx_store<T, NW_, XC, AL, XF>(sDproj, sPlT, dkp, a.sg.t, (int64_t)j0 * TT, a.T, xpart, xc0);
         if constexpr (SCN) {
-            const T *gtn = (const T *)(smem + (j0 & 1) * Ly::TB + Ly::oGt);
             const T *gnn = (const T *)(smem + (j0 & 1) * Ly::TB + Ly::oG);
 #pragma unroll
             for (int k = 0; k < NQD; ++k)
                 if (w + k * NW_ < 8)
-                    dv_finish<T, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], gnn, gtn, sSc2, dvp, a.sg.t, (int64_t)j0 * TT, a.T,
+                    dv_finish<T, CAUSAL, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1, dvacc[k], gnn, sSc2, dvp, a.sg.t, (int64_t)j0 * TT, a.T,
                                  vpart);
         }
     }
@@ -3445,22 +3402,17 @@ __global__ __launch_bounds__(threads_of(SP), 2) void k_bwd_out(Args a) {
 // per CU (backward 1.52 -> 1.38 ms at C4's shape, K=4); the forward, which has
 // no block sum, keeps a region of that size, since smaller forward layouts (4
 // or 6 workgroups per CU) measured 2.5% slower.
-template <typename T, int SP, bool BWD> struct ProbsL {
-    static constexpr int NW_ = SP / WB;
-    static constexpr int LDN = NatL<T, true>::LD, LDC = ld_of<float>(NCOL), LDDP = sw_ld<T, NCOL>();
+template <typename T, int SP, int KB, bool BWD> struct ProbsL {
+    static constexpr int NW_ = SP / WB, NC = ncol_of<SP, KB>();
+    static constexpr int LDN = NatL<T, true>::LD, LDC = ld_of<float>(NC), LDDP = sw_ld<T, NCOL>();
     static constexpr size_t oX = 0;
-    static constexpr size_t oPl = align16(oX + sizeof(T) * TT * LDN);
-    static constexpr size_t oPlLo = align16(oPl + sizeof(T) * NCOL * LDN);
-    static constexpr size_t oPlT = align16(oPlLo + sizeof(T) * NCOL * LDN);
+    static constexpr size_t oPlT = align16(oX + sizeof(T) * TT * LDN);
     static constexpr size_t oDproj = align16(oPlT + sizeof(T) * D * LDDP);
     static constexpr size_t oSig = align16(oDproj + sizeof(T) * TT * LDDP);  // sp, sm, th
     static_assert(64 * NW_ <= 3 * TT * LDC, "block-sum scratch inside the sigmoid rows");
     static constexpr size_t oRed = BWD ? oSig : align16(oSig + sizeof(float) * 3 * TT * LDC);
-    static constexpr size_t oHash = align16(oSig + sizeof(float) * 3 * TT * LDC + (BWD ? 0 : sizeof(float) * 64 * NW_));
-    static constexpr size_t oShare = align16(oHash + HashOps<T, 4>::bytes);
-    template <int KB> static constexpr size_t bytes() {
-        return align16(oShare + (KB > 4 ? WideHash<T, KB>::bytes(NW_) : 0));
-    }
+    static constexpr size_t oShare = align16(oSig + sizeof(float) * 3 * TT * LDC + (BWD ? 0 : sizeof(float) * 64 * NW_));
+    static constexpr size_t bytes = align16(oShare + (KB > 4 ? WideHash<T, KB>::bytes(NW_) : 0));
 };
 
 // the lane's 4 buckets (s0 .. s0+3) of token row p (S fp32 per row)
@@ -3488,19 +3440,18 @@ __device__ __forceinline__ f32x4 load_row4(const float *row, int s0, int S) {
 template <typename T, int SP, int KB, bool BWD>
 __global__ __launch_bounds__(threads_of(SP)) void k_probs(Args a) {
     if (a.inv_temp_ptr) a.inv_temp = *a.inv_temp_ptr;  // uniform scalar load
-    using Ly = ProbsL<T, SP, BWD>;
+    using Ly = ProbsL<T, SP, KB, BWD>;
     using NL = NatL<T, true>;
-    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDC = Ly::LDC, LDDP = Ly::LDDP;
-    __shared__ __align__(16) unsigned char smem[Ly::template bytes<KB>()];
-    T *sX = (T *)(smem + Ly::oX), *sPl = (T *)(smem + Ly::oPl), *sPlLo = (T *)(smem + Ly::oPlLo);
-    T *sPlT = (T *)(smem + Ly::oPlT), *sDproj = (T *)(smem + Ly::oDproj);
+    constexpr int NW_ = Ly::NW_, NTH = 64 * NW_, LDC = Ly::LDC, LDDP = Ly::LDDP, NC = Ly::NC;
+    __shared__ __align__(16) unsigned char smem[Ly::bytes];
+    T *sX = (T *)(smem + Ly::oX), *sPlT = (T *)(smem + Ly::oPlT), *sDproj = (T *)(smem + Ly::oDproj);
     float *sSp = (float *)(smem + Ly::oSig), *sSm = sSp + TT * LDC, *sTh = sSp + 2 * TT * LDC;
     float *sRed = (float *)(smem + Ly::oRed), *sShare = (float *)(smem + Ly::oShare);
-    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<T, KB>());
+    const WgPos wp = wg_pos(a.nseg, a.M * a.B * a.H, a.nslice, sliced<KB>());
     if (!wp.live) return;
     const int w = wave_id(), g = lg(), i = li(), sw = WB * w, z = wp.z,
               sg = z * SP + sw;
-    const PlaneBlocks pbk(z, SP, KB, a.L, !sliced<T, KB>());  // projection columns of this slice
+    const PlaneBlocks<NW_> pbk(z, SP, KB, a.L, !sliced<KB>(), NC);  // projection columns of this slice
     const int n = wp.n, seg = wp.seg;
     const int m = n / (a.B * a.H);
     const int ntiles = (int)((a.T + TT - 1) / TT);  // the host bounds T by 2^35
@@ -3510,23 +3461,20 @@ __global__ __launch_bounds__(threads_of(SP)) void k_probs(Args a) {
     T *dxp = BWD ? (T *)a.dq + stream_off(a.sg, n, a.B, a.H) : nullptr;
     constexpr int XC = xcols_of(SP, KB);
     constexpr bool XF = xpart_f32(is_bf16<T>(), SP, KB);
-    void *xpart = BWD && sliced<T, KB>() ? xpart_at<T, SP, KB>(a.dqpart, z, n, a) : nullptr;
+    void *xpart = BWD && sliced<KB>() ? xpart_at<T, SP, KB>(a.dqpart, z, n, a) : nullptr;
     const int xc0 = ((z * SP) >> KB) * KB;  // first projection column of the slice's tables
 
     HashOps<T, KB> ho;
     WideHash<T, KB> wh;
+    PlaneSrc<T, NL, true> pcw;
+    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), nullptr);
     if constexpr (BWD) {
         if constexpr (KB <= 4)
-            ho.init((T *)(smem + Ly::oHash), NTH);
+            ho.init();
         else
             wh.init(sg);
         zero_lds<T>(sDproj, TT * LDDP, NTH);
-    }
-    load_planes<T, NTH, NL>(a.planes + m * a.planes_m_stride, a.L * a.K, sPl, is_bf16<T>() ? sPlLo : nullptr,
-                            BWD ? sPlT : nullptr);
-    if constexpr (BWD && KB <= 4) {
-        __syncthreads();  // the hash table in LDS; its operand to registers
-        ho.cache();
+        load_planes_t<T, NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, sPlT);
     }
     CarryA<T> tsum = 0;  // this thread's share of sum du * th
     Prefetch<T, NTH> px_;
@@ -3534,15 +3482,15 @@ __global__ __launch_bounds__(threads_of(SP)) void k_probs(Args a) {
     for (int jt = j0; jt < j1; ++jt) {
         const int64_t t0 = (int64_t)jt * TT;
         __syncthreads();  // the previous tile's readers of sX, sSig, sDproj are done
-        px_.template commit<NL>(sX, nullptr);
+        px_.template commit<NL>(sX);
         if (jt + 1 < j1) px_.issue(xp, a.sq.t, t0 + TT, a.T);  // next tile, in flight during this one
         __syncthreads();
         for (int q = w; q < pbk.tasks(); q += NW_) {
-            project_tile<T, NL>(sX, sPl, sPlLo, pbk.mc(q), q & 1, a.inv_temp, sSp, sSm, BWD ? sTh : nullptr);
+            project_tile<T, NL, false, NC>(sX, pcw, pbk.mc(q), pbk.half(q), a.inv_temp, sSp, sSm, BWD ? sTh : nullptr);
         }
         __syncthreads();
         f32x4 P[2];
-        probs_st<KB>(sSp, sSm, sg, a.S, jt + 1 < ntiles ? TT : lastv, P);
+        probs_st<KB, false, false, NC>(sSp, sSm, sg, a.S, jt + 1 < ntiles ? TT : lastv, P);
         const int s0 = sg + 4 * g;
         if constexpr (!BWD) {
             for (int nt = 0; nt < 2; ++nt) {
@@ -3556,11 +3504,11 @@ __global__ __launch_bounds__(threads_of(SP)) void k_probs(Args a) {
                 dP[nt] = t < a.T ? load_row4(a.dprobs + ((int64_t)n * a.T + t) * a.S, s0, a.S) : zero4();
             }
             if constexpr (KB <= 4) {
-                tsum += softhash_bwd<KB, T>(P, dP, sSp, sSm, sTh, sg, a.L, a.inv_temp, sDproj, ho);
+                tsum += softhash_bwd<KB, T, false, NC>(P, dP, sSp, sSm, sTh, sg, a.L, a.inv_temp, sDproj, ho);
             } else {
                 softhash_share<KB, T>(P, dP, wh, sShare);
                 __syncthreads();
-                tsum += softhash_combine<KB, T, SP, NTH>(sShare, sSp, sSm, sTh, z, a.L, a.inv_temp, sDproj);
+                tsum += softhash_combine<KB, T, SP, NTH, false, NC>(sShare, sSp, sSm, sTh, z, a.L, a.inv_temp, sDproj);
             }
             __syncthreads();
             dx_store<T, NW_, XC, false, XF>(sDproj, sPlT, dxp, a.sg.t, t0, a.T, xpart, xc0);
