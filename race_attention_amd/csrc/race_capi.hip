@@ -37,12 +37,32 @@ int ok() {
     return RACE_OK;
 }
 
-constexpr int64_t kTargetBlocks = 2048;  // workgroups per forward phase (256 CUs x 8)
-// The backward's tile kernels hold one workgroup per CU (LDS): fewer, longer
-// segments there amortise each workgroup's set-up (state rows, planes,
-// constant tables, the first tile's load) over more tiles.  A backward
-// segment is fmul forward segments, so its boundaries are forward ones.
-constexpr int64_t kTargetBlocksBwd = 512;
+// Workgroups per forward phase of long sequences (256 CUs x 8: several rounds
+// of whole segments even out), and the tiles per segment from which that many
+// pay.  A segment costs its workgroup's set-up (state row, planes, the first
+// tile's load: about 2 tiles' time) and 65 fp64 words a bucket of state written,
+// scanned and read again (66 KB a pass at 128 buckets, 4 passes; a tile's rows
+// are 24 KB), so shorter sequences run fewer, longer segments: as many
+// workgroups as are resident at once (target_blocks).  K=4 L=8 bf16 16 x 16384
+// tokens, us: 2048 workgroups of 4 tiles 418 (the scan alone 58), 512 of 16 296;
+// 8 x 262001: 2048 of 32 tiles 2080, 512 of 128 1987; K=3 L=8 48 x 4001: 2016 of
+// 3 280, 768 of 8 234; fp32 K=4 L=8 8 x 8192: 2048 of 1 433, 256 of 8 282.
+constexpr int64_t kTargetBlocks = 2048;
+constexpr int64_t kLongSegTiles = 64;
+// Up to this many tiles (and slices) in all, segments stay one tile each: there
+// the state of an automatic forward is also that of seg_tiles = 1, which
+// backward calls with either are used with.
+constexpr int64_t kOneTileBlocks = 1024;
+// Resident workgroups (256 CUs) of the forward and of the backward tile kernels
+// by slice size: 8-, 4- and 2-wave workgroups.  The backward of 128 buckets and
+// the fp32 kernels hold one 8-wave workgroup per CU; the bf16 backward of 64
+// and 32 buckets holds two and four, and half a round more measured the same or
+// better (K=4 L=4 48 x 8192 global: 768 workgroups 350 us, 384 401).
+int64_t target_blocks(bool bf, int SP, bool bwd) {
+    if (SP == 128) return bf && !bwd ? 512 : 256;
+    if (SP == 64) return bf ? 768 : 512;
+    return bf ? 1024 : 512;
+}
 // Longest segment, forward or backward, in 32-token tiles (8192 tokens).
 // The bf16 kernels carry B in fp32 MFMA accumulators through a segment:
 // k_fwd_reduce and k_bwd_reduce add tile sums from the segment's start,
@@ -93,12 +113,40 @@ void slice_plan(int dtype, int K, int S, int &SP, int &nslice) {
 // Work-items of a 1-D launch: the dispatch packet counts them in 32 bits.
 constexpr int64_t kMaxWorkItems = 0xFFFFFFFFll;
 
+// Tiles per segment of a short sequence: 1 to 4 rounds of target_blocks
+// workgroups, whichever the cost in tiles -- per round a segment and 2 tiles of
+// set-up, per workgroup its state passes (none read per segment by the
+// non-causal operator: half) -- says is shortest.  One 8-wave workgroup per CU
+// only where that leaves segments of 8 tiles: the backward then still joins
+// pairs of forward segments.
+int64_t short_tiles(const race_desc *d, const Plan &p, int64_t per) {
+    int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, false);
+    if (tb < 512 && p.ntiles * per < 8 * tb) tb = 512;
+    const double row = 0.018 * p.SP / 128 * (d->causal ? 1.0 : 0.5);
+    int64_t best = p.ntiles;
+    double cost = 1e300;
+    for (int r = 1; r <= 4; ++r) {
+        int64_t nseg = tb * r / per;
+        nseg = nseg < 1 ? 1 : (nseg > p.ntiles ? p.ntiles : nseg);
+        const int64_t tps = (p.ntiles + nseg - 1) / nseg;
+        nseg = (p.ntiles + tps - 1) / tps;
+        const double c = (double)((nseg * per + tb - 1) / tb) * (double)(tps + 2) + (double)(nseg * per) * row;
+        if (c < cost) {
+            cost = c;
+            best = tps;
+        }
+    }
+    return best;
+}
+
 // bwd: the backward's plan (longer segments of whole forward ones, at most
 // kMaxSegTiles); it rejects an explicit seg_tiles above kMaxSegTiles.
 // walks: the automatic plan of a call whose state a backward may walk (every
 // call but the no-allocation forward and the probability outputs) caps its
 // segments at kMaxSegTiles.
-int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true) {
+// probs: the probability outputs, which keep no state and run kTargetBlocks
+// workgroups at any length.
+int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true, bool probs = false) {
     if (!d) return fail(RACE_E_INVALID, "descriptor is NULL");
     if (d->dtype != RACE_DTYPE_F32 && d->dtype != RACE_DTYPE_BF16)
         return fail(RACE_E_INVALID, "dtype %d is not RACE_DTYPE_F32 or RACE_DTYPE_BF16", d->dtype);
@@ -140,6 +188,7 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true) 
         int64_t nseg = (kTargetBlocks + per - 1) / per;
         if (nseg > p.ntiles) nseg = p.ntiles;
         tps = (p.ntiles + nseg - 1) / nseg;
+        if (tps < kLongSegTiles && !probs && p.ntiles * per > kOneTileBlocks) tps = short_tiles(d, p, per);
         if (walks && tps > kMaxSegTiles) tps = kMaxSegTiles;
     }
     p.tps = (int)(tps < p.ntiles ? tps : p.ntiles);
@@ -162,12 +211,13 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true) 
         // covers the sequence); explicit seg_tiles keeps the forward's
         // (a segment is at most kMaxSegTiles long: m * tps tiles, or the whole
         // sequence when that is shorter)
-        int64_t m = (int64_t)p.fnseg * p.N * p.nslice / kTargetBlocksBwd;
+        const int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, true);
+        int64_t m = ((int64_t)p.fnseg * p.N * p.nslice + tb - 1) / tb;
         if (walks && p.ntiles > kMaxSegTiles && m > kMaxSegTiles / p.tps) m = kMaxSegTiles / p.tps;
         if (m > 1) {
-            const int64_t tb = (int64_t)p.tps * m;
+            const int64_t tl = (int64_t)p.tps * m;
             p.fmul = m < p.fnseg ? (int)m : p.fnseg;
-            p.tps = (int)(tb < p.ntiles ? tb : p.ntiles);
+            p.tps = (int)(tl < p.ntiles ? tl : p.ntiles);
             p.nseg = (int)((p.ntiles + p.tps - 1) / p.tps);
         }
     }
@@ -339,6 +389,24 @@ bool exact_walk(const race_desc *d) {
     return d->causal && (d->inv_temp_ptr != nullptr || (double)d->K * std::fabs((double)d->inv_temp) > 2.0);
 }
 
+// Segment scans: the causal operator reads a prefix (forward) or suffix
+// (backward) row per segment, the non-causal one only the totals.
+void fwd_scan(const race_desc *d, const Plan &p, const Args &a, int elems, hipStream_t s) {
+    const dim3 grid((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N);
+    if (d->causal)
+        k_fwd_scan<<<grid, SCAN_THREADS, 0, s>>>(a.fstate, a.fdelta, p.nseg, elems);
+    else
+        k_seg_totals<<<grid, SCAN_THREADS * TOT_WAVES, 0, s>>>(a.fstate + (int64_t)p.nseg * elems, p.nseg + 1, a.fdelta,
+                                                               p.nseg, elems);
+}
+void bwd_scan(const race_desc *d, const Plan &p, const Args &a, int elems, hipStream_t s) {
+    const dim3 grid((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N);
+    if (d->causal)
+        k_bwd_scan<<<grid, SCAN_THREADS, 0, s>>>(a.rstate, a.rdelta, p.nseg, elems);
+    else
+        k_seg_totals<<<grid, SCAN_THREADS * TOT_WAVES, 0, s>>>(a.rstate, p.nseg, a.rdelta, p.nseg, elems);
+}
+
 template <typename T, int SP, int KB> int fwd_impl(const race_desc *d, const Plan &p, Args a, hipStream_t s) {
     const dim3 grid = tile_grid(p);
     constexpr bool ALC = al_compiled<T, SP, KB>();
@@ -351,7 +419,7 @@ template <typename T, int SP, int KB> int fwd_impl(const race_desc *d, const Pla
     }
     const int elems = p.Spad * SROW;
     if (run_phase(d, RACE_PHASE_SCAN))
-        k_fwd_scan<<<dim3((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N), SCAN_THREADS, 0, s>>>(a.fstate, a.fdelta, p.nseg, elems);
+        fwd_scan(d, p, a, elems, s);
     if (run_phase(d, RACE_PHASE_OUT)) {
         if (d->causal && al)
             k_fwd_out<T, SP, true, KB, false, ALC><<<grid, threads_of(SP), 0, s>>>(a);
@@ -386,8 +454,7 @@ int bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_inv_temp, hi
     }
     const int elems = p.Spad * SROW;
     if (run_phase(d, RACE_PHASE_SCAN))
-        k_bwd_scan<<<dim3((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N), SCAN_THREADS, 0, s>>>(a.rstate, a.rdelta, p.nseg, elems,
-                                                                            d->causal);
+        bwd_scan(d, p, a, elems, s);
     if (run_phase(d, RACE_PHASE_OUT)) {
         if (d->causal && al) {
             if constexpr (ALC) {
@@ -424,7 +491,7 @@ template <typename T, int SP, int KB> int gn_fwd_impl(const race_desc *d, const 
     }
     const int elems = p.Spad * SROW;
     if (run_phase(d, RACE_PHASE_SCAN))
-        k_fwd_scan<<<dim3((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N), SCAN_THREADS, 0, s>>>(a.fstate, a.fdelta, p.nseg, elems);
+        fwd_scan(d, p, a, elems, s);
     if (run_phase(d, RACE_PHASE_OUT)) {
         if (ALC && whole_tiles(d, p))
             k_fwd_out<T, SP, true, KB, true, ALC><<<grid, threads_of(SP), 0, s>>>(a);
@@ -466,7 +533,7 @@ int gn_bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_beta, hip
     }
     const int elems = p.Spad * SROW;
     if (run_phase(d, RACE_PHASE_SCAN))
-        k_bwd_scan<<<dim3((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N), SCAN_THREADS, 0, s>>>(a.rstate, a.rdelta, p.nseg, elems, 1);
+        bwd_scan(d, p, a, elems, s);
     if (run_phase(d, RACE_PHASE_OUT)) {
         if (al)
             k_bwd_out<T, SP, true, KB, true, ALC><<<grid, threads_of(SP), 0, s>>>(a);
@@ -742,14 +809,14 @@ int race_bwd(const race_desc *d, const void *q, const void *k, const void *v, co
 
 size_t race_probs_bwd_workspace_bytes(const race_desc *d) {
     Plan p;
-    if (make_plan(d, p, false, false) != RACE_OK) return 0;
+    if (make_plan(d, p, false, false, true) != RACE_OK) return 0;
     ok();
     return probs_ws_core(p) + p.xpart_bytes;
 }
 
 int race_probs(const race_desc *d, const void *x, const float *planes, float *P, void *stream) {
     Plan p;
-    int rc = make_plan(d, p, false, false);
+    int rc = make_plan(d, p, false, false, true);
     if (rc || (rc = check_tensor("x", x, d->q_stride, p.esize, d->T)) || (rc = check_den("P", P))) return rc;
     if (!planes) return fail(RACE_E_INVALID, "planes is NULL");
     Args a = base_args(d, p, planes);
@@ -763,7 +830,7 @@ int race_probs(const race_desc *d, const void *x, const float *planes, float *P,
 int race_probs_bwd(const race_desc *d, const void *x, const float *planes, const float *dP, void *dx,
                    float *grad_inv_temp, void *ws, size_t ws_bytes, void *stream) {
     Plan p;
-    int rc = make_plan(d, p, false, false);
+    int rc = make_plan(d, p, false, false, true);
     if (rc || (rc = check_tensor("x", x, d->q_stride, p.esize, d->T)) || (rc = check_den("dP", dP)) ||
         (rc = check_out("dx", dx, d->g_stride, p.esize, d)))
         return rc;

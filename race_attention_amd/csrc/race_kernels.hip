@@ -66,7 +66,7 @@ struct Args {
     double *fstate;  // [N][fnseg+1][Spad][D+1] exclusive forward-segment prefixes; [fnseg] = totals
     double *fdelta;  // [N][nseg][Spad][D+1]
     float *rdelta;   // [N][nseg][Spad][D+1]  per-segment (U, alpha) sums
-    float *rstate;   // [N][nseg][Spad][D+1]  exclusive suffixes (non-causal: totals)
+    float *rstate;   // [N][nseg][Spad][D+1]  exclusive suffixes (non-causal: totals, in row 0)
     double *tpart;   // [2][N][nseg][nslice] partial sums of dU*th
     // sliced() instantiations: per-slice partial outputs [nslice][N][T][D] in the element type (bf16 or
     // fp32), summed in fp32 by k_slice_sum
@@ -2737,34 +2737,62 @@ void k_bwd_reduce(Args a) {
     if (threadIdx.x == 0) a.tpart[((int64_t)n * a.nseg + seg) * a.nslice + z] = ts;
 }
 
-// exclusive suffix over segments (causal) or totals (non-causal)
-__global__ __launch_bounds__(SCAN_THREADS) void k_bwd_scan(float *rstate, const float *rdelta, int nseg, int elems,
-                                                           int causal) {
+// exclusive suffix over segments
+__global__ __launch_bounds__(SCAN_THREADS) void k_bwd_scan(float *rstate, const float *rdelta, int nseg, int elems) {
     const int n = blockIdx.y, e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= elems) return;
     const float *src = rdelta + (int64_t)n * nseg * elems + e;
     float *dst = rstate + (int64_t)n * nseg * elems + e;
     double acc = 0.0;
-    if (causal) {  // segments in reverse order
-        int s = nseg;
-        for (; s >= SCAN_BATCH; s -= SCAN_BATCH) {
-            float v[SCAN_BATCH];
+    int s = nseg;
+    for (; s >= SCAN_BATCH; s -= SCAN_BATCH) {
+        float v[SCAN_BATCH];
 #pragma unroll
-            for (int j = 0; j < SCAN_BATCH; ++j) v[j] = src[(int64_t)(s - 1 - j) * elems];
+        for (int j = 0; j < SCAN_BATCH; ++j) v[j] = src[(int64_t)(s - 1 - j) * elems];
 #pragma unroll
-            for (int j = 0; j < SCAN_BATCH; ++j) {
-                dst[(int64_t)(s - 1 - j) * elems] = (float)acc;
-                acc += v[j];
-            }
+        for (int j = 0; j < SCAN_BATCH; ++j) {
+            dst[(int64_t)(s - 1 - j) * elems] = (float)acc;
+            acc += v[j];
         }
-        for (; s > 0; --s) {
-            const float v = src[(int64_t)(s - 1) * elems];
-            dst[(int64_t)(s - 1) * elems] = (float)acc;
-            acc += v;
+    }
+    for (; s > 0; --s) {
+        const float v = src[(int64_t)(s - 1) * elems];
+        dst[(int64_t)(s - 1) * elems] = (float)acc;
+        acc += v;
+    }
+}
+
+// Totals over segments (the non-causal operator): dst[n * rows][e] = the sum of
+// delta[n][seg][e], added in fp64.  The workgroup's waves take a quarter of the
+// segments each and their sums are added in wave order, so the chain of loads is
+// a quarter as long (fp32 K=2 L=5, 4 x 4096 tokens: the backward's totals took
+// 36 us as one thread's two walks over 128 segments).
+constexpr int TOT_WAVES = 4;
+template <typename V>
+__global__ __launch_bounds__(SCAN_THREADS * TOT_WAVES) void k_seg_totals(V *dst, int rows, const V *delta, int nseg,
+                                                                         int elems) {
+    static_assert(SCAN_THREADS == 64, "one wave per quarter");
+    __shared__ double part[TOT_WAVES][SCAN_THREADS];
+    const int n = blockIdx.y, l = threadIdx.x & 63, w = threadIdx.x >> 6, e = blockIdx.x * SCAN_THREADS + l;
+    const int s0 = (int)((int64_t)nseg * w / TOT_WAVES), s1 = (int)((int64_t)nseg * (w + 1) / TOT_WAVES);
+    double acc = 0.0;
+    if (e < elems) {
+        const V *src = delta + (int64_t)n * nseg * elems + e;
+        int s = s0;
+        for (; s + SCAN_BATCH <= s1; s += SCAN_BATCH) {
+            V v[SCAN_BATCH];
+#pragma unroll
+            for (int j = 0; j < SCAN_BATCH; ++j) v[j] = src[(int64_t)(s + j) * elems];
+#pragma unroll
+            for (int j = 0; j < SCAN_BATCH; ++j) acc += v[j];
         }
-    } else {
-        for (int s = 0; s < nseg; ++s) acc += src[(int64_t)s * elems];
-        for (int s = 0; s < nseg; ++s) dst[(int64_t)s * elems] = (float)acc;
+        for (; s < s1; ++s) acc += src[(int64_t)s * elems];
+    }
+    part[w][l] = acc;
+    __syncthreads();
+    if (w == 0 && e < elems) {
+        for (int j = 1; j < TOT_WAVES; ++j) acc += part[j][l];
+        dst[(int64_t)n * rows * elems + e] = (V)acc;
     }
 }
 
@@ -2977,7 +3005,7 @@ void k_bwd_out(Args a) {
         zero_lds<T>(sSc2, TT * LDT, NTH);  // its (t < 16 <= tau) block stays zero
     }
     // reverse carries (U, alpha) after the segment; forward state at the segment end
-    const float *rs = a.rstate + ((int64_t)n * a.nseg + seg) * a.Spad * SROW;
+    const float *rs = a.rstate + ((int64_t)n * a.nseg + (CAUSAL ? seg : 0)) * a.Spad * SROW;
     const double *fs =
         a.fstate + ((int64_t)n * (a.fnseg + 1) + min((seg + 1) * a.fmul, a.fnseg)) * a.Spad * SROW;
     f32x4 Ut[4];  // U^T[d = 16md + 4g + e][s = sw + i]

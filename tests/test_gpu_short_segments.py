@@ -1,0 +1,63 @@
+"""Segment plans of short and medium sequences, and the totals of the
+non-causal scans.
+
+Plans (CPU, from the library's buffer sizes): a sequence whose automatic
+segments would be short runs about as many workgroups as are resident at once,
+never more than the 256-tile walk bound a segment; up to 1024 tiles in all keep
+one-tile segments; the backward's segments are whole forward ones.
+
+Totals (GPU): four waves share a stream's segments; segment counts around the
+waves and the 16-load batches, against the fp64 oracle with the parity bars."""
+import ctypes
+
+import pytest
+import torch
+
+from helpers import TOL, compare, make_case, run_gpu, run_oracle
+
+
+def _segments(B, T, H, K, L, dtype, causal=1):
+    import bench
+    from race_attention_amd import _lib
+    d = _lib.RaceDesc()
+    d.M, d.B, d.T, d.H, d.D, d.L, d.K = 1, B, T, H, 64, L, K
+    d.causal, d.dtype, d.eps, d.inv_temp = causal, dtype, 1e-6, 0.125
+    lib = _lib.load()
+    sb, bw = lib.race_state_bytes(ctypes.byref(d)), lib.race_bwd_workspace_bytes(ctypes.byref(d))
+    return bench.scan_bytes(sb, bw, B * H, T, L, K)[2:]
+
+
+@pytest.mark.parametrize("B,T,H,K,L,fnseg,nseg", [
+    (2, 16384, 8, 4, 8, 32, 16),     # 512 forward workgroups, 256 backward ones
+    (1, 262001, 8, 4, 8, 64, 32),    # the same, of 128 and 256 tiles
+    (1, 1 << 20, 8, 4, 8, 256, 128),  # long: 2048 and 1024
+    (4, 4001, 12, 3, 8, 16, 16),     # 64 buckets: 768
+    (1, 8192, 4, 4, 8, 256, 64),     # 1024 tiles: one-tile forward segments
+    (1, 20, 1, 4, 8, 1, 1),
+])
+def test_short_sequence_plans(B, T, H, K, L, fnseg, nseg):
+    from race_attention_amd import _lib
+    assert _segments(B, T, H, K, L, _lib.RACE_DTYPE_BF16) == (fnseg, nseg)
+
+
+def test_plans_cover_the_sequence_within_the_walk_bound():
+    from race_attention_amd import _lib
+    for causal in (0, 1):
+        for B, H in ((1, 1), (1, 4), (2, 12), (64, 6)):
+            for K, L in ((2, 5), (4, 4), (4, 8), (8, 4)):
+                for T in (1, 33, 785, 1024, 4097, 30000, 250001):
+                    f, b = _segments(B, T, H, K, L, _lib.RACE_DTYPE_BF16, causal)
+                    ntiles = -(-T // 32)
+                    assert 1 <= b <= f <= ntiles
+                    assert -(-ntiles // f) <= 256 and (ntiles <= 256 or -(-ntiles // b) <= 256), (B, H, K, L, T, f, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nseg", [1, 2, 3, 4, 5, 7, 63, 64, 65, 69])
+def test_noncausal_totals(dev, nseg):
+    for dtype in (torch.float32, torch.bfloat16):
+        L, K, T = 5, 2, 32 * nseg - 5
+        q, k, v, do, planes = make_case(T=T, H=2, L=L, K=K, dtype=dtype, seed=nseg)
+        gpu = run_gpu(q, k, v, do, planes, L=L, K=K, causal=False, inv_temp=0.8, dev=dev, seg_tiles=1)
+        ref = run_oracle(q, k, v, do, planes, causal=False, inv_temp=0.8)
+        compare(f"totals nseg={nseg} {dtype}", gpu[:4] + (ref[4],), ref, TOL[dtype])
