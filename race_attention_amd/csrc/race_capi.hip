@@ -665,12 +665,29 @@ int bwd_args(const race_desc *d, const Plan &p, const void *q, const void *k, co
     return RACE_OK;
 }
 
-// prefix mean: segment length so that NS * nseg ~ 4096 waves
-int64_t pm_tseg(int64_t NS, int64_t T) {
-    int64_t nseg = (4096 + NS - 1) / NS;
+// prefix mean: segment length so that NS * nseg ~ 4096 waves, or (k_pm4_*, rows
+// of 16 tokens) ~ 16384 rows of 16 lanes; at most 4096 segments a stream, which
+// the scans walk one after the other.
+int64_t pm_tseg(int64_t NS, int64_t T, bool rows) {
+    int64_t nseg = ((rows ? 16384 : 4096) + NS - 1) / NS;
+    if (nseg > 4096) nseg = 4096;
     if (nseg > T) nseg = T;
     if (nseg < 1) nseg = 1;
-    return (T + nseg - 1) / nseg;
+    const int64_t t = (T + nseg - 1) / nseg;
+    return rows ? (t + 15) / 16 * 16 : t;
+}
+// Whether the k_pm4_* kernels take a call: 16-byte pieces of at most 16 lanes'
+// columns.  The scalar arrays need no alignment.
+bool pm_rows(int64_t D, const void *a, const void *b, const void *c, const void *d) {
+    const uintptr_t m = (uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d;
+    return D % 4 == 0 && D <= 64 && m % 16 == 0;
+}
+size_t pm_workspace(int64_t NS, int64_t T, int64_t D, bool rows) {
+    const int64_t tseg = pm_tseg(NS, T, rows), nseg = (T + tseg - 1) / tseg;
+    const size_t row = (size_t)(D + 1) * sizeof(double);
+    // forward: delta + state; backward adds invA, alpha, rdelta, rstate
+    return (size_t)NS * nseg * row + (size_t)NS * (nseg + 1) * row + 2 * (size_t)NS * T * sizeof(double) +
+           2 * (size_t)NS * nseg * row;
 }
 
 int pm_check(const void *a, const char *na, int64_t NS, int64_t T, int64_t D) {
@@ -996,11 +1013,8 @@ int race_bwd_global(const race_desc *d, const void *q, const void *k, const void
 
 size_t race_prefix_mean_workspace_bytes(int64_t NS, int64_t T, int64_t D) {
     if (NS < 1 || T < 1 || D < 1) return 0;
-    const int64_t tseg = pm_tseg(NS, T), nseg = (T + tseg - 1) / tseg;
-    const size_t row = (size_t)(D + 1) * sizeof(double);
-    // forward: delta + state; backward adds invA, alpha, rdelta, rstate
-    return (size_t)NS * nseg * row + (size_t)NS * (nseg + 1) * row + 2 * (size_t)NS * T * sizeof(double) +
-           2 * (size_t)NS * nseg * row;
+    // the arrays' alignment, which picks the kernels, is not known here: room for either
+    return cmax(pm_workspace(NS, T, D, false), pm_workspace(NS, T, D, true));
 }
 
 int race_prefix_mean_fwd(const float *w, const float *v, float *E, int64_t NS, int64_t T, int64_t D, double eps,
@@ -1010,15 +1024,24 @@ int race_prefix_mean_fwd(const float *w, const float *v, float *E, int64_t NS, i
         return rc;
     const size_t need = race_prefix_mean_workspace_bytes(NS, T, D);
     if (!ws || ws_bytes < need) return fail(RACE_E_WORKSPACE, "workspace %zu bytes < required %zu", ws_bytes, need);
-    const int64_t tseg = pm_tseg(NS, T);
+    const bool rows = pm_rows(D, v, E, nullptr, nullptr);
+    const int64_t tseg = pm_tseg(NS, T, rows);
     const int nseg = (int)((T + tseg - 1) / tseg);
     double *delta = (double *)ws;
     double *state = delta + NS * nseg * (D + 1);
     hipStream_t s = (hipStream_t)stream;
     const int elems = (int)(D + 1);
-    k_pm_reduce<<<dim3(nseg, (unsigned)NS), 64, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
-    k_pm_scan<<<dim3((elems + 255) / 256, (unsigned)NS), 256, 0, s>>>(state, delta, nseg, elems);
-    k_pm_out<<<dim3(nseg, (unsigned)NS), 64, 0, s>>>(w, v, E, state, T, (int)D, tseg, nseg, eps);
+    const dim3 grid(nseg, (unsigned)NS), rgrid((nseg + PM4_ROWS - 1) / PM4_ROWS, (unsigned)NS),
+        sgrid((elems + PM_SCAN_THREADS - 1) / PM_SCAN_THREADS, (unsigned)NS);
+    if (rows)
+        k_pm4_reduce<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
+    else
+        k_pm_reduce<<<grid, 64, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
+    k_pm_scan<<<sgrid, PM_SCAN_THREADS, 0, s>>>(state, delta, nseg, elems);
+    if (rows)
+        k_pm4_out<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, E, state, T, (int)D, tseg, nseg, eps);
+    else
+        k_pm_out<<<grid, 64, 0, s>>>(w, v, E, state, T, (int)D, tseg, nseg, eps);
     return launched("race_prefix_mean_fwd");
 }
 
@@ -1031,7 +1054,8 @@ int race_prefix_mean_bwd(const float *w, const float *v, const float *gE, float 
         return rc;
     const size_t need = race_prefix_mean_workspace_bytes(NS, T, D);
     if (!ws || ws_bytes < need) return fail(RACE_E_WORKSPACE, "workspace %zu bytes < required %zu", ws_bytes, need);
-    const int64_t tseg = pm_tseg(NS, T);
+    const bool rows = pm_rows(D, v, gE, gV, nullptr);
+    const int64_t tseg = pm_tseg(NS, T, rows);
     const int nseg = (int)((T + tseg - 1) / tseg);
     double *delta = (double *)ws;
     double *state = delta + NS * nseg * (D + 1);
@@ -1041,12 +1065,22 @@ int race_prefix_mean_bwd(const float *w, const float *v, const float *gE, float 
     double *rstate = rdelta + NS * nseg * (D + 1);
     hipStream_t s = (hipStream_t)stream;
     const int elems = (int)(D + 1);
-    const dim3 grid(nseg, (unsigned)NS);
-    k_pm_reduce<<<grid, 64, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
-    k_pm_scan<<<dim3((elems + 255) / 256, (unsigned)NS), 256, 0, s>>>(state, delta, nseg, elems);
-    k_pm_bw_fwd<<<grid, 64, 0, s>>>(w, v, gE, state, invA, alpha, rdelta, T, (int)D, tseg, nseg, eps);
-    k_pm_rscan<<<dim3((elems + 255) / 256, (unsigned)NS), 256, 0, s>>>(rstate, rdelta, nseg, elems);
-    k_pm_bw_rev<<<grid, 64, 0, s>>>(w, v, gE, invA, alpha, rstate, gW, gV, T, (int)D, tseg, nseg);
+    const dim3 grid(nseg, (unsigned)NS), rgrid((nseg + PM4_ROWS - 1) / PM4_ROWS, (unsigned)NS),
+        sgrid((elems + PM_SCAN_THREADS - 1) / PM_SCAN_THREADS, (unsigned)NS);
+    if (rows)
+        k_pm4_reduce<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
+    else
+        k_pm_reduce<<<grid, 64, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
+    k_pm_scan<<<sgrid, PM_SCAN_THREADS, 0, s>>>(state, delta, nseg, elems);
+    if (rows)
+        k_pm4_bw_fwd<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, gE, state, invA, alpha, rdelta, T, (int)D, tseg, nseg, eps);
+    else
+        k_pm_bw_fwd<<<grid, 64, 0, s>>>(w, v, gE, state, invA, alpha, rdelta, T, (int)D, tseg, nseg, eps);
+    k_pm_rscan<<<sgrid, PM_SCAN_THREADS, 0, s>>>(rstate, rdelta, nseg, elems);
+    if (rows)
+        k_pm4_bw_rev<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, gE, invA, alpha, rstate, gW, gV, T, (int)D, tseg, nseg);
+    else
+        k_pm_bw_rev<<<grid, 64, 0, s>>>(w, v, gE, invA, alpha, rstate, gW, gV, T, (int)D, tseg, nseg);
     return launched("race_prefix_mean_bwd");
 }
 
