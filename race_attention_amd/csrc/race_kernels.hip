@@ -1864,6 +1864,22 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL> struct FwdO
     static constexpr size_t bytes = SCN ? bytes2 : bytes1;
 };
 
+// acc += A B^T over all SP buckets of two [row][s] operand rows.  fp32 sums each
+// 32 buckets on their own first: one chain of 128 rounds twice as much as four
+// of 32 (out and dV of K=4 L=8 against fp64: 1.9e-7, 2.1e-7; 0.9e-7, 1.0e-7 so).
+template <typename T, int SP> __device__ __forceinline__ void bucket_mma(f32x4 &acc, const T *pa, const T *pb) {
+#pragma unroll
+    for (int kp = 0; kp < SP / 32; ++kp) {
+        if constexpr (is_bf16<T>() || SP == 32) {
+            mma(acc, ld_frag(pa + 32 * kp), ld_frag(pb + 32 * kp));
+        } else {
+            f32x4 c = zero4();
+            mma(c, ld_frag(pa + 32 * kp), ld_frag(pb + 32 * kp));
+            acc += c;
+        }
+    }
+}
+
 // Output tile (d = 16md.., t = 16nt..).  With sDen set, den is summed from
 // the waves' shares (sDen [NW_][TT]) and the md == 0 tiles write it (sliced
 // instantiations: this slice's den share, a partial).  GN also divides the
@@ -1877,8 +1893,7 @@ __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T
     const int g = lg(), i = li();
     const T *pb = sw_frag_ptr<T, SP>(sBT, 16 * md + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
     f32x4 O = zero4();
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) mma(O, ld_frag(pb + 32 * kp), ld_frag(pw + 32 * kp));
+    bucket_mma<T, SP>(O, pb, pw);
     if constexpr (CAUSAL) {
         f32x4 Sc[2];
 #pragma unroll
@@ -1886,8 +1901,7 @@ __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T
             Sc[mt] = zero4();
             if (mt <= nt) {
                 const T *pp = sw_frag_ptr<T, SP>(Pts, 16 * mt + i);
-#pragma unroll
-                for (int kp = 0; kp < SP / 32; ++kp) mma(Sc[mt], ld_frag(pp + 32 * kp), ld_frag(pw + 32 * kp));
+                bucket_mma<T, SP>(Sc[mt], pp, pw);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (16 * mt + 4 * g + e > 16 * nt + i) Sc[mt][e] = 0.f;  // keep t' <= t
@@ -1924,8 +1938,7 @@ template <typename T, int SP> __device__ void sc_fwd_tile(int r, const T *Pts, c
     const int g = lg(), i = li(), mt = r == 2 ? 1 : 0, nt = r == 0 ? 0 : 1;
     const T *pp = sw_frag_ptr<T, SP>(Pts, 16 * mt + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
     f32x4 acc = zero4();
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) mma(acc, ld_frag(pp + 32 * kp), ld_frag(pw + 32 * kp));
+    bucket_mma<T, SP>(acc, pp, pw);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if (16 * mt + 4 * g + e > 16 * nt + i) acc[e] = 0.f;  // keep t' <= t
@@ -1938,8 +1951,7 @@ template <typename T, int SP> __device__ f32x4 fwd_out_partial(int md, int nt, c
     const int i = li();
     const T *pb = sw_frag_ptr<T, SP>(sBT, 16 * md + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
     f32x4 O = zero4();
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) mma(O, ld_frag(pb + 32 * kp), ld_frag(pw + 32 * kp));
+    bucket_mma<T, SP>(O, pb, pw);
     return O;
 }
 // Output tiles (md, 0) and (md, 1): their carried-state parts from one read
@@ -1953,8 +1965,16 @@ template <typename T, int SP> __device__ void fwd_out_partial2(int md, const T *
 #pragma unroll
     for (int kp = 0; kp < SP / 32; ++kp) {
         const Frag<T> b = ld_frag(pb + 32 * kp);
-        mma(O[0], b, ld_frag(pw0 + 32 * kp));
-        mma(O[1], b, ld_frag(pw1 + 32 * kp));
+        if constexpr (is_bf16<T>()) {
+            mma(O[0], b, ld_frag(pw0 + 32 * kp));
+            mma(O[1], b, ld_frag(pw1 + 32 * kp));
+        } else {  // 32 buckets' sums on their own first (bucket_mma)
+            f32x4 c0 = zero4(), c1 = zero4();
+            mma(c0, b, ld_frag(pw0 + 32 * kp));
+            mma(c1, b, ld_frag(pw1 + 32 * kp));
+            O[0] += c0;
+            O[1] += c1;
+        }
     }
 }
 template <typename T, int SP, bool GN, bool AL = false, class NL = NatL<T, true>, bool VNAT = true>
@@ -2860,8 +2880,7 @@ template <typename T, int SP> __device__ void sc2_tile(int r, const T *Wts, cons
     const int g = lg(), i = li(), mt = r == 0 ? 0 : 1, nt = r == 2 ? 1 : 0;
     const T *pw = sw_frag_ptr<T, SP>(Wts, 16 * mt + i), *pp = sw_frag_ptr<T, SP>(Pts, 16 * nt + i);
     f32x4 acc = zero4();
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) mma(acc, ld_frag(pw + 32 * kp), ld_frag(pp + 32 * kp));
+    bucket_mma<T, SP>(acc, pw, pp);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if (16 * mt + 4 * g + e < 16 * nt + i) acc[e] = 0.f;  // keep t >= tau
@@ -2900,8 +2919,7 @@ template <typename T, int SP> __device__ f32x4 dv_part(int md, int nt, const T *
     const int i = li();
     const T *pu = sw_frag_ptr<T, SP>(sUT, 16 * md + i), *pp = sw_frag_ptr<T, SP>(Pts, 16 * nt + i);
     f32x4 acc = zero4();
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) mma(acc, ld_frag(pu + 32 * kp), ld_frag(pp + 32 * kp));
+    bucket_mma<T, SP>(acc, pu, pp);
     return acc;
 }
 template <typename T, bool CAUSAL, bool AL = false, class NL = NatL<T, true>>
