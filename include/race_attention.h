@@ -217,6 +217,13 @@ int race_prefix_mean_bwd(const float *w, const float *v, const float *gE,
 int race_fwd_noalloc(const race_desc *d, const void *q, const void *k, const void *v,
                      const float *planes, void *out, void *stream);
 
+/* The learnable temperature's value (misc/vit.py:923) in one launch:
+ *   out[0] = 1 / c, out[1] = d out[0] / d logit, c = min(max(exp(logit), lo), hi),
+ * from a device fp32 scalar to two device fp32 scalars (exp's gradient passes the
+ * clamp where lo <= exp(logit) <= hi, as torch's clamp does).  out[0] can be a
+ * descriptor's inv_temp_ptr. */
+int race_inv_temp(const float *logit, float lo, float hi, float *out, void *stream);
+
 /* Message for the last failing call on this thread ("" if none). */
 const char *race_last_error(void);
 

@@ -6,6 +6,7 @@ ROCm device, the calls raise -- there is no CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -47,6 +48,7 @@ EXPORTS = (
     "race_fwd_global_workspace_bytes", "race_bwd_global_workspace_bytes", "race_fwd_global", "race_bwd_global",
     "race_prefix_mean_workspace_bytes", "race_prefix_mean_fwd", "race_prefix_mean_bwd",
     "race_fwd_noalloc",
+    "race_inv_temp",
     "race_last_error", "race_abi_version",
 )
 
@@ -99,12 +101,36 @@ def load():
         lib.race_prefix_mean_bwd.restype = ctypes.c_int
         lib.race_fwd_noalloc.argtypes = [dp, vp, vp, vp, vp, vp, vp]
         lib.race_fwd_noalloc.restype = ctypes.c_int
+        lib.race_inv_temp.argtypes = [vp, ctypes.c_float, ctypes.c_float, vp, vp]
+        lib.race_inv_temp.restype = ctypes.c_int
         lib.race_last_error.argtypes = []
         lib.race_last_error.restype = ctypes.c_char_p
         lib.race_abi_version.argtypes = []
         lib.race_abi_version.restype = ctypes.c_int
         _lib = lib
         return lib
+
+
+TORCH_PATH = os.path.join(HERE, "_race_torch.so")
+_calls = None
+
+
+def calls():
+    """The C++ autograd calls (csrc/race_torch.cpp), bound to this library (raises if they have not been built)."""
+    global _calls
+    if _calls is None:
+        load()
+        with _lock:
+            if _calls is None:
+                if not os.path.exists(TORCH_PATH):
+                    raise RaceError(f"{TORCH_PATH} is not built; run `python race_attention_amd/build.py`")
+                import torch  # noqa: F401  (its libraries)
+                spec = importlib.util.spec_from_file_location("_race_torch", TORCH_PATH)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                mod.bind(LIB_PATH, RaceError)
+                _calls = mod
+    return _calls
 
 
 def check(rc: int, what: str) -> None:

@@ -13,7 +13,7 @@ from .functional import race_bucket_probs
 
 
 def _planes_and_temp(ace):
-    return ace.planes(), 1.0 / ace.scale()
+    return ace.planes(), ace.inv_temp() if hasattr(ace, "inv_temp") else 1.0 / ace.scale()
 
 
 def race_bucket_probs_from_qk(attn, Q: torch.Tensor, K: torch.Tensor):

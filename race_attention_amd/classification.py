@@ -43,7 +43,7 @@ class BatchedACE(_vit.BatchedACE):
         (misc/classification.py:641-659): den = (sum_s P_Q A_s).clamp_min(eps)."""
         M, B, T, H, dk = Khf.shape
         assert M == self.M and dk == self.d_k
-        inv_temp = 1.0 / self.scale()
+        inv_temp = self.inv_temp()
         kw = None
         if mask is not None:
             kw, f = _mask_terms(mask, M, B, T, H)

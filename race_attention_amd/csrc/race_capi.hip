@@ -1109,6 +1109,14 @@ int race_fwd_noalloc(const race_desc *d, const void *q, const void *k, const voi
     return fwd_dispatch<float>(&dd, p, a, s);
 }
 
+int race_inv_temp(const float *logit, float lo, float hi, float *out, void *stream) {
+    int rc;
+    if ((rc = check_den("logit", logit)) || (rc = check_den("out", out))) return rc;
+    if (!(lo > 0.f) || !(hi >= lo)) return fail(RACE_E_INVALID, "bounds must be 0 < lo <= hi (got %g, %g)", lo, hi);
+    k_inv_temp<<<1, 64, 0, (hipStream_t)stream>>>(logit, lo, hi, out);
+    return launched("race_inv_temp");
+}
+
 const char *race_last_error(void) { return g_err.c_str(); }
 
 int race_abi_version(void) { return 3; }

@@ -21,6 +21,11 @@ from den).
 
 ``RACEPrefixMeanFlatFn`` is the autograd Function of misc/race.py:9-24 with the
 flat prefix mean computed by the HIP kernels instead of the CPU extension.
+
+``race_attention``, ``race_attention_ex``, ``race_attention_global`` and
+``race_bucket_probs`` run ordinary calls through the C++ autograd calls of
+csrc/race_torch.cpp; what those do not take goes through the Functions here,
+which make the same C ABI calls.
 """
 from __future__ import annotations
 
@@ -215,9 +220,46 @@ class RACEFunction(torch.autograd.Function):
                 None, git if want else None, None, None, None, None)
 
 
+class LogitTemp:
+    """The inverse of a learnable temperature exp(logit) clamped to [lo, hi]
+    (misc/vit.py:923), for the inv_temp argument of the operator: the C++ calls
+    compute it and its gradient in one launch each; value() is the same as
+    torch expressions."""
+
+    __slots__ = ("logit", "lo", "hi")
+
+    def __init__(self, logit, lo, hi):
+        self.logit, self.lo, self.hi = logit, float(lo), float(hi)
+
+    def value(self):
+        return 1.0 / self.logit.exp().clamp(self.lo, self.hi)
+
+
+def _native(kind, q, k, v, planes, temp, kmask, L, K, causal, want_den, eps):
+    """The C++ call of an operator, or None where it is not one that those take."""
+    if not (torch.is_tensor(q) and q.is_cuda):
+        return None
+    lo = hi = -1.0
+    if isinstance(temp, LogitTemp):
+        temp, lo, hi = temp.logit, temp.lo, temp.hi
+    elif isinstance(temp, int):
+        temp = float(temp)
+    mod = _lib.calls()
+    return mod.call(getattr(mod, kind), q, k, v, planes, temp, kmask, int(L), int(K), bool(causal), want_den,
+                    float(eps), lo, hi)
+
+
+def _plain_temp(temp):
+    return temp.value() if isinstance(temp, LogitTemp) else temp
+
+
 def race_attention(Qhf, Khf, Vhf, planes, *, L, K, causal, inv_temp, eps=1e-6):
-    """Differentiable RACE operator on [M,B,T,H,D] tensors (see module doc)."""
-    return RACEFunction.apply(Qhf, Khf, Vhf, planes, inv_temp, L, K, causal, eps)
+    """Differentiable RACE operator on [M,B,T,H,D] tensors (see module doc).
+    inv_temp: a float, a 0-dim tensor or a LogitTemp."""
+    out = _native("F1", Qhf, Khf, Vhf, planes, inv_temp, None, L, K, causal, False, eps)
+    if out is not None:
+        return out
+    return RACEFunction.apply(Qhf, Khf, Vhf, planes, _plain_temp(inv_temp), L, K, causal, eps)
 
 
 # ------------------------------------------------- bucket probabilities as an output
@@ -294,7 +336,10 @@ def race_bucket_probs(x, planes, *, L, K, inv_temp):
     """Soft bucket probabilities of x [M,B,T,H,D] -> [M,B,H,T,L,2^K] fp32
     (differentiable in x and a tensor inv_temp)."""
     M, B, T, H, _ = x.shape
-    return RACEProbsFunction.apply(x, planes, inv_temp, L, K).view(M, B, H, T, L, 1 << K)
+    P = _native("PROBS", x, x, x, planes, inv_temp, None, L, K, False, False, 1e-6)
+    if P is None:
+        P = RACEProbsFunction.apply(x, planes, _plain_temp(inv_temp), L, K)
+    return P.view(M, B, H, T, L, 1 << K)
 
 
 # ------------------------------------------------- key weights and den (F1 extras)
@@ -407,7 +452,12 @@ class RACEExFunction(torch.autograd.Function):
 def race_attention_ex(Qhf, Khf, Vhf, planes, *, L, K, inv_temp, kmask=None, with_den=False, eps=1e-6):
     """Non-causal RACE on [M,B,T,H,D] with per-token key weights kmask [B,T]
     on P_K.  Returns out, or (out, den [M,B,H,T] unclamped) with with_den."""
-    out, den = RACEExFunction.apply(Qhf, Khf, Vhf, planes, inv_temp, kmask, L, K, eps, bool(with_den))
+    res = None
+    if kmask is None or not kmask.requires_grad:
+        res = _native("EX", Qhf, Khf, Vhf, planes, inv_temp, kmask, L, K, False, bool(with_den), eps)
+    if res is not None:
+        return res
+    out, den = RACEExFunction.apply(Qhf, Khf, Vhf, planes, _plain_temp(inv_temp), kmask, L, K, eps, bool(with_den))
     return (out, den) if with_den else out
 
 
@@ -520,6 +570,10 @@ class RACEGlobalFunction(torch.autograd.Function):
 
 def race_attention_global(Qhf, Khf, Vhf, planes, *, L, K, beta, floor=1e-6):
     """Differentiable F2 operator on [M,B,T,H,D] tensors -> (out, den [M,B,H,T])."""
+    if not isinstance(beta, LogitTemp):
+        res = _native("GLOBAL", Qhf, Khf, Vhf, planes, beta, None, L, K, True, True, floor)
+        if res is not None:
+            return res
     return RACEGlobalFunction.apply(Qhf, Khf, Vhf, planes, beta, L, K, floor)
 
 

@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from .functional import race_attention, race_attention_ex
+from .functional import LogitTemp, race_attention, race_attention_ex
 from .race import _corner_protos, merge_heads, planes_from_T
 
 
@@ -43,10 +43,17 @@ class BatchedACE(nn.Module):
     def scale(self) -> torch.Tensor:
         return self.logit_temp.exp().clamp(1e-2, self.temp_max)
 
+    def inv_temp(self):
+        """1 / scale() for the operator: on the GPU as the logit and its bounds,
+        which the kernels' side turns into the value and its gradient."""
+        if self.logit_temp.is_cuda and type(self).scale is BatchedACE.scale:
+            return LogitTemp(self.logit_temp, 1e-2, self.temp_max)
+        return 1.0 / self.scale()
+
     def forward(self, Khf, Vhf, Qhf, eps: float = 1e-6):
         M, B, T, H, dk = Khf.shape
         assert M == self.M and dk == self.d_k
-        inv_temp = 1.0 / self.scale()
+        inv_temp = self.inv_temp()
         return race_attention(Qhf, Khf, Vhf, self.planes(), L=self.L, K=self.K, causal=False,
                               inv_temp=inv_temp, eps=eps)
 
@@ -91,7 +98,7 @@ class RACEAttentionWithDenom(RACEAttention):
     def _ace_with_denom(self, Khf, Vhf, Qhf, eps: float = 1e-6):
         """(out [M,B,T,H,d_k], den [M,B,T,H]) (misc/vit.py:1452-1510)."""
         ace = self.ace
-        out, den = race_attention_ex(Qhf, Khf, Vhf, ace.planes(), L=ace.L, K=ace.K, inv_temp=1.0 / ace.scale(),
+        out, den = race_attention_ex(Qhf, Khf, Vhf, ace.planes(), L=ace.L, K=ace.K, inv_temp=ace.inv_temp(),
                                      with_den=True, eps=eps)
         return out, den.clamp_min(eps).permute(0, 1, 3, 2)
 
