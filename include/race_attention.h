@@ -124,6 +124,21 @@ int race_bwd_ex(const race_desc *d, const void *q, const void *k, const void *v,
                 void *dv, float *grad_inv_temp, void *ws, size_t ws_bytes,
                 void *stream);
 
+/* The padded module's estimator in one call (misc/classification.py:576-592
+ * multiplies P_K, P_Q and V by the [B,T] mask): race_fwd_ex / race_bwd_ex with
+ * V_t, out_t and den_t also multiplied by mask[b][t] -- V and out by the mask
+ * rounded to the element type, each product rounded to it -- and dout, dden and dv
+ * likewise in the backward.  mask is not nullable; sizes as race_fwd_ex's and
+ * race_bwd's. */
+int race_fwd_padded(const race_desc *d, const void *q, const void *k, const void *v,
+                    const float *planes, const float *mask, void *out, float *den,
+                    void *state, void *ws, size_t ws_bytes, void *stream);
+int race_bwd_padded(const race_desc *d, const void *q, const void *k, const void *v,
+                    const float *planes, const float *mask, const void *dout,
+                    const float *dden, const void *state, void *dq, void *dk,
+                    void *dv, float *grad_inv_temp, void *ws, size_t ws_bytes,
+                    void *stream);
+
 /* ---------------------------------------------------------------------
  * Bucket probabilities as an output, for the hybrid consumers that read
  * them (race_bucket_probs_from_qk, misc/arxiv_64K.py:1580-1644;

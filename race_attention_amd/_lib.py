@@ -44,6 +44,7 @@ EXPORTS = (
     "race_state_bytes", "race_fwd_workspace_bytes", "race_bwd_workspace_bytes",
     "race_fwd", "race_bwd",
     "race_fwd_ex_workspace_bytes", "race_fwd_ex", "race_bwd_ex",
+    "race_fwd_padded", "race_bwd_padded",
     "race_probs_bwd_workspace_bytes", "race_probs", "race_probs_bwd",
     "race_fwd_global_workspace_bytes", "race_bwd_global_workspace_bytes", "race_fwd_global", "race_bwd_global",
     "race_prefix_mean_workspace_bytes", "race_prefix_mean_fwd", "race_prefix_mean_bwd",
@@ -89,6 +90,8 @@ def load():
         lib.race_fwd_ex.restype = ctypes.c_int
         lib.race_bwd_ex.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
         lib.race_bwd_ex.restype = ctypes.c_int
+        lib.race_fwd_padded.argtypes, lib.race_fwd_padded.restype = lib.race_fwd_ex.argtypes, ctypes.c_int
+        lib.race_bwd_padded.argtypes, lib.race_bwd_padded.restype = lib.race_bwd_ex.argtypes, ctypes.c_int
         lib.race_fwd_global.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
         lib.race_fwd_global.restype = ctypes.c_int
         lib.race_bwd_global.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]

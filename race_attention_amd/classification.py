@@ -6,10 +6,9 @@ the padding mask), RACEAttention (:595-626) and RACEAttentionWithDenom
 logit_temp) and shapes; the attention core runs in the HIP library
 (race_attention_amd.functional.race_attention_ex).
 
-The reference multiplies P_K, P_Q and V by the [B,T] mask (:580-585).  The
-kernels take the mask as key weights on P_K; the V and P_Q factors are
-elementwise on the operator's input and output (out_t = m_t (P_Q E)_t,
-den_t = m_t sum_s P_Q A_s) and are applied here.
+The reference multiplies P_K, P_Q and V by the [B,T] mask (:580-585); the V and
+P_Q factors are elementwise on the operator's input and output (out_t = m_t
+(P_Q E)_t, den_t = m_t sum_s P_Q A_s), and the kernels apply all three.
 """
 from __future__ import annotations
 
@@ -17,13 +16,7 @@ import torch
 from torch import nn
 
 from . import vit as _vit
-from .functional import race_attention_ex
-
-
-def _mask_terms(mask, M, B, T, H):
-    """[B,T] mask -> (fp32 [B,T] key weights, [1,B,T,1,1] factor)."""
-    m = mask.to(torch.float32)
-    return m, m.view(1, B, T, 1, 1)
+from .functional import race_attention_ex, race_attention_padded
 
 
 class BatchedACE(_vit.BatchedACE):
@@ -44,17 +37,12 @@ class BatchedACE(_vit.BatchedACE):
         M, B, T, H, dk = Khf.shape
         assert M == self.M and dk == self.d_k
         inv_temp = self.inv_temp()
-        kw = None
-        if mask is not None:
-            kw, f = _mask_terms(mask, M, B, T, H)
-            Vhf = Vhf * f.to(Vhf.dtype)
-        res = race_attention_ex(Qhf, Khf, Vhf, self.planes(), L=self.L, K=self.K, inv_temp=inv_temp, kmask=kw,
-                                with_den=with_den, eps=eps)
+        kw = dict(L=self.L, K=self.K, inv_temp=inv_temp, with_den=with_den, eps=eps)
+        if mask is None:
+            res = race_attention_ex(Qhf, Khf, Vhf, self.planes(), **kw)
+        else:
+            res = race_attention_padded(Qhf, Khf, Vhf, self.planes(), mask=mask, **kw)
         out, den = res if with_den else (res, None)
-        if mask is not None:
-            out = out * f.to(out.dtype)
-            if den is not None:
-                den = den * kw.view(1, B, 1, T)
         if den is None:
             return out
         return out, den.clamp_min(eps).permute(0, 1, 3, 2)

@@ -872,11 +872,18 @@ size_t race_fwd_ex_workspace_bytes(const race_desc *d) {
     return p.gfws;  // den partials per slice, like the global mode
 }
 
-int race_fwd_ex(const race_desc *d, const void *q, const void *k, const void *v, const float *planes,
-                const float *kmask, void *out, float *den, void *state, void *ws, size_t ws_bytes, void *stream) {
+} // extern "C"
+
+namespace race {
+namespace {
+
+// race_fwd_ex, and with full race_fwd_padded: the weights also on V, out and den
+int fwd_ex(const race_desc *d, const void *q, const void *k, const void *v, const float *planes, const float *kmask,
+           bool full, void *out, float *den, void *state, void *ws, size_t ws_bytes, void *stream) {
     Plan p;
     int rc = make_plan(d, p);
     if (rc) return rc;
+    if (full && !kmask) return fail(RACE_E_INVALID, "kmask is NULL");
     if (d->causal && (kmask || den))
         return fail(RACE_E_UNSUPPORTED, "key weights and den are implemented for the non-causal operator");
     if ((rc = check_tensor("q", q, d->q_stride, p.esize, d->T)) || (rc = check_tensor("k", k, d->k_stride, p.esize, d->T)) ||
@@ -893,6 +900,7 @@ int race_fwd_ex(const race_desc *d, const void *q, const void *k, const void *v,
     a.v = v;
     a.out = out;
     a.kw = kmask;
+    a.kwv = full;
     a.den = den;
     a.fstate = (double *)state;
     a.fdelta = (double *)ws;
@@ -903,22 +911,51 @@ int race_fwd_ex(const race_desc *d, const void *q, const void *k, const void *v,
     return fwd_dispatch<float>(d, p, a, s);
 }
 
-int race_bwd_ex(const race_desc *d, const void *q, const void *k, const void *v, const float *planes,
-                const float *kmask, const void *dout, const float *dden, const void *state, void *dq, void *dk,
-                void *dv, float *grad_inv_temp, void *ws, size_t ws_bytes, void *stream) {
+int bwd_ex(const race_desc *d, const void *q, const void *k, const void *v, const float *planes, const float *kmask,
+           bool full, const void *dout, const float *dden, const void *state, void *dq, void *dk, void *dv,
+           float *grad_inv_temp, void *ws, size_t ws_bytes, void *stream) {
     Plan p;
     int rc = make_plan(d, p, true);
     if (rc) return rc;
+    if (full && !kmask) return fail(RACE_E_INVALID, "kmask is NULL");
     if (d->causal && (kmask || dden))
         return fail(RACE_E_UNSUPPORTED, "key weights and den are implemented for the non-causal operator");
     if ((kmask && (rc = check_den("kmask", kmask))) || (dden && (rc = check_den("dden", dden)))) return rc;
     Args a;
     if ((rc = bwd_args(d, p, q, k, v, planes, dout, state, dq, dk, dv, ws, ws_bytes, a))) return rc;
     a.kw = kmask;
+    a.kwv = full;
     a.dden = dden;
     hipStream_t s = (hipStream_t)stream;
     if (d->dtype == RACE_DTYPE_BF16) return bwd_dispatch<bf16>(d, p, a, grad_inv_temp, s);
     return bwd_dispatch<float>(d, p, a, grad_inv_temp, s);
+}
+
+} // namespace
+} // namespace race
+
+extern "C" {
+
+int race_fwd_ex(const race_desc *d, const void *q, const void *k, const void *v, const float *planes,
+                const float *kmask, void *out, float *den, void *state, void *ws, size_t ws_bytes, void *stream) {
+    return fwd_ex(d, q, k, v, planes, kmask, false, out, den, state, ws, ws_bytes, stream);
+}
+
+int race_bwd_ex(const race_desc *d, const void *q, const void *k, const void *v, const float *planes,
+                const float *kmask, const void *dout, const float *dden, const void *state, void *dq, void *dk,
+                void *dv, float *grad_inv_temp, void *ws, size_t ws_bytes, void *stream) {
+    return bwd_ex(d, q, k, v, planes, kmask, false, dout, dden, state, dq, dk, dv, grad_inv_temp, ws, ws_bytes, stream);
+}
+
+int race_fwd_padded(const race_desc *d, const void *q, const void *k, const void *v, const float *planes,
+                    const float *mask, void *out, float *den, void *state, void *ws, size_t ws_bytes, void *stream) {
+    return fwd_ex(d, q, k, v, planes, mask, true, out, den, state, ws, ws_bytes, stream);
+}
+
+int race_bwd_padded(const race_desc *d, const void *q, const void *k, const void *v, const float *planes,
+                    const float *mask, const void *dout, const float *dden, const void *state, void *dq, void *dk,
+                    void *dv, float *grad_inv_temp, void *ws, size_t ws_bytes, void *stream) {
+    return bwd_ex(d, q, k, v, planes, mask, true, dout, dden, state, dq, dk, dv, grad_inv_temp, ws, ws_bytes, stream);
 }
 
 size_t race_fwd_global_workspace_bytes(const race_desc *d) {

@@ -88,7 +88,12 @@ struct Args {
     float *gsum;
     // per-token key weights [B][T] on P_K (non-causal padding mask; nullable).
     // Non-causal F1 also writes den [N][T] when den is set and reads dden.
+    // kwv: the weights, rounded to the element type, also multiply V, the output
+    // and (as they are) den, and so dO, dV and dden: the padded module's factors on
+    // P_K, P_Q and V, which as torch expressions are a pass over an M-fold V and
+    // one over the output in each direction.
     const float *kw;
+    int kwv;
     // bucket probabilities as an output: probs [N][T][S] fp32 (k_probs) and
     // their upstream gradient dprobs (k_probs_bwd; x in q, dx in dq)
     float *probs;
@@ -410,6 +415,18 @@ template <typename T, int NTH, bool AL = false> struct Prefetch {
             if (idx < CHUNKS && t < rem) v[j] = ld_at<chunk_t>(base, tile_off(t, st, c * EPC, sizeof(T)));
         }
     }
+    // the rows times per-token weights that a RowW issued with them
+    template <class RW> __device__ __forceinline__ void scale(const RW &rw) {
+        typedef T elems_t __attribute__((ext_vector_type(EPC)));
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            elems_t e = __builtin_bit_cast(elems_t, v[j]);
+            const float w = as_operand<T>(rw.w[j]);
+#pragma unroll
+            for (int q = 0; q < EPC; ++q) e[q] = from_f32<T>(to_f32((T)e[q]) * w);
+            v[j] = __builtin_bit_cast(chunk_t, e);
+        }
+    }
     template <class NL = NatL<T, false>> __device__ __forceinline__ void commit(T *nat) const {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
@@ -421,6 +438,19 @@ template <typename T, int NTH, bool AL = false> struct Prefetch {
             } else {
                 *reinterpret_cast<chunk_t *>(nat + NL::off(t, c * EPC)) = v[j];
             }
+        }
+    }
+};
+
+// Per-token weights of the rows a Prefetch PF holds (0 past the sequence's end).
+template <class PF, int NTH> struct RowW {
+    float w[PF::PER];
+    __device__ __forceinline__ void issue(const float *__restrict__ kw, int64_t t0, int64_t Tn) {
+        const int rem = tile_rows(t0, Tn);
+#pragma unroll
+        for (int j = 0; j < PF::PER; ++j) {
+            const int t = ((int)threadIdx.x + j * NTH) / PF::CPR;
+            w[j] = t < rem ? kw[t0 + t] : 0.f;
         }
     }
 };
@@ -1745,6 +1775,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
     } else {
         Prefetch<T, NTH, AL> pk_[GT];
         Prefetch<T, NTH, AL> pv_[GT];
+        RowW<Prefetch<T, NTH, AL>, NTH> rw_[GT];
         TokPre pt_[GT];
         auto issue = [&](int jg) {
 #pragma unroll
@@ -1755,6 +1786,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
                 pk_[u].issue(kp, a.sk.t, t0, send);
                 pv_[u].issue(vp, a.sv.t, t0, send);
                 if (kwp) pt_[u].issue(kwp, nullptr, t0, send);
+                if (kwp && a.kwv) rw_[u].issue(kwp, t0, send);
             }
         };
         if (j0 < j1) issue(j0);
@@ -1769,6 +1801,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
 #pragma unroll
             for (int u = 0; u < GT; ++u) {
                 pk_[u].template commit<NL>(sK + u * TT * LDN);
+                if (kwp && a.kwv) pv_[u].scale(rw_[u]);
                 pv_[u].template commit<VL>(sVt + u * Ly::VTE);
                 if (kwp) pt_[u].commit(sTok + u * 2 * TT);
             }
@@ -1888,9 +1921,13 @@ template <typename T, int SP, bool CAUSAL, bool GN = false, bool AL = false, cla
           bool VNAT = true>
 __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T *Wts, const T *sVt, T *op,
                              int64_t st, int64_t t0, int64_t Tn, T *part, const float *sDen = nullptr,
-                             float *den = nullptr, float eps = 0.f) {
+                             float *den = nullptr, float eps = 0.f, const float *kw = nullptr) {
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li();
+    // non-causal: the token's weight on the output and den
+    float wt = 1.f;
+    if constexpr (!CAUSAL)
+        if (kw && 16 * nt + i < tile_rows(t0, Tn)) wt = kw[t0 + 16 * nt + i];
     const T *pb = sw_frag_ptr<T, SP>(sBT, 16 * md + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
     f32x4 O = zero4();
     bucket_mma<T, SP>(O, pb, pw);
@@ -1920,8 +1957,12 @@ __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T
 #pragma unroll
             for (int e = 0; e < 4; ++e) O[e] *= r;
         }
-        if (md == 0 && g == 0 && (AL || t < tile_rows(t0, Tn))) den[t0 + t] = dn;
+        if (md == 0 && g == 0 && (AL || t < tile_rows(t0, Tn))) den[t0 + t] = CAUSAL ? dn : dn * wt;
     }
+    if constexpr (!CAUSAL)
+        if (kw)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) O[e] *= as_operand<T>(wt);
     if ((AL || t < tile_rows(t0, Tn))) {
         if (part)
             store4<T>(part_at(part, t0, t, 16 * md + 4 * g), O);
@@ -2039,6 +2080,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
     T *op = (T *)a.out + stream_off(a.so, n, a.B, a.H);
     T *opart = sliced<KB>() ? (T *)a.opart + ((int64_t)z * a.M * a.B * a.H + n) * a.T * D : nullptr;
     const bool want_den = GN || (!CAUSAL && a.den);
+    const float *kwp = !CAUSAL && a.kw && a.kwv ? a.kw + (int64_t)((n / a.H) % a.B) * a.T : nullptr;
     float *sDen = want_den ? (float *)(smem + Ly::oDen) : nullptr;
     float *denp = !want_den       ? nullptr
                   : sliced<KB>() ? a.denpart + ((int64_t)z * a.M * a.B * a.H + n) * a.T
@@ -2325,7 +2367,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
         __syncthreads();
         for (int q = w; q < 8; q += NW_)
             fwd_out_tile<T, SP, CAUSAL, GN, AL, VL, VNAT>(q >> 1, q & 1, sBT, sPts, sWts, sVt, op, a.so.t, t0, a.T, opart, sDen,
-                                            denp, a.eps);
+                                            denp, a.eps, kwp);
         if constexpr (CAUSAL) {
             // carry: B[s][d] += sum_t P_K[t][s] V[t][d]
             for (int md = 0; md < 4; ++md) {
@@ -2459,6 +2501,8 @@ void k_bwd_reduce(Args a) {
     const float *ddp = GS && !GP       ? a.gden + (int64_t)n * a.T
                        : (GN || !CAUSAL) && a.dden ? a.dden + (int64_t)n * a.T
                                                    : nullptr;
+    // non-causal: per-token weights on dO and dden
+    const float *kwp = !CAUSAL && a.kw && a.kwv ? a.kw + (int64_t)((n / a.H) % a.B) * a.T : nullptr;
     float *gsp = GP ? a.gsum + ((int64_t)z * a.M * a.B * a.H + n) * a.T : nullptr;
     // GC writes the per-token terms for k_bwd_out (GS: k_gn_terms does)
     float *rdw = GC ? a.rden + (int64_t)n * a.T : nullptr;
@@ -2497,6 +2541,7 @@ void k_bwd_reduce(Args a) {
     wait_state_loads();
     Prefetch<T, NTH, AL> pq_, pk_, pg_;  // pg_: non-causal dO
     Prefetch2<T, NTH, AL> pgv_;          // causal dO (first half of the waves) and V
+    RowW<Prefetch<T, NTH, AL>, NTH> rw_;
     TokPre pt_;
     // Writes the prefetched rows to token block b.
     auto commit = [&](int b) {
@@ -2508,6 +2553,7 @@ void k_bwd_reduce(Args a) {
             pk_.template commit<NL>((T *)(tb + Ly::oK));
             pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oV));
         } else {
+            if (kwp) pg_.scale(rw_);
             pg_.template commit<NL>((T *)(tb + Ly::oG));
         }
         if constexpr (GN) {
@@ -2524,11 +2570,12 @@ void k_bwd_reduce(Args a) {
             pgv_.issue(gp, a.sdo.t, vp, a.sv.t, (int64_t)j0 * TT, a.T);
         } else {
             pg_.issue(gp, a.sdo.t, (int64_t)j0 * TT, a.T);
+            if (kwp) rw_.issue(kwp, (int64_t)j0 * TT, a.T);
         }
         if constexpr (GN) {
             pt_.issue(denp, ddp, (int64_t)j0 * TT, a.T);
         } else if constexpr (!CAUSAL) {
-            if (ddp) pt_.issue(ddp, nullptr, (int64_t)j0 * TT, a.T);
+            if (ddp) pt_.issue(ddp, kwp, (int64_t)j0 * TT, a.T);
         }
         commit(NB == 2 ? (int)(j0 & 1) : 0);
     }
@@ -2547,11 +2594,12 @@ void k_bwd_reduce(Args a) {
                 pgv_.issue(gp, a.sdo.t, vp, a.sv.t, tn, a.T);
             } else {
                 pg_.issue(gp, a.sdo.t, tn, a.T);
+                if (kwp) rw_.issue(kwp, tn, a.T);
             }
             if constexpr (GN) {
                 pt_.issue(denp, ddp, tn, a.T);
             } else if constexpr (!CAUSAL) {
-                if (ddp) pt_.issue(ddp, nullptr, tn, a.T);
+                if (ddp) pt_.issue(ddp, kwp, tn, a.T);
             }
         };
         // one token block: loads issued ahead of the barrier; two: after it,
@@ -2670,7 +2718,7 @@ void k_bwd_reduce(Args a) {
                 }
                 if constexpr (!CAUSAL && !GN) {
                     if (ddp) {  // den = sum_s P_Q A_s: dP_Q += h A, dA += h P_Q
-                        const float h = sTokIn[16 * nt + i];
+                        const float h = kwp ? sTokIn[16 * nt + i] * sTokIn[TT + 16 * nt + i] : sTokIn[16 * nt + i];
                         for (int e = 0; e < 4; ++e) {
                             dA[nt][e] += h * PQ[nt][e];
                             dPQ[nt][e] += h * (float)a0[e];
@@ -3056,6 +3104,8 @@ void k_bwd_out(Args a) {
     wait_state_loads();
     Prefetch<T, NTH, AL> pq_, pk_, pvn_;  // pvn_: non-causal V (natural only)
     Prefetch2<T, NTH, AL> pgv_;                // causal dO (first half of the waves) and V
+    RowW<Prefetch<T, NTH, AL>, NTH> rw_;       // the weights of pvn_'s rows
+    const bool kwv = kwp && a.kwv;
     TokPre pt_;
     // Writes the prefetched rows to token block b.
     auto commit = [&](int b) {
@@ -3067,6 +3117,7 @@ void k_bwd_out(Args a) {
             pq_.template commit<NL>((T *)(tb + Ly::oQ));
             pgv_.template commit<NL>((T *)(tb + Ly::oG), (T *)(tb + Ly::oV));
         } else {
+            if (kwv) pvn_.scale(rw_);
             pvn_.template commit<NL>((T *)(tb + Ly::oV));
             if (kwp) pt_.commit(tok);
         }
@@ -3139,6 +3190,7 @@ void k_bwd_out(Args a) {
             pgv_.issue(gp, a.sdo.t, vp, a.sv.t, tl, a.T);
         } else {
             pvn_.issue(vp, a.sv.t, tl, a.T);
+            if (kwv) rw_.issue(kwp, tl, a.T);
             if (kwp) pt_.issue(kwp, nullptr, tl, a.T);
         }
         if constexpr (GN) pt_.issue(rdp, gdp, tl, a.T);
@@ -3167,6 +3219,7 @@ void k_bwd_out(Args a) {
                 pgv_.issue(gp, a.sdo.t, vp, a.sv.t, tn, a.T);
             } else {
                 pvn_.issue(vp, a.sv.t, tn, a.T);
+                if (kwv) rw_.issue(kwp, tn, a.T);
                 if (kwp) pt_.issue(kwp, nullptr, tn, a.T);
             }
             if constexpr (GN) pt_.issue(rdp, gdp, tn, a.T);
@@ -3381,10 +3434,13 @@ void k_bwd_out(Args a) {
             // non-causal: dV^T = U^T P_K^T; dP_K = alpha + v . U (totals)
 #pragma unroll
             for (int k = 0; k < NQD; ++k)
-                if (w + k * NW_ < 8)
-                    dv_finish<T, CAUSAL, AL>((w + k * NW_) >> 1, (w + k * NW_) & 1,
-                                             dv_part<T, SP>((w + k * NW_) >> 1, (w + k * NW_) & 1, sUT, sPts), sG, sSc2,
-                                             dvp, a.sg.t, t0, a.T, vpart);
+                if (w + k * NW_ < 8) {
+                    const int md = (w + k * NW_) >> 1, nt = (w + k * NW_) & 1;
+                    f32x4 dv = dv_part<T, SP>(md, nt, sUT, sPts);
+                    if (kwv)  // V's weight
+                        for (int e = 0; e < 4; ++e) dv[e] *= as_operand<T>(sTok[16 * nt + i]);
+                    dv_finish<T, CAUSAL, AL>(md, nt, dv, sG, sSc2, dvp, a.sg.t, t0, a.T, vpart);
+                }
             const UOps<T, HL> uo(Ut);
             for (int nt = 0; nt < 2; ++nt) {
                 f32x4 c = zero4();

@@ -36,7 +36,8 @@ using torch::autograd::variable_list;
 // ------------------------------------------------------------ the operator library
 #define RACE_FNS(X)                                                                                              \
     X(race_state_bytes) X(race_fwd_workspace_bytes) X(race_bwd_workspace_bytes) X(race_fwd) X(race_bwd)          \
-    X(race_fwd_ex_workspace_bytes) X(race_fwd_ex) X(race_bwd_ex) X(race_fwd_global_workspace_bytes)              \
+    X(race_fwd_ex_workspace_bytes) X(race_fwd_ex) X(race_bwd_ex) X(race_fwd_padded) X(race_bwd_padded)           \
+    X(race_fwd_global_workspace_bytes)                                                                            \
     X(race_bwd_global_workspace_bytes) X(race_fwd_global) X(race_bwd_global) X(race_probs_bwd_workspace_bytes)   \
     X(race_probs) X(race_probs_bwd) X(race_inv_temp) X(race_last_error)
 struct Lib {
@@ -99,7 +100,7 @@ void strides4(const Tensor &x, int64_t *st) {
 void *ptr(const Tensor &x) { return x.data_ptr(); }
 float *fptr(const Tensor &x) { return x.defined() ? static_cast<float *>(x.data_ptr()) : nullptr; }
 
-enum Kind : int64_t { F1 = 0, EX = 1, GLOBAL = 2, PROBS = 3 };
+enum Kind : int64_t { F1 = 0, EX = 1, GLOBAL = 2, PROBS = 3, PADDED = 4 };
 
 // What the forward and the backward of one call share beside tensors.
 struct Cfg {
@@ -170,17 +171,19 @@ Fwd forward_impl(const Cfg &c, const Tensor &q0, const Tensor &k0, const Tensor 
     if (!sb) throw NotTaken();
     f.state = bytes(sb, q);
     if (c.den) f.den = fp32({d.M, d.B, d.H, d.T}, q);
-    const Tensor ws = bytes(c.kind == F1   ? lib.race_fwd_workspace_bytes(&d)
-                            : c.kind == EX ? lib.race_fwd_ex_workspace_bytes(&d)
-                                           : lib.race_fwd_global_workspace_bytes(&d),
+    const bool ex = c.kind == EX || c.kind == PADDED;
+    const Tensor ws = bytes(c.kind == F1 ? lib.race_fwd_workspace_bytes(&d)
+                            : ex         ? lib.race_fwd_ex_workspace_bytes(&d)
+                                         : lib.race_fwd_global_workspace_bytes(&d),
                             q);
     void *s = stream_of(q);
     const size_t wb = (size_t)ws.numel();
     const int rc =
         c.kind == F1 ? lib.race_fwd(&d, ptr(q), ptr(k), ptr(v), fptr(planes), ptr(f.out), ptr(f.state), ptr(ws), wb, s)
-        : c.kind == EX
-            ? lib.race_fwd_ex(&d, ptr(q), ptr(k), ptr(v), fptr(planes), fptr(kmask), ptr(f.out), fptr(f.den),
-                              ptr(f.state), ptr(ws), wb, s)
+        : ex
+            ? (c.kind == EX ? lib.race_fwd_ex : lib.race_fwd_padded)(&d, ptr(q), ptr(k), ptr(v), fptr(planes),
+                                                                     fptr(kmask), ptr(f.out), fptr(f.den),
+                                                                     ptr(f.state), ptr(ws), wb, s)
             : lib.race_fwd_global(&d, ptr(q), ptr(k), ptr(v), fptr(planes), ptr(f.out), fptr(f.den), ptr(f.state),
                                   ptr(ws), wb, s);
     if (rc != RACE_OK) throw NotTaken();
@@ -231,9 +234,10 @@ struct Operator : torch::autograd::Function<Operator> {
         if (c.kind == F1) {
             rc = lib.race_bwd(&d, ptr(q), ptr(k), ptr(v), fptr(planes), ptr(dout), ptr(state), ptr(dq), ptr(dk),
                               ptr(dv), fptr(git), ptr(ws), wb, s);
-        } else if (c.kind == EX) {
-            rc = lib.race_bwd_ex(&d, ptr(q), ptr(k), ptr(v), fptr(planes), fptr(kmask), ptr(dout), fptr(dden),
-                                 ptr(state), ptr(dq), ptr(dk), ptr(dv), fptr(git), ptr(ws), wb, s);
+        } else if (c.kind == EX || c.kind == PADDED) {
+            rc = (c.kind == EX ? lib.race_bwd_ex : lib.race_bwd_padded)(
+                &d, ptr(q), ptr(k), ptr(v), fptr(planes), fptr(kmask), ptr(dout), fptr(dden), ptr(state), ptr(dq),
+                ptr(dk), ptr(dv), fptr(git), ptr(ws), wb, s);
         } else {
             const Tensor out = usable(saved[7]);
             strides4(out, d.o_stride);
@@ -329,8 +333,9 @@ py::object call(int64_t kind, py::handle hq, py::handle hk, py::handle hv, py::h
     if (!hmask.is_none()) {
         if (!is_tensor(hmask)) return py::none();
         mask = THPVariable_Unpack(hmask.ptr());
-        if (!plain(mask) || mask.dim() != 2 || mask.size(0) != q.size(1) || mask.size(1) != q.size(2)) return py::none();
+        if (!plain(mask) || mask.requires_grad() || mask.dim() != 2 || mask.size(0) != q.size(1) || mask.size(1) != q.size(2)) return py::none();
     }
+    if (kind == PADDED && !mask.defined()) return py::none();
     try {
         py::gil_scoped_release nogil;
         const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() ||
@@ -370,4 +375,5 @@ PYBIND11_MODULE(_race_torch, m) {
     m.attr("EX") = (int64_t)EX;
     m.attr("GLOBAL") = (int64_t)GLOBAL;
     m.attr("PROBS") = (int64_t)PROBS;
+    m.attr("PADDED") = (int64_t)PADDED;
 }

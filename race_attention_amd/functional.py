@@ -461,6 +461,24 @@ def race_attention_ex(Qhf, Khf, Vhf, planes, *, L, K, inv_temp, kmask=None, with
     return (out, den) if with_den else out
 
 
+def race_attention_padded(Qhf, Khf, Vhf, planes, *, L, K, inv_temp, mask, with_den=False, eps=1e-6):
+    """The padded estimator (misc/classification.py:576-592): the [B,T] mask
+    multiplies P_K, P_Q and V.  Returns out, or (out, den [M,B,H,T]) with
+    with_den; the mask receives a gradient only through the torch expressions
+    that are used where it requires one."""
+    res = _native("PADDED", Qhf, Khf, Vhf, planes, inv_temp, mask, L, K, False, bool(with_den), eps)
+    if res is not None:
+        return res
+    B, T = Qhf.shape[1:3]
+    kw = mask.to(torch.float32)
+    f = kw.view(1, B, T, 1, 1)
+    res = race_attention_ex(Qhf, Khf, Vhf * f.to(Vhf.dtype), planes, L=L, K=K, inv_temp=inv_temp, kmask=kw,
+                            with_den=with_den, eps=eps)
+    out, den = res if with_den else (res, None)
+    out = out * f.to(out.dtype)
+    return (out, den * kw.view(1, B, 1, T)) if with_den else out
+
+
 # ------------------------------------------------- global normalisation (F2)
 def _den_check(den, M, B, H, T, name):
     if den.shape != (M, B, H, T) or den.dtype != torch.float32:
