@@ -58,9 +58,14 @@ constexpr int64_t kOneTileBlocks = 1024;
 // the fp32 kernels hold one 8-wave workgroup per CU; the bf16 backward of 64
 // and 32 buckets holds two and four, and half a round more measured the same or
 // better (K=4 L=4 48 x 8192 global: 768 workgroups 350 us, 384 401).
-int64_t target_blocks(bool bf, int SP, bool bwd) {
+// The non-causal forward of 32 buckets holds six (fp32 four), forward us with
+// the causal operator's four (fp32 two) and with these: bf16 K=2 L=5 384 x 785
+// 75 -> 70, 576 x 197 54 -> 49, K=3 L=4 32 x 16384 105 -> 98, fp32 48 x 3000
+// 82 -> 60.
+int64_t target_blocks(bool bf, int SP, bool bwd, bool causal) {
     if (SP == 128) return bf && !bwd ? 512 : 256;
     if (SP == 64) return bf ? 768 : 512;
+    if (!bwd && !causal) return bf ? 1536 : 1024;
     return bf ? 1024 : 512;
 }
 // Longest segment, forward or backward, in 32-token tiles (8192 tokens).
@@ -114,19 +119,21 @@ void slice_plan(int dtype, int K, int S, int &SP, int &nslice) {
 constexpr int64_t kMaxWorkItems = 0xFFFFFFFFll;
 
 // Tiles per segment of a short sequence: 1 to 4 rounds of target_blocks
-// workgroups, whichever the cost in tiles -- per round a segment and 2 tiles of
-// set-up, per workgroup its state passes (none read per segment by the
-// non-causal operator: half) -- says is shortest.  One 8-wave workgroup per CU
+// workgroups (non-causal: half of one too, where that saves one-tile segments),
+// whichever the cost in tiles -- per round a segment and 2 tiles of set-up, per
+// workgroup its state passes (none read per segment by the non-causal operator:
+// half) -- says is shortest.  One 8-wave workgroup per CU
 // only where that leaves segments of 8 tiles: the backward then still joins
 // pairs of forward segments.
 int64_t short_tiles(const race_desc *d, const Plan &p, int64_t per) {
-    int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, false);
+    int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, false, d->causal);
     if (tb < 512 && p.ntiles * per < 8 * tb) tb = 512;
     const double row = 0.018 * p.SP / 128 * (d->causal ? 1.0 : 0.5);
     int64_t best = p.ntiles;
     double cost = 1e300;
-    for (int r = 1; r <= 4; ++r) {
-        int64_t nseg = tb * r / per;
+    for (const int half : {1, 2, 4, 6, 8}) {
+        if (half == 1 && d->causal) continue;
+        int64_t nseg = tb * half / (2 * per);
         nseg = nseg < 1 ? 1 : (nseg > p.ntiles ? p.ntiles : nseg);
         const int64_t tps = (p.ntiles + nseg - 1) / nseg;
         nseg = (p.ntiles + tps - 1) / tps;
@@ -211,8 +218,18 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true, 
         // covers the sequence); explicit seg_tiles keeps the forward's
         // (a segment is at most kMaxSegTiles long: m * tps tiles, or the whole
         // sequence when that is shorter)
-        const int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, true);
-        int64_t m = ((int64_t)p.fnseg * p.N * p.nslice + tb - 1) / tb;
+        // The non-causal backward reads no state row but the totals, so its
+        // segments are its own: one residency of them.
+        const int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, true, d->causal);
+        if (!d->causal) {
+            int64_t nb = tb / (p.N * p.nslice);
+            nb = nb < 1 ? 1 : (nb > p.ntiles ? p.ntiles : nb);
+            int64_t tl = (p.ntiles + nb - 1) / nb;
+            if (walks && tl > kMaxSegTiles) tl = kMaxSegTiles;
+            p.tps = (int)tl;
+            p.nseg = (int)((p.ntiles + tl - 1) / tl);
+        }
+        int64_t m = !d->causal ? 1 : ((int64_t)p.fnseg * p.N * p.nslice + tb - 1) / tb;
         if (walks && p.ntiles > kMaxSegTiles && m > kMaxSegTiles / p.tps) m = kMaxSegTiles / p.tps;
         if (m > 1) {
             const int64_t tl = (int64_t)p.tps * m;
@@ -307,6 +324,7 @@ Args base_args(const race_desc *d, const Plan &p, const float *planes) {
     a.nseg = p.nseg;
     a.tps = p.tps;
     a.fnseg = p.fnseg;
+    a.fdrows = p.nseg;
     a.fmul = p.fmul;
     a.nslice = p.nslice;
     a.Spad = p.Spad;
@@ -390,12 +408,15 @@ bool exact_walk(const race_desc *d) {
 }
 
 // Segment scans: the causal operator reads a prefix (forward) or suffix
-// (backward) row per segment, the non-causal one only the totals.
+// (backward) row per segment, the non-causal one only the totals.  With one
+// segment its sums are the totals and the reduce kernels write them in place
+// (lone_segment): no launch (1536 streams of 197 tokens, K=2 L=5: the two took
+// 19 and 16 us of 224).
 void fwd_scan(const race_desc *d, const Plan &p, const Args &a, int elems, hipStream_t s) {
     const dim3 grid((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N);
     if (d->causal)
         k_fwd_scan<<<grid, SCAN_THREADS, 0, s>>>(a.fstate, a.fdelta, p.nseg, elems);
-    else
+    else if (p.nseg > 1)
         k_seg_totals<<<grid, SCAN_THREADS * TOT_WAVES, 0, s>>>(a.fstate + (int64_t)p.nseg * elems, p.nseg + 1, a.fdelta,
                                                                p.nseg, elems);
 }
@@ -403,11 +424,22 @@ void bwd_scan(const race_desc *d, const Plan &p, const Args &a, int elems, hipSt
     const dim3 grid((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N);
     if (d->causal)
         k_bwd_scan<<<grid, SCAN_THREADS, 0, s>>>(a.rstate, a.rdelta, p.nseg, elems);
-    else
+    else if (p.nseg > 1)
         k_seg_totals<<<grid, SCAN_THREADS * TOT_WAVES, 0, s>>>(a.rstate, p.nseg, a.rdelta, p.nseg, elems);
 }
 
+void lone_segment(const race_desc *d, const Plan &p, Args &a, bool bwd) {
+    if (d->causal || p.nseg > 1) return;
+    if (bwd) {
+        a.rdelta = a.rstate;
+    } else {  // row 1 of the state's 2
+        a.fdelta = a.fstate + (size_t)p.Spad * SROW;
+        a.fdrows = 2;
+    }
+}
+
 template <typename T, int SP, int KB> int fwd_impl(const race_desc *d, const Plan &p, Args a, hipStream_t s) {
+    lone_segment(d, p, a, false);
     const dim3 grid = tile_grid(p);
     constexpr bool ALC = al_compiled<T, SP, KB>();
     const bool al = ALC && whole_tiles(d, p);
@@ -440,6 +472,7 @@ template <typename T, int SP, int KB> int fwd_impl(const race_desc *d, const Pla
 
 template <typename T, int SP, int KB>
 int bwd_impl(const race_desc *d, const Plan &p, Args a, float *grad_inv_temp, hipStream_t s) {
+    lone_segment(d, p, a, true);
     const dim3 grid = tile_grid(p);
     constexpr bool ALC = al_compiled<T, SP, KB>();
     const bool al = ALC && whole_tiles(d, p);

@@ -64,7 +64,8 @@ struct Args {
     int fnseg, fmul;
     int nslice, Spad;  // bucket slices (grid z) of SP buckets each; Spad = nslice * SP
     double *fstate;  // [N][fnseg+1][Spad][D+1] exclusive forward-segment prefixes; [fnseg] = totals
-    double *fdelta;  // [N][nseg][Spad][D+1]
+    double *fdelta;  // [N][nseg][Spad][D+1], streams fdrows rows apart
+    int fdrows;
     float *rdelta;   // [N][nseg][Spad][D+1]  per-segment (U, alpha) sums
     float *rstate;   // [N][nseg][Spad][D+1]  exclusive suffixes (non-causal: totals, in row 0)
     double *tpart;   // [2][N][nseg][nslice] partial sums of dU*th
@@ -1809,7 +1810,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
             work(jg, b);
         }
     }
-    double *out = a.fdelta + ((int64_t)n * a.nseg + seg) * a.Spad * SROW;
+    double *out = a.fdelta + ((int64_t)n * a.fdrows + seg) * a.Spad * SROW;
     for (int md = 0; md < 4; ++md)
         for (int e = 0; e < 4; ++e)
             out[sidx(sg + i, 16 * md + 4 * g + e)] = BM ? (double)accBm[md][e] : accB[md][e];
@@ -3868,8 +3869,8 @@ __global__ __launch_bounds__(ELEM_THREADS) void k_gn_terms(const float *gsum, in
 }
 
 // grad_inv_temp = sum of all partials, in a fixed order (a small launch at the
-// end of every backward with a temperature gradient: the wave's butterfly in
-// place of one thread's 256 LDS reads, 4.8 -> 2.9 us)
+// end of every backward with a temperature gradient: 4.7 us, most of it the
+// launch and the first load)
 __global__ __launch_bounds__(256) void k_temp_sum(const double *tpart, int64_t count, float *out) {
     __shared__ double red[4];
     double acc = 0.0;

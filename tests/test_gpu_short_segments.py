@@ -4,7 +4,8 @@ non-causal scans.
 Plans (CPU, from the library's buffer sizes): a sequence whose automatic
 segments would be short runs about as many workgroups as are resident at once,
 never more than the 256-tile walk bound a segment; up to 1024 tiles in all keep
-one-tile segments; the backward's segments are whole forward ones.
+one-tile segments; the causal backward's segments are whole forward ones, the
+non-causal one's its own.
 
 Totals (GPU): four waves share a stream's segments; segment counts around the
 waves and the 16-load batches, against the fp64 oracle with the parity bars."""
@@ -61,3 +62,25 @@ def test_noncausal_totals(dev, nseg):
         gpu = run_gpu(q, k, v, do, planes, L=L, K=K, causal=False, inv_temp=0.8, dev=dev, seg_tiles=1)
         ref = run_oracle(q, k, v, do, planes, causal=False, inv_temp=0.8)
         compare(f"totals nseg={nseg} {dtype}", gpu[:4] + (ref[4],), ref, TOL[dtype])
+
+
+def test_noncausal_backward_segments_are_their_own():
+    """384 streams of 10 tiles at 32 buckets: the forward's 3-tile segments are
+    no divisor of the backward's 5-tile ones."""
+    from race_attention_amd import _lib
+    assert _segments(64, 300, 6, 2, 5, _lib.RACE_DTYPE_BF16, causal=0) == (4, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,H,K,L,dtype", [
+    (64, 300, 6, 2, 5, torch.bfloat16),  # 4 forward segments, 2 backward ones
+    (64, 300, 6, 2, 5, torch.float32),
+    (130, 37, 8, 2, 5, torch.bfloat16),  # one segment per stream: the sums are the totals
+    (130, 37, 8, 2, 5, torch.float32),
+    (65, 40, 16, 8, 2, torch.bfloat16),  # the same, over bucket slices
+])
+def test_noncausal_automatic_segments(dev, B, T, H, K, L, dtype):
+    q, k, v, do, planes = make_case(B=B, T=T, H=H, L=L, K=K, dtype=dtype, seed=B)
+    gpu = run_gpu(q, k, v, do, planes, L=L, K=K, causal=False, inv_temp=0.8, dev=dev)
+    ref = run_oracle(q, k, v, do, planes, causal=False, inv_temp=0.8)
+    compare(f"auto {B}x{H}x{T} K={K} {dtype}", gpu[:4] + (ref[4],), ref, TOL[dtype])
