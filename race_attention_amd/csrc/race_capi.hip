@@ -384,18 +384,22 @@ void dx_finish(const Plan &p, const race_desc *d, const void *part, const Args &
 }
 
 // Whole-tile instantiations (template flag AL of the tile kernels): compiled
-// for the causal bf16 slices of 128 buckets at 4 and 8 hash bits, and used
-// when every tile holds TT tokens (T % TT == 0) and every bucket of every
-// slice is one of the S buckets, so no load, store or probability needs a
-// row or bucket guard.  Elsewhere the template argument is false and both
-// branches below launch the same kernel.
+// for the causal bf16 slices of 128 buckets at 4 and 8 hash bits and of 32 and
+// 64 at 2 to 4, and used when every tile holds TT tokens (T % TT == 0) and
+// every bucket of every slice is one of the S buckets, so no load, store or
+// probability needs a row or bucket guard.  Those of 32 and 64 buckets do the
+// general ones' arithmetic (walk_f64) without the guards: forward + backward of
+// 48 x 8192, us: K=4 L=4 351 -> 319 (global 354 -> 324), L=2 354 -> 319 (396 ->
+// 358), K=3 L=8 390 -> 364, L=4 369 -> 332, K=2 L=16 374 -> 349, L=8 357 -> 323.
+// Elsewhere the template argument is false and both branches below launch the
+// same kernel.
 template <typename T, int SP, int KB> constexpr bool al_compiled() {
-    return std::is_same<T, bf16>::value && SP == 128 && (KB == 4 || KB == 8);
+    return std::is_same<T, bf16>::value && (SP == 128 ? KB == 4 || KB == 8 : KB >= 2 && KB <= 4);
 }
 bool whole_tiles(const race_desc *d, const Plan &p) { return d->T % TT == 0 && p.S == p.Spad; }
 
 // The causal F1 operator walks the forward state B back through each backward
-// segment (k_bwd_out); its whole-tile bf16 instantiations do it in fp32, the
+// segment (k_bwd_out); its whole-tile bf16 instantiations of 128 buckets do it in fp32, the
 // others in fp64 (race_kernels.hip walk_f64).  A table's logits differ by at
 // most 2 K |inv_temp| (|tanh| <= 1 per bit), so at most e^(2 K |inv_temp|)
 // separates its largest and smallest probability: above K |inv_temp| = 2
@@ -444,7 +448,7 @@ template <typename T, int SP, int KB> int fwd_impl(const race_desc *d, const Pla
     constexpr bool ALC = al_compiled<T, SP, KB>();
     const bool al = ALC && whole_tiles(d, p);
     if (run_phase(d, RACE_PHASE_REDUCE)) {
-        if (al && !exact_walk(d))
+        if (al && (SP < 128 || !exact_walk(d)))
             k_fwd_reduce<T, SP, KB, ALC><<<grid, threads_of(SP), 0, s>>>(a);
         else
             k_fwd_reduce<T, SP, KB><<<grid, threads_of(SP), 0, s>>>(a);

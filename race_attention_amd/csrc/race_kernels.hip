@@ -741,6 +741,9 @@ __device__ __forceinline__ float corner_tanh(const float *sp, const float *sm, i
     }
 }
 
+// Whether every wave has at most one projection task of two tensors.
+template <int SP, int NC> __host__ __device__ constexpr bool one_task() { return 4 * (NC / 16) <= SP / WB; }
+
 // Projection columns a workgroup of NW waves needs: the K columns of every
 // table its bucket slice [z SP, (z+1) SP) touches, as 16-column blocks
 // pb0 .. pb0+nb-1 (one task per block and 16-token half).  A slice of part of a
@@ -1104,14 +1107,16 @@ template <typename T, int SP, int KB> __host__ __device__ constexpr bool hl_ops(
 // dA, whose factor W / (A + eps) is largest where A (hence B) is smallest,
 // takes that error as it is.  Both sides change together: fp32 sums and an
 // fp32 walk round the same tile sums the same way, and their errors partly
-// cancel.  Every bf16 instantiation but the whole-tile ones (4- and 8-bit,
-// 128 buckets), whose fp32 accumulators keep the registers of k_bwd_out's
+// cancel.  Every bf16 instantiation but the whole-tile ones of 128 buckets (4-
+// and 8-bit), whose fp32 accumulators keep the registers of k_bwd_out's
 // two-wave and k_fwd_reduce's four-wave occupancy.  Where the bucket
 // probabilities can span a wide range, the host runs whole tiles through the
 // generic k_fwd_reduce and the whole-tile k_bwd_out with XW (race_capi.hip
 // exact_walk): their tile sums come from the same P_K and V operands in the
 // same order, so the fp64 walk subtracts exactly what the sums added.
-template <typename T, bool AL> __host__ __device__ constexpr bool walk_f64() { return is_bf16<T>() && !AL; }
+template <typename T, int SP, bool AL> __host__ __device__ constexpr bool walk_f64() {
+    return is_bf16<T>() && !(AL && SP == 128);
+}
 // R = X - bf16(X) (exact in fp32): the lo part of a tile pair whose hi part is
 // the round-to-nearest operand the kernels take from X
 __device__ __forceinline__ void lo_rem(const f32x4 (&X)[2], f32x4 (&R)[2]) {
@@ -1667,7 +1672,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
     // instantiations' fp32 MFMA accumulators (walk_f64).  Tile sums are added
     // tile by tile in token order.
     constexpr bool HL = hl_ops<T, SP, KB>();  // P_K as a hi + lo pair
-    constexpr bool BM = is_bf16<T>() && !walk_f64<T, AL>();
+    constexpr bool BM = is_bf16<T>() && !walk_f64<T, SP, AL>();
     double accB[4][4], accA[4];
     f32x4 accBm[4];
     for (int e = 0; e < 4; ++e) {
@@ -1880,8 +1885,9 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL> struct FwdO
     static constexpr size_t oKEnd = align16(oK + (CAUSAL ? sizeof(T) * TT * LDN : 0));
     static_assert(!ALIAS || oKEnd <= oBT, "Q/K tiles must fit in the P_K / W region");
     // Whole 4-bit tiles (QKP in the kernel) keep the Q and K rows apart from the
-    // P_K / W rows all the same, so the next tile's can be committed early
-    static constexpr bool QKP = AL && KB == 4;
+    // P_K / W rows all the same, so the next tile's can be committed and
+    // projected early (8 waves: beside the output tiles of half of them)
+    static constexpr bool QKP = AL && KB == 4 && SP == 128;
     static constexpr size_t oQ2 = ALIAS ? oEnd : oKEnd;
     static constexpr size_t oK2 = align16(oQ2 + (QKP ? sizeof(T) * TT * LDN : 0));
     // [NW_][TT] per-wave den shares (GN; non-causal F1 when den is requested)
@@ -2162,11 +2168,16 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
         }
         // whole tiles: at most one projection task per wave (Q first), one code path
         auto project_al = [&]() {
-            if (2 * pbk.tasks() >= NW_ || w < 2 * pbk.tasks()) {
-                const bool isq = w < pbk.tasks();
-                const int r = pbk.task(w);
+            auto one = [&](int q) {
+                const bool isq = q < pbk.tasks();
+                const int r = pbk.task(q);
                 project_tile<T, NL, PR, NC>(isq ? sQ : sK, pcw, pbk.mc(r), pbk.half(r), a.inv_temp, isq ? sSpQ : sSpK,
                                             isq ? sSmQ : sSmK, nullptr);
+            };
+            if constexpr (one_task<SP, NC>()) {
+                if (2 * pbk.tasks() >= NW_ || w < 2 * pbk.tasks()) one(w);
+            } else {
+                for (int q = w; q < 2 * pbk.tasks(); q += NW_) one(q);
             }
         };
         if constexpr (QKP) {
@@ -2989,7 +3000,7 @@ __device__ void dv_finish(int md, int nt, f32x4 acc, const T *sG, const T *sc2, 
 // GN (global normalisation, causal only): W = P_Q rd and dA = gd P_Q per
 // token (rd = 1/max(den, eps), gd = dL/d den), so the reverse walk needs
 // neither the forward state nor G.
-template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL = false, bool XW = walk_f64<T, AL>()>
+template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL = false, bool XW = walk_f64<T, SP, AL>()>
 __global__ __launch_bounds__(threads_of(SP)) __attribute__((amdgpu_waves_per_eu(2, bwd_max_waves(SP, CAUSAL))))
 void k_bwd_out(Args a) {
     if (a.inv_temp_ptr) a.inv_temp = *a.inv_temp_ptr;  // uniform scalar load
@@ -3224,7 +3235,7 @@ void k_bwd_out(Args a) {
                 if (kwp) pt_.issue(kwp, nullptr, tn, a.T);
             }
             if constexpr (GN) pt_.issue(rdp, gdp, tn, a.T);
-            if constexpr (AL && MT2) {
+            if constexpr (AL && MT2 && one_task<SP, NC>()) {
                 // whole tiles: at most one task per wave, K (first half) or Q --
                 // one code path on scalar-selected rows, which the compiler can
                 // interleave with the rest of the phase
