@@ -260,3 +260,51 @@ def test_streams_and_graph_capture(dev):
         g.replay()
         torch.cuda.synchronize()
         _equal([t.detach().clone() for t in res], [t.detach() for t in step(*_leaves(new))])
+
+
+@pytest.mark.parametrize("use", ["layer", "layer then exp"])
+def test_checkpoint_of_an_operator(dev, use):
+    """Non-reentrant checkpointing ends its recomputation with an exception from
+    the hook that packs the last saved tensor, which can be the operator's."""
+    from torch.utils.checkpoint import checkpoint
+
+    from race_attention_amd.functional import race_attention, race_bucket_probs
+    x, do, planes = _inputs(dev)
+
+    def layer(q, k, v):
+        out = race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5)
+        return out if use == "layer" else out.exp()
+
+    leaves = _leaves(x)
+    want = torch.autograd.grad(layer(*leaves), leaves, do)
+    _equal(want, torch.autograd.grad(checkpoint(layer, *leaves, use_reentrant=False), leaves, do))
+    probs = lambda q: race_bucket_probs(q, planes, L=L, K=K, inv_temp=0.5)
+    dP = torch.rand_like(probs(x[0]))
+    want = torch.autograd.grad(probs(leaves[0]), leaves[0], dP)
+    _equal(want, torch.autograd.grad(checkpoint(probs, leaves[0], use_reentrant=False), leaves[0], dP))
+
+
+def test_exceptions_keep_their_types(dev):
+    from race_attention_amd.functional import race_attention
+
+    class Stop(Exception):
+        pass
+
+    def stop(t):
+        raise Stop
+
+    x, do, planes = _inputs(dev)
+    q, k, v = _leaves(x)
+    with torch.autograd.graph.saved_tensors_hooks(stop, lambda t: t), pytest.raises(Stop):
+        race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5)
+    # the caching allocator's own limit (nothing is asked of the device)
+    big = torch.zeros(1, 8, 16384, 8, 64, device=dev, dtype=torch.bfloat16)
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(1e-9)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            race_attention(big, big, big, planes, L=L, K=K, causal=True, inv_temp=0.5)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    _equal([race_attention(*x, planes, L=L, K=K, causal=True, inv_temp=0.5)],
+           [race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5).detach()])
