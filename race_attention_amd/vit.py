@@ -46,7 +46,8 @@ class BatchedACE(nn.Module):
     def inv_temp(self):
         """1 / scale() for the operator: on the GPU as the logit and its bounds,
         which the kernels' side turns into the value and its gradient."""
-        if self.logit_temp.is_cuda and type(self).scale is BatchedACE.scale:
+        if (self.logit_temp.is_cuda and getattr(self.scale, "__func__", None) is BatchedACE.scale
+                and isinstance(self.temp_max, (int, float))):
             return LogitTemp(self.logit_temp, 1e-2, self.temp_max)
         return 1.0 / self.scale()
 

@@ -308,3 +308,26 @@ def test_exceptions_keep_their_types(dev):
         torch.cuda.set_per_process_memory_fraction(1.0)
     _equal([race_attention(*x, planes, L=L, K=K, causal=True, inv_temp=0.5)],
            [race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5).detach()])
+
+
+@pytest.mark.parametrize("where", ["class", "instance"])
+def test_a_scale_of_the_program_is_used(dev, where):
+    """A scale() that a program put in place, in a subclass or on the module."""
+    from race_attention_amd import vit
+    from race_attention_amd.functional import race_attention
+    (q, k, v), do, planes = _inputs(dev)
+
+    class Fixed(vit.BatchedACE):
+        def scale(self):
+            return 4.0 * self.logit_temp.exp()
+
+    ace = (Fixed if where == "class" else vit.BatchedACE)(d_k=64, K=K, L=L, M=1).to(dev)
+    if where == "instance":
+        ace.scale = lambda: 4.0 * ace.logit_temp.exp()
+    got = ace(k, v, q)
+    want = race_attention(q, k, v, ace.planes(), L=L, K=K, causal=False,
+                          inv_temp=(1.0 / (4.0 * ace.logit_temp.exp())).detach())
+    _equal([got.detach()], [want])
+    if where == "instance":  # no upper bound
+        ace = vit.BatchedACE(d_k=64, K=K, L=L, M=1, temp_max=None).to(dev)
+        assert torch.equal(ace(k, v, q), race_attention(q, k, v, ace.planes(), L=L, K=K, causal=False, inv_temp=1.0))
