@@ -370,9 +370,7 @@ py::object call(int64_t kind, py::handle hq, py::handle hk, py::handle hv, py::h
 
 PYBIND11_MODULE(_race_torch, m) {
     m.def("bind", &bind);
-    // errors as torch's own calls raise them: an exception of a saved-tensor hook as itself (checkpointing stops its
-    // recomputation with one) and torch.OutOfMemoryError, which pybind11 alone would turn into RuntimeError
-    m.def("call", torch::wrap_pybind_function(&call));
+    m.def("call", &call);
     m.attr("F1") = (int64_t)F1;
     m.attr("EX") = (int64_t)EX;
     m.attr("GLOBAL") = (int64_t)GLOBAL;
