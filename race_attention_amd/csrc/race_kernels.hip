@@ -3510,23 +3510,34 @@ void k_bwd_out(Args a) {
 // backward dP -> dx (dq's pointer and strides; sliced instantiations write
 // fp32 partials) with the temperature-gradient partials.
 // =====================================================================
-// One layout for both directions, except the end-of-kernel block sum's
-// scratch [64 * NW_]: the backward reuses its sigmoid rows for it (the last
-// tile reads them before its last barrier), which brings it to 4 workgroups
-// per CU (backward 1.52 -> 1.38 ms at C4's shape, K=4); the forward, which has
-// no block sum, keeps a region of that size, since smaller forward layouts (4
-// or 6 workgroups per CU) measured 2.5% slower.
+// One layout for both directions.  The backward's end-of-kernel block sum takes
+// the sigmoid rows as its scratch (the last tile reads them before its last
+// barrier).  Planes: in registers, but as rows in LDS for 64 and 128 buckets at 4
+// bits (bf16), where the registers cost waves (128-bucket backward: 78 VGPRs, 3
+// workgroups per CU in place of 4) and more workgroups per CU than 4 (128-bucket
+// forward: 3) write more streams at once and are slower; the layout is padded
+// to that many.  Forward + backward, 16 x 65536, us: K=4 L=8 391 with registers,
+// 376 with rows, K=4 L=4 245 and 229; at K=2 L=5 registers 170, rows 243, K=3 L=2
+// 157 and 230, K=3 L=8 237 and 238; fp32 K=4 L=8 8 x 65536 230 and 781.
+template <typename T, int SP, int KB> __host__ __device__ constexpr bool probs_planes_reg() {
+    return !(is_bf16<T>() && KB == 4 && SP >= 64);
+}
 template <typename T, int SP, int KB, bool BWD> struct ProbsL {
+    using PS = PlaneSrc<T, NatL<T, true>, probs_planes_reg<T, SP, KB>()>;
     static constexpr int NW_ = SP / WB, NC = ncol_of<SP, KB>();
     static constexpr int LDN = NatL<T, true>::LD, LDC = ld_of<float>(NC), LDDP = sw_ld<T, NCOL>();
     static constexpr size_t oX = 0;
-    static constexpr size_t oPlT = align16(oX + sizeof(T) * TT * LDN);
+    static constexpr size_t oPl = align16(oX + sizeof(T) * TT * LDN);
+    static constexpr size_t oPlT = align16(oPl + PS::lds_bytes);
     static constexpr size_t oDproj = align16(oPlT + sizeof(T) * D * LDDP);
     static constexpr size_t oSig = align16(oDproj + sizeof(T) * TT * LDDP);  // sp, sm, th
     static_assert(64 * NW_ <= 3 * TT * LDC, "block-sum scratch inside the sigmoid rows");
     static constexpr size_t oRed = BWD ? oSig : align16(oSig + sizeof(float) * 3 * TT * LDC);
     static constexpr size_t oShare = align16(oSig + sizeof(float) * 3 * TT * LDC + (BWD ? 0 : sizeof(float) * 64 * NW_));
-    static constexpr size_t bytes = align16(oShare + (KB > 4 ? WideHash<T, KB>::bytes(NW_) : 0));
+    static constexpr size_t used = align16(oShare + (KB > 4 ? WideHash<T, KB>::bytes(NW_) : 0));
+    // LDS of 160 KB / 4 and (128-bucket forward) / 3 workgroups at most
+    static constexpr size_t least = PS::lds_bytes == 0 ? 0 : (BWD || SP < 128 ? 36864 : 41984);
+    static constexpr size_t bytes = used > least ? used : least;
 };
 
 // the lane's 4 buckets (s0 .. s0+3) of token row p (S fp32 per row)
@@ -3580,8 +3591,8 @@ __global__ __launch_bounds__(threads_of(SP)) void k_probs(Args a) {
 
     HashOps<T, KB> ho;
     WideHash<T, KB> wh;
-    PlaneSrc<T, NL, true> pcw;
-    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), nullptr);
+    typename Ly::PS pcw;
+    pcw.template init<NTH>(a.planes + m * a.planes_m_stride, a.L * a.K, pbk.mc(pbk.task(w)), (T *)(smem + Ly::oPl));
     if constexpr (BWD) {
         if constexpr (KB <= 4)
             ho.init();
