@@ -411,6 +411,16 @@ bool exact_walk(const race_desc *d) {
     return d->causal && (d->inv_temp_ptr != nullptr || (double)d->K * std::fabs((double)d->inv_temp) > 2.0);
 }
 
+// Up to TOT_FEW segments leave k_seg_totals' waves one element a lane or none.
+template <typename V> void seg_totals(V *dst, int rows, const V *delta, const Plan &p, int elems, hipStream_t s) {
+    if (p.nseg <= TOT_FEW)
+        k_seg_totals_few<<<dim3((elems + TOT_FEW_THREADS - 1) / TOT_FEW_THREADS, (unsigned)p.N), TOT_FEW_THREADS, 0, s>>>(
+            dst, rows, delta, p.nseg, elems);
+    else
+        k_seg_totals<<<dim3((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N), SCAN_THREADS * TOT_WAVES, 0, s>>>(
+            dst, rows, delta, p.nseg, elems);
+}
+
 // Segment scans: the causal operator reads a prefix (forward) or suffix
 // (backward) row per segment, the non-causal one only the totals.  With one
 // segment its sums are the totals and the reduce kernels write them in place
@@ -421,15 +431,14 @@ void fwd_scan(const race_desc *d, const Plan &p, const Args &a, int elems, hipSt
     if (d->causal)
         k_fwd_scan<<<grid, SCAN_THREADS, 0, s>>>(a.fstate, a.fdelta, p.nseg, elems);
     else if (p.nseg > 1)
-        k_seg_totals<<<grid, SCAN_THREADS * TOT_WAVES, 0, s>>>(a.fstate + (int64_t)p.nseg * elems, p.nseg + 1, a.fdelta,
-                                                               p.nseg, elems);
+        seg_totals(a.fstate + (int64_t)p.nseg * elems, p.nseg + 1, a.fdelta, p, elems, s);
 }
 void bwd_scan(const race_desc *d, const Plan &p, const Args &a, int elems, hipStream_t s) {
     const dim3 grid((elems + SCAN_THREADS - 1) / SCAN_THREADS, (unsigned)p.N);
     if (d->causal)
         k_bwd_scan<<<grid, SCAN_THREADS, 0, s>>>(a.rstate, a.rdelta, p.nseg, elems);
     else if (p.nseg > 1)
-        k_seg_totals<<<grid, SCAN_THREADS * TOT_WAVES, 0, s>>>(a.rstate, p.nseg, a.rdelta, p.nseg, elems);
+        seg_totals(a.rstate, p.nseg, a.rdelta, p, elems, s);
 }
 
 void lone_segment(const race_desc *d, const Plan &p, Args &a, bool bwd) {
