@@ -298,7 +298,8 @@ def test_exceptions_keep_their_types(dev):
     with torch.autograd.graph.saved_tensors_hooks(stop, lambda t: t), pytest.raises(Stop):
         race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5)
     # the caching allocator's own limit (nothing is asked of the device)
-    big = torch.zeros(1, 8, 16384, 8, 64, device=dev, dtype=torch.bfloat16)
+    # an output of 33 GB, more than any block that earlier calls left in the cache, from an expanded input
+    big = torch.zeros(1, 1, 16384, 8, 64, device=dev, dtype=torch.bfloat16).expand(1, 2000, -1, -1, -1)
     torch.cuda.empty_cache()
     torch.cuda.set_per_process_memory_fraction(1e-9)
     try:
