@@ -10,10 +10,11 @@ from __future__ import annotations
 import torch
 
 from .functional import race_bucket_probs
+from .vit import operator_temp
 
 
 def _planes_and_temp(ace):
-    return ace.planes(), ace.inv_temp() if hasattr(ace, "inv_temp") else 1.0 / ace.scale()
+    return ace.planes(), operator_temp(ace)
 
 
 def race_bucket_probs_from_qk(attn, Q: torch.Tensor, K: torch.Tensor):

@@ -36,8 +36,7 @@ class BatchedACE(_vit.BatchedACE):
         (misc/classification.py:641-659): den = (sum_s P_Q A_s).clamp_min(eps)."""
         M, B, T, H, dk = Khf.shape
         assert M == self.M and dk == self.d_k
-        inv_temp = self.inv_temp()
-        kw = dict(L=self.L, K=self.K, inv_temp=inv_temp, with_den=with_den, eps=eps)
+        kw = dict(L=self.L, K=self.K, inv_temp=_vit.operator_temp(self), with_den=with_den, eps=eps)
         if mask is None:
             res = race_attention_ex(Qhf, Khf, Vhf, self.planes(), **kw)
         else:

@@ -43,20 +43,27 @@ class BatchedACE(nn.Module):
     def scale(self) -> torch.Tensor:
         return self.logit_temp.exp().clamp(1e-2, self.temp_max)
 
-    def inv_temp(self):
-        """1 / scale() for the operator: on the GPU as the logit and its bounds,
-        which the kernels' side turns into the value and its gradient."""
-        if (self.logit_temp.is_cuda and getattr(self.scale, "__func__", None) is BatchedACE.scale
-                and isinstance(self.temp_max, (int, float))):
-            return LogitTemp(self.logit_temp, 1e-2, self.temp_max)
-        return 1.0 / self.scale()
-
     def forward(self, Khf, Vhf, Qhf, eps: float = 1e-6):
         M, B, T, H, dk = Khf.shape
         assert M == self.M and dk == self.d_k
-        inv_temp = self.inv_temp()
+        inv_temp = operator_temp(self)
         return race_attention(Qhf, Khf, Vhf, self.planes(), L=self.L, K=self.K, causal=False,
                               inv_temp=inv_temp, eps=eps)
+
+
+_SCALE = BatchedACE.scale  # as defined above, whatever a program puts in its place
+
+
+def operator_temp(ace):
+    """1 / ace.scale() for the operator: with BatchedACE's own scale() on the GPU
+    as the logit and its bounds, which the kernels' side turns into the value and
+    its gradient.  A scale() put in its place (in a subclass, on the class or on
+    the module) is called.  (No method: a program's module may hold an attribute
+    of any name.)"""
+    if (isinstance(ace, BatchedACE) and ace.logit_temp.is_cuda and getattr(ace.scale, "__func__", None) is _SCALE
+            and isinstance(ace.temp_max, (int, float))):
+        return LogitTemp(ace.logit_temp, 1e-2, ace.temp_max)
+    return 1.0 / ace.scale()
 
 
 class RACEAttention(nn.Module):
@@ -99,7 +106,7 @@ class RACEAttentionWithDenom(RACEAttention):
     def _ace_with_denom(self, Khf, Vhf, Qhf, eps: float = 1e-6):
         """(out [M,B,T,H,d_k], den [M,B,T,H]) (misc/vit.py:1452-1510)."""
         ace = self.ace
-        out, den = race_attention_ex(Qhf, Khf, Vhf, ace.planes(), L=ace.L, K=ace.K, inv_temp=ace.inv_temp(),
+        out, den = race_attention_ex(Qhf, Khf, Vhf, ace.planes(), L=ace.L, K=ace.K, inv_temp=operator_temp(ace),
                                      with_den=True, eps=eps)
         return out, den.clamp_min(eps).permute(0, 1, 3, 2)
 

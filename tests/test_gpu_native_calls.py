@@ -332,3 +332,41 @@ def test_a_scale_of_the_program_is_used(dev, where):
     if where == "instance":  # no upper bound
         ace = vit.BatchedACE(d_k=64, K=K, L=L, M=1, temp_max=None).to(dev)
         assert torch.equal(ace(k, v, q), race_attention(q, k, v, ace.planes(), L=L, K=K, causal=False, inv_temp=1.0))
+
+
+def test_a_scale_put_on_the_class_and_an_attribute_of_any_name(dev, monkeypatch):
+    """A program that replaces BatchedACE.scale itself, and modules that hold an
+    attribute named inv_temp: scale() is what counts, in the layer, the padded
+    layer and the bucket probabilities."""
+    from types import SimpleNamespace
+
+    from race_attention_amd import classification, vit
+    from race_attention_amd.buckets import race_bucket_probs_from_qk
+    from race_attention_amd.functional import race_attention, race_attention_ex, race_bucket_probs
+    (q, k, v), do, planes = _inputs(dev)
+
+    def check(cls, name, scale):
+        ace = cls(d_k=64, K=K, L=L, M=1).to(dev)
+        ace.inv_temp = torch.tensor(99.0, device=dev)
+        kw = dict(L=L, K=K, inv_temp=(1.0 / scale(ace)).detach())
+        if name == "vit":
+            want = race_attention(q, k, v, ace.planes(), causal=False, **kw)
+        else:
+            want = race_attention_ex(q, k, v, ace.planes(), **kw)
+        _equal([ace(k, v, q).detach()], [want])
+        got = race_bucket_probs_from_qk(SimpleNamespace(ace=ace, M=1), q[0], k[0])
+        _equal([t.detach() for t in got], [race_bucket_probs(t, ace.planes(), **kw) for t in (q, k)])
+
+    for cls, name in ((vit.BatchedACE, "vit"), (classification.BatchedACE, "padded")):
+        check(cls, name, lambda ace: ace.logit_temp.exp())
+    monkeypatch.setattr(vit.BatchedACE, "scale", lambda self: 4.0 * self.logit_temp.exp())
+    for cls, name in ((vit.BatchedACE, "vit"), (classification.BatchedACE, "padded")):
+        check(cls, name, lambda ace: 4.0 * ace.logit_temp.exp())
+
+    class Own:  # any object with planes() and scale()
+        L, K, inv_temp = L, K, 99.0
+        planes = staticmethod(lambda: planes)
+        scale = staticmethod(lambda: torch.tensor(2.0, device=dev))
+
+    got = race_bucket_probs_from_qk(SimpleNamespace(ace=Own, M=1), q[0], k[0])
+    _equal(got, [race_bucket_probs(t, planes, L=L, K=K, inv_temp=0.5) for t in (q, k)])
