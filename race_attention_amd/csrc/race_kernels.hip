@@ -1555,6 +1555,43 @@ __device__ void dx_store(const T *dproj, const T *plt, T *dst, int64_t st, int64
     }
 }
 
+// acc += A B, 32 deep.  fp32 sums each half of the product (QUARTERS: each
+// quarter, half the error for 8 more registers) on its own and adds them once:
+// eight 4-deep steps onto a sum round eight times at the sum's size.  CHAIN: the
+// steps on acc all the same, where acc is still zero, and for the carried sums of
+// 64 and 128 buckets, whose backward spills 20 to 40 VGPRs otherwise (K=4 L=4 48 x
+// 4096, backward 357 us, 414) and whose carries measure no larger an error.
+template <typename T, bool CHAIN = false, bool QUARTERS = false>
+__device__ __forceinline__ void mma_add(f32x4 &acc, const Frag<T> &a, const Frag<T> &b) {
+    if constexpr (is_bf16<T>() || CHAIN) {
+        mma(acc, a, b);
+    } else {
+        constexpr int Q = QUARTERS ? 2 : 1;
+        f32x4 c[2 * Q];
+#pragma unroll
+        for (int q = 0; q < 2 * Q; ++q) c[q] = zero4();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int q = Q * e / 4;
+            c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.lo[e], b.lo[e], c[q], 0, 0, 0);
+            c[Q + q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.hi[e], b.hi[e], c[Q + q], 0, 0, 0);
+        }
+        if constexpr (QUARTERS)
+            acc += (c[0] + c[1]) + (c[2] + c[3]);
+        else
+            acc += c[0] + c[1];
+    }
+}
+
+// Sum of the waves' shares s[w * TT] of a token, in wave order; fp32 adds pairs
+// of waves first, half the roundings at the sum's size.
+template <typename T, int NW> __device__ __forceinline__ float wave_sum(const float *s) {
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w += is_bf16<T>() ? 1 : 2) x += is_bf16<T>() ? s[w * TT] : s[w * TT] + s[(w + 1) * TT];
+    return x;
+}
+
 // Waves per SIMD the backward tile kernels are scheduled for: the causal
 // 128-bucket workgroups run one per CU (2 waves per SIMD, whatever their LDS
 // would allow, at more than 128 registers).
@@ -1904,20 +1941,24 @@ template <typename T, int SP, bool CAUSAL, int KB, bool GN, bool AL> struct FwdO
     static constexpr size_t bytes = SCN ? bytes2 : bytes1;
 };
 
-// acc += A B^T over all SP buckets of two [row][s] operand rows.  fp32 sums each
-// 32 buckets on their own first: one chain of 128 rounds twice as much as four
-// of 32 (out and dV of K=4 L=8 against fp64: 1.9e-7, 2.1e-7; 0.9e-7, 1.0e-7 so).
-template <typename T, int SP> __device__ __forceinline__ void bucket_mma(f32x4 &acc, const T *pa, const T *pb) {
-#pragma unroll
-    for (int kp = 0; kp < SP / 32; ++kp) {
-        if constexpr (is_bf16<T>() || SP == 32) {
-            mma(acc, ld_frag(pa + 32 * kp), ld_frag(pb + 32 * kp));
-        } else {
-            f32x4 c = zero4();
-            mma(c, ld_frag(pa + 32 * kp), ld_frag(pb + 32 * kp));
-            acc += c;
-        }
+// A B^T over all SP buckets of two [row][s] operand rows.  fp32 sums each 32
+// buckets on their own, and of 128 each half.  With mma_add's halves and quarters
+// of the products within the tile, out and dV of K=4 L=8, 3001 tokens, are 0.81
+// and 0.90 1e-7 off fp64 (2-norm); four workgroups of 32 buckets with their
+// outputs summed were 0.88 and 0.97, products in one chain each 1.11 and 1.40.
+template <typename T, int SP> __device__ __forceinline__ f32x4 bucket_mma(const T *pa, const T *pb) {
+    f32x4 acc = zero4();
+    if constexpr (!is_bf16<T>() && SP == 128) {
+        f32x4 half = zero4();
+        mma_add<T>(half, ld_frag(pa + 64), ld_frag(pb + 64));
+        mma_add<T>(half, ld_frag(pa + 96), ld_frag(pb + 96));
+        mma_add<T>(acc, ld_frag(pa), ld_frag(pb));
+        mma_add<T>(acc, ld_frag(pa + 32), ld_frag(pb + 32));
+        return acc + half;
     }
+#pragma unroll
+    for (int kp = 0; kp < SP / 32; ++kp) mma_add<T, SP == 32>(acc, ld_frag(pa + 32 * kp), ld_frag(pb + 32 * kp));
+    return acc;
 }
 
 // Output tile (d = 16md.., t = 16nt..).  With sDen set, den is summed from
@@ -1936,8 +1977,7 @@ __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T
     if constexpr (!CAUSAL)
         if (kw && 16 * nt + i < tile_rows(t0, Tn)) wt = kw[t0 + 16 * nt + i];
     const T *pb = sw_frag_ptr<T, SP>(sBT, 16 * md + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
-    f32x4 O = zero4();
-    bucket_mma<T, SP>(O, pb, pw);
+    f32x4 O = bucket_mma<T, SP>(pb, pw);
     if constexpr (CAUSAL) {
         f32x4 Sc[2];
 #pragma unroll
@@ -1945,20 +1985,18 @@ __device__ void fwd_out_tile(int md, int nt, const T *sBT, const T *Pts, const T
             Sc[mt] = zero4();
             if (mt <= nt) {
                 const T *pp = sw_frag_ptr<T, SP>(Pts, 16 * mt + i);
-                bucket_mma<T, SP>(Sc[mt], pp, pw);
+                Sc[mt] = bucket_mma<T, SP>(pp, pw);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (16 * mt + 4 * g + e > 16 * nt + i) Sc[mt][e] = 0.f;  // keep t' <= t
             }
         }
-        mma(O, col_operand<T, NL, VNAT>(sVt, md), frag_acc<T>(Sc[0], Sc[1]));
+        mma_add<T>(O, col_operand<T, NL, VNAT>(sVt, md), frag_acc<T>(Sc[0], Sc[1]));
     }
     const int t = 16 * nt + i;
     if (GN || !CAUSAL ? sDen != nullptr : false) {
         constexpr int NW_ = SP / WB;
-        float dn = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW_; ++w) dn += sDen[w * TT + t];
+        const float dn = wave_sum<T, NW_>(sDen + t);
         if (GN && !part) {
             const float r = 1.0f / fmaxf(dn, eps);
 #pragma unroll
@@ -1985,8 +2023,7 @@ template <typename T, int SP> __device__ void sc_fwd_tile(int r, const T *Pts, c
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li(), mt = r == 2 ? 1 : 0, nt = r == 0 ? 0 : 1;
     const T *pp = sw_frag_ptr<T, SP>(Pts, 16 * mt + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
-    f32x4 acc = zero4();
-    bucket_mma<T, SP>(acc, pp, pw);
+    f32x4 acc = bucket_mma<T, SP>(pp, pw);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if (16 * mt + 4 * g + e > 16 * nt + i) acc[e] = 0.f;  // keep t' <= t
@@ -1998,9 +2035,7 @@ template <typename T, int SP> __device__ void sc_fwd_tile(int r, const T *Pts, c
 template <typename T, int SP> __device__ f32x4 fwd_out_partial(int md, int nt, const T *sBT, const T *Wts) {
     const int i = li();
     const T *pb = sw_frag_ptr<T, SP>(sBT, 16 * md + i), *pw = sw_frag_ptr<T, SP>(Wts, 16 * nt + i);
-    f32x4 O = zero4();
-    bucket_mma<T, SP>(O, pb, pw);
-    return O;
+    return bucket_mma<T, SP>(pb, pw);
 }
 // Output tiles (md, 0) and (md, 1): their carried-state parts from one read
 // of the B^T operand.
@@ -2013,16 +2048,8 @@ template <typename T, int SP> __device__ void fwd_out_partial2(int md, const T *
 #pragma unroll
     for (int kp = 0; kp < SP / 32; ++kp) {
         const Frag<T> b = ld_frag(pb + 32 * kp);
-        if constexpr (is_bf16<T>()) {
-            mma(O[0], b, ld_frag(pw0 + 32 * kp));
-            mma(O[1], b, ld_frag(pw1 + 32 * kp));
-        } else {  // 32 buckets' sums on their own first (bucket_mma)
-            f32x4 c0 = zero4(), c1 = zero4();
-            mma(c0, b, ld_frag(pw0 + 32 * kp));
-            mma(c1, b, ld_frag(pw1 + 32 * kp));
-            O[0] += c0;
-            O[1] += c1;
-        }
+        mma_add<T>(O[0], b, ld_frag(pw0 + 32 * kp));
+        mma_add<T>(O[1], b, ld_frag(pw1 + 32 * kp));
     }
 }
 template <typename T, int SP, bool GN, bool AL = false, class NL = NatL<T, true>, bool VNAT = true>
@@ -2030,13 +2057,11 @@ __device__ void fwd_out_final(int md, int nt, f32x4 O, const T *sVt, const T *sc
                               int64_t Tn, T *part, const float *sDen, float *den, float eps) {
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li();
-    mma(O, col_operand<T, NL, VNAT>(sVt, md), ld_frag_pi(sc + (16 * nt + i) * LDT));
+    mma_add<T>(O, col_operand<T, NL, VNAT>(sVt, md), ld_frag_pi(sc + (16 * nt + i) * LDT));
     const int t = 16 * nt + i;
     if (GN && sDen != nullptr) {
         constexpr int NW_ = SP / WB;
-        float dn = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW_; ++w) dn += sDen[w * TT + t];
+        const float dn = wave_sum<T, NW_>(sDen + t);
         if (!part) {
             const float r = 1.0f / fmaxf(dn, eps);
 #pragma unroll
@@ -2271,7 +2296,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
             // carry: B[s][d] += sum_t P_K[t][s] V[t][d]
             for (int md = 0; md < 4; ++md) {
                 const Frag<T> vo = col_operand<T, VL, VNAT>(sVt, md);
-                mma(Bc[md], Pf, vo);
+                mma_add<T, (SP > 32)>(Bc[md], Pf, vo);
                 if constexpr (HL) mma(Bc[md], Pl, vo);
             }
             for (int e = 0; e < 4; ++e) a0[e] += (CarryA<T>)tot[e];
@@ -2384,7 +2409,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
             // carry: B[s][d] += sum_t P_K[t][s] V[t][d]
             for (int md = 0; md < 4; ++md) {
                 const Frag<T> vo = col_operand<T, VL, VNAT>(sVt, md);
-                mma(Bc[md], Pf, vo);
+                mma_add<T, (SP > 32)>(Bc[md], Pf, vo);
                 if constexpr (HL) mma(Bc[md], Pl, vo);
             }
             for (int e = 0; e < 4; ++e) a0[e] += (CarryA<T>)tot[e];
@@ -2747,12 +2772,12 @@ void k_bwd_reduce(Args a) {
         for (int md = 0; md < 4; ++md) {
             if constexpr (!GP) {
                 const Frag<T> go = col_operand<T, NL>(sG, md);
-                mma(Ut[md], go, Wf);
+                mma_add<T, (SP > 32)>(Ut[md], go, Wf);
                 if constexpr (HL) mma(Ut[md], go, Wl);
             }
             if constexpr (CAUSAL) {
                 const Frag<T> vo = col_operand<T, NL>(sV, md);
-                mma(Bt[md], vo, Pf);
+                mma_add<T, (SP > 32)>(Bt[md], vo, Pf);
                 if constexpr (HL) mma(Bt[md], vo, Pl);
             }
         }
@@ -2762,10 +2787,7 @@ void k_bwd_reduce(Args a) {
             __syncthreads();  // every wave's share of sum_s P_Q G
             for (int nt = 0; nt < 2; ++nt) {
                 const int t = 16 * nt + i;
-                float sq = 0.f;
-#pragma unroll
-                for (int v = 0; v < NW_; ++v) sq += sGs[v * TT + t];
-                const float dn = sTokIn[t];
+                const float sq = wave_sum<T, NW_>(sGs + t), dn = sTokIn[t];
                 gd[nt] = sTokIn[TT + t] - (dn >= a.eps ? rd[nt] * rd[nt] * sq : 0.f);
                 if (rdw && w == 0 && g == 0 && t < tile_rows(t0, a.T)) {
                     rdw[t0 + t] = rd[nt];
@@ -2958,8 +2980,7 @@ template <typename T, int SP> __device__ void sc2_tile(int r, const T *Wts, cons
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li(), mt = r == 0 ? 0 : 1, nt = r == 2 ? 1 : 0;
     const T *pw = sw_frag_ptr<T, SP>(Wts, 16 * mt + i), *pp = sw_frag_ptr<T, SP>(Pts, 16 * nt + i);
-    f32x4 acc = zero4();
-    bucket_mma<T, SP>(acc, pw, pp);
+    f32x4 acc = bucket_mma<T, SP>(pw, pp);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if (16 * mt + 4 * g + e < 16 * nt + i) acc[e] = 0.f;  // keep t >= tau
@@ -2997,16 +3018,14 @@ template <typename T, bool HL> struct UOps {
 template <typename T, int SP> __device__ f32x4 dv_part(int md, int nt, const T *sUT, const T *Pts) {
     const int i = li();
     const T *pu = sw_frag_ptr<T, SP>(sUT, 16 * md + i), *pp = sw_frag_ptr<T, SP>(Pts, 16 * nt + i);
-    f32x4 acc = zero4();
-    bucket_mma<T, SP>(acc, pu, pp);
-    return acc;
+    return bucket_mma<T, SP>(pu, pp);
 }
 template <typename T, bool CAUSAL, bool AL = false, class NL = NatL<T, true>>
 __device__ void dv_finish(int md, int nt, f32x4 acc, const T *sG, const T *sc2, T *dvp, int64_t st, int64_t t0,
                           int64_t Tn, T *part) {
     constexpr int LDT = ldp_of<T>(TT);
     const int g = lg(), i = li();
-    if constexpr (CAUSAL) mma(acc, col_operand<T, NL>(sG, md), ld_frag_pi(sc2 + (16 * nt + i) * LDT));
+    if constexpr (CAUSAL) mma_add<T, false, true>(acc, col_operand<T, NL>(sG, md), ld_frag_pi(sc2 + (16 * nt + i) * LDT));
     const int t = 16 * nt + i;
     if ((AL || t < tile_rows(t0, Tn))) {
         if (part)
@@ -3449,7 +3468,7 @@ void k_bwd_out(Args a) {
             // ---- U^T[d][s] += sum_t g[t][d] W[t][s]  (the dV tiles read the LDS copy of U)
             for (int md = 0; md < 4; ++md) {
                 const Frag<T> go = col_operand<T, NL>(sG, md);
-                mma(Ut[md], go, Wf);
+                mma_add<T, (SP > 32)>(Ut[md], go, Wf);
                 if constexpr (HL) mma(Ut[md], go, Wl);
             }
             // the tile's three Sc2 blocks, once each, for its dV tiles (stored in
