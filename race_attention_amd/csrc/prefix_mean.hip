@@ -206,12 +206,21 @@ struct Pm4Pos {
     int seg, l;          // segment; lane in its row (columns 4l ..)
     bool live, col;      // the segment exists; the lane has columns
 };
-__device__ __forceinline__ Pm4Pos pm4_pos(int64_t T, int D, int64_t tseg, int nseg) {
+// Rows are numbered over (stream, segment), so that a workgroup's rows all work
+// where streams are many and segments few (backward, 16384 x 197, us: segments of
+// one stream 4729, these 1092, a wave per segment 1606).  From 4 segments on a
+// stream's rows start a new wave: the shorter last segment holds up one wave of a
+// stream's, not the next stream's rows too (128 x 197, 13 segments: 26.9 us, not
+// 29.4).
+__host__ __device__ __forceinline__ int pm4_stride(int nseg) { return nseg < 4 ? nseg : (nseg + 3) / 4 * 4; }
+__device__ __forceinline__ Pm4Pos pm4_pos(int64_t NS, int64_t T, int D, int64_t tseg, int nseg) {
     Pm4Pos p;
-    p.ns = blockIdx.y;
-    p.seg = (int)blockIdx.x * PM4_ROWS + (threadIdx.x >> 4);
+    const uint32_t row = blockIdx.x * PM4_ROWS + (threadIdx.x >> 4);
+    const uint32_t stride = (uint32_t)pm4_stride(nseg);
+    p.ns = row / stride;
+    p.seg = (int)(row % stride);
     p.l = threadIdx.x & 15;
-    p.live = p.seg < nseg;
+    p.live = p.ns < NS && p.seg < nseg;
     p.col = 4 * p.l < D;
     p.t0 = p.seg * tseg;
     p.t1 = min(T, p.t0 + tseg);
@@ -233,9 +242,9 @@ __device__ __forceinline__ void pm4_rows(const float *__restrict__ x, const Pm4P
 }
 
 __global__ __launch_bounds__(256) void k_pm4_reduce(const float *__restrict__ w, const float *__restrict__ v,
-                                                    double *__restrict__ delta, int64_t T, int D, int64_t tseg,
-                                                    int nseg) {
-    const Pm4Pos p = pm4_pos(T, D, tseg, nseg);
+                                                    double *__restrict__ delta, int64_t NS, int64_t T, int D,
+                                                    int64_t tseg, int nseg) {
+    const Pm4Pos p = pm4_pos(NS, T, D, tseg, nseg);
     if (!p.live) return;  // whole rows
     double B[4] = {0.0, 0.0, 0.0, 0.0}, A = 0.0;
     for (int64_t c = p.t0; c < p.t1; c += 16) {
@@ -257,9 +266,9 @@ __global__ __launch_bounds__(256) void k_pm4_reduce(const float *__restrict__ w,
 }
 
 __global__ __launch_bounds__(256) void k_pm4_out(const float *__restrict__ w, const float *__restrict__ v,
-                                                 float *__restrict__ E, const double *__restrict__ state, int64_t T,
-                                                 int D, int64_t tseg, int nseg, double eps) {
-    const Pm4Pos p = pm4_pos(T, D, tseg, nseg);
+                                                 float *__restrict__ E, const double *__restrict__ state, int64_t NS,
+                                                 int64_t T, int D, int64_t tseg, int nseg, double eps) {
+    const Pm4Pos p = pm4_pos(NS, T, D, tseg, nseg);
     if (!p.live) return;
     const double *st = state + (p.ns * (nseg + 1) + p.seg) * (int64_t)(D + 1);
     double B[4], A = st[D];
@@ -289,9 +298,9 @@ __global__ __launch_bounds__(256) void k_pm4_out(const float *__restrict__ w, co
 __global__ __launch_bounds__(256) void k_pm4_bw_fwd(const float *__restrict__ w, const float *__restrict__ v,
                                                     const float *__restrict__ gE, const double *__restrict__ state,
                                                     double *__restrict__ invA, double *__restrict__ alpha,
-                                                    double *__restrict__ rdelta, int64_t T, int D, int64_t tseg,
-                                                    int nseg, double eps) {
-    const Pm4Pos p = pm4_pos(T, D, tseg, nseg);
+                                                    double *__restrict__ rdelta, int64_t NS, int64_t T, int D,
+                                                    int64_t tseg, int nseg, double eps) {
+    const Pm4Pos p = pm4_pos(NS, T, D, tseg, nseg);
     if (!p.live) return;
     const double *st = state + (p.ns * (nseg + 1) + p.seg) * (int64_t)(D + 1);
     double B[4], bsum[4] = {0.0, 0.0, 0.0, 0.0}, A = st[D], asum = 0.0;
@@ -341,8 +350,9 @@ __global__ __launch_bounds__(256) void k_pm4_bw_rev(const float *__restrict__ w,
                                                     const float *__restrict__ gE, const double *__restrict__ invA,
                                                     const double *__restrict__ alpha,
                                                     const double *__restrict__ rstate, float *__restrict__ gW,
-                                                    float *__restrict__ gV, int64_t T, int D, int64_t tseg, int nseg) {
-    const Pm4Pos p = pm4_pos(T, D, tseg, nseg);
+                                                    float *__restrict__ gV, int64_t NS, int64_t T, int D, int64_t tseg,
+                                                    int nseg) {
+    const Pm4Pos p = pm4_pos(NS, T, D, tseg, nseg);
     if (!p.live) return;
     const double *rs = rstate + (p.ns * nseg + p.seg) * (int64_t)(D + 1);
     double beta[4], asuf = rs[D];

@@ -1114,15 +1114,15 @@ int race_prefix_mean_fwd(const float *w, const float *v, float *E, int64_t NS, i
     double *state = delta + NS * nseg * (D + 1);
     hipStream_t s = (hipStream_t)stream;
     const int elems = (int)(D + 1);
-    const dim3 grid(nseg, (unsigned)NS), rgrid((nseg + PM4_ROWS - 1) / PM4_ROWS, (unsigned)NS),
+    const dim3 grid(nseg, (unsigned)NS), rgrid((unsigned)((NS * pm4_stride(nseg) + PM4_ROWS - 1) / PM4_ROWS)),
         sgrid((elems + PM_SCAN_THREADS - 1) / PM_SCAN_THREADS, (unsigned)NS);
     if (rows)
-        k_pm4_reduce<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
+        k_pm4_reduce<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, delta, NS, T, (int)D, tseg, nseg);
     else
         k_pm_reduce<<<grid, 64, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
     k_pm_scan<<<sgrid, PM_SCAN_THREADS, 0, s>>>(state, delta, nseg, elems);
     if (rows)
-        k_pm4_out<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, E, state, T, (int)D, tseg, nseg, eps);
+        k_pm4_out<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, E, state, NS, T, (int)D, tseg, nseg, eps);
     else
         k_pm_out<<<grid, 64, 0, s>>>(w, v, E, state, T, (int)D, tseg, nseg, eps);
     return launched("race_prefix_mean_fwd");
@@ -1148,20 +1148,20 @@ int race_prefix_mean_bwd(const float *w, const float *v, const float *gE, float 
     double *rstate = rdelta + NS * nseg * (D + 1);
     hipStream_t s = (hipStream_t)stream;
     const int elems = (int)(D + 1);
-    const dim3 grid(nseg, (unsigned)NS), rgrid((nseg + PM4_ROWS - 1) / PM4_ROWS, (unsigned)NS),
+    const dim3 grid(nseg, (unsigned)NS), rgrid((unsigned)((NS * pm4_stride(nseg) + PM4_ROWS - 1) / PM4_ROWS)),
         sgrid((elems + PM_SCAN_THREADS - 1) / PM_SCAN_THREADS, (unsigned)NS);
     if (rows)
-        k_pm4_reduce<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
+        k_pm4_reduce<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, delta, NS, T, (int)D, tseg, nseg);
     else
         k_pm_reduce<<<grid, 64, 0, s>>>(w, v, delta, T, (int)D, tseg, nseg);
     k_pm_scan<<<sgrid, PM_SCAN_THREADS, 0, s>>>(state, delta, nseg, elems);
     if (rows)
-        k_pm4_bw_fwd<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, gE, state, invA, alpha, rdelta, T, (int)D, tseg, nseg, eps);
+        k_pm4_bw_fwd<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, gE, state, invA, alpha, rdelta, NS, T, (int)D, tseg, nseg, eps);
     else
         k_pm_bw_fwd<<<grid, 64, 0, s>>>(w, v, gE, state, invA, alpha, rdelta, T, (int)D, tseg, nseg, eps);
     k_pm_rscan<<<sgrid, PM_SCAN_THREADS, 0, s>>>(rstate, rdelta, nseg, elems);
     if (rows)
-        k_pm4_bw_rev<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, gE, invA, alpha, rstate, gW, gV, T, (int)D, tseg, nseg);
+        k_pm4_bw_rev<<<rgrid, 16 * PM4_ROWS, 0, s>>>(w, v, gE, invA, alpha, rstate, gW, gV, NS, T, (int)D, tseg, nseg);
     else
         k_pm_bw_rev<<<grid, 64, 0, s>>>(w, v, gE, invA, alpha, rstate, gW, gV, T, (int)D, tseg, nseg);
     return launched("race_prefix_mean_bwd");

@@ -33,7 +33,9 @@ def _both(w, v, gE, eps):
 
 
 @pytest.mark.parametrize("NS,T,D", [(1, 1, 4), (3, 15, 64), (2, 16, 8), (5, 17, 60), (2, 31, 64), (1, 33, 64),
-                                    (40, 513, 12), (1, 70001, 64), (3000, 18, 32)])
+                                    (40, 513, 12), (1, 70001, 64), (3000, 18, 32),
+                                    # rows of several streams in one workgroup: 24 and 11 segments a stream, 2, and 1
+                                    (700, 600, 64), (1500, 170, 20), (16390, 20, 16), (9001, 37, 64)])
 def test_rows_and_general_kernels_agree(dev, oracle, NS, T, D):
     g = torch.Generator().manual_seed(NS + 3 * T + 7 * D)
     w = torch.rand(NS, T, generator=g)
