@@ -53,11 +53,13 @@ constexpr int64_t kLongSegTiles = 64;
 // the state of an automatic forward is also that of seg_tiles = 1, which
 // backward calls with either are used with.
 constexpr int64_t kOneTileBlocks = 1024;
-// Resident workgroups (256 CUs) of the forward and of the backward tile kernels
-// by slice size: 8-, 4- and 2-wave workgroups.  The backward of 128 buckets and
-// the fp32 kernels hold one 8-wave workgroup per CU; the bf16 backward of 64
-// and 32 buckets holds two and four, and half a round more measured the same or
-// better (K=4 L=4 48 x 8192 global: 768 workgroups 350 us, 384 401).
+// Workgroups that a launch of the forward and of the backward tile kernels aims
+// at, by slice size (8-, 4- and 2-wave workgroups; 256 CUs).  128 buckets: what is
+// resident, two per CU in the bf16 forward, one in the backward and in fp32.  Fewer
+// buckets: more than is resident where that measured the same or better -- the
+// causal bf16 backward holds two workgroups of 64 buckets per CU, and of 32 two
+// (k_bwd_out, one wave per SIMD) or three (k_bwd_reduce), the fp32 one of either
+// one or two (K=4 L=4 48 x 8192 global: 768 workgroups 350 us, 384 401).
 // The non-causal forward of 32 buckets holds six (fp32 four), forward us with
 // the causal operator's four (fp32 two) and with these: bf16 K=2 L=5 384 x 785
 // 75 -> 70, 576 x 197 54 -> 49, K=3 L=4 32 x 16384 105 -> 98, fp32 48 x 3000
@@ -118,13 +120,44 @@ void slice_plan(int dtype, int K, int S, int &SP, int &nslice) {
 // Work-items of a 1-D launch: the dispatch packet counts them in 32 bits.
 constexpr int64_t kMaxWorkItems = 0xFFFFFFFFll;
 
+// Workgroups of a launch over nseg segments a stream, as the busiest XCD sees it
+// times 8: the workgroups go round the 8 XCDs (32 CUs each), those of a sliced
+// launch in groups of the slices of one segment (K=6 L=5, 3 slices, 7 streams of
+// 12 segments are 252 workgroups, but 33 on four XCDs: a second round).
+int64_t launch_wgs(const Plan &p, int64_t nseg) { return (nseg * p.N + 7) / 8 * 8 * p.nslice; }
+// Time, in tiles, of a launch of wgs workgroups that walk `tiles` tiles, r of
+// them resident per CU: whole rounds, and a last one with fewer per CU, which
+// run faster for it.
+double rounds_cost(int64_t wgs, int64_t r, int64_t tiles) {
+    const int64_t n = (wgs + 255) / 256, rem = n % r;
+    return ((double)(n / r) + (rem ? 0.5 + 0.5 * (double)rem / (double)r : 0.0)) * (double)(tiles + 2);
+}
+
+// The causal backward of 128 buckets runs one workgroup per CU: of the joins of 1
+// to `most` of fnseg forward segments (tps tiles each) into one backward segment,
+// the one whose launch takes the fewest tiles in whole rounds, and those tiles.
+double whole_rounds(const Plan &p, int64_t fnseg, int64_t tps, int64_t most, int64_t &join) {
+    double cost = 1e300;
+    for (int64_t j = 1; j <= most && j <= fnseg; ++j) {
+        const double c = rounds_cost(launch_wgs(p, (fnseg + j - 1) / j), 1, j * tps);
+        if (c < cost) {
+            cost = c;
+            join = j;
+        }
+    }
+    return cost;
+}
+
 // Tiles per segment of a short sequence: 1 to 4 rounds of target_blocks
 // workgroups (non-causal: half of one too, where that saves one-tile segments),
 // whichever the cost in tiles -- per round a segment and 2 tiles of set-up, per
 // workgroup its state passes (none read per segment by the non-causal operator:
 // half) -- says is shortest.  One 8-wave workgroup per CU
 // only where that leaves segments of 8 tiles: the backward then still joins
-// pairs of forward segments.
+// pairs of forward segments.  With 128 causal buckets the backward's rounds count
+// too, at twice the forward's time a tile: one forward segment would leave it no
+// choice (K=6 L=5, 3 slices, 96 streams x 1000, us, forward and backward: one
+// segment 184 and 530, three 156 and 420).
 int64_t short_tiles(const race_desc *d, const Plan &p, int64_t per) {
     int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, false, d->causal);
     if (tb < 512 && p.ntiles * per < 8 * tb) tb = 512;
@@ -137,13 +170,55 @@ int64_t short_tiles(const race_desc *d, const Plan &p, int64_t per) {
         nseg = nseg < 1 ? 1 : (nseg > p.ntiles ? p.ntiles : nseg);
         const int64_t tps = (p.ntiles + nseg - 1) / nseg;
         nseg = (p.ntiles + tps - 1) / tps;
-        const double c = (double)((nseg * per + tb - 1) / tb) * (double)(tps + 2) + (double)(nseg * per) * row;
+        double c = (double)((launch_wgs(p, nseg) + tb - 1) / tb) * (double)(tps + 2) + (double)(nseg * per) * row;
+        int64_t join;
+        if (d->causal && p.SP == 128) c += 2 * whole_rounds(p, nseg, tps, kMaxSegTiles / tps, join);
         if (c < cost) {
             cost = c;
             best = tps;
         }
     }
     return best;
+}
+
+// Tiles per backward segment of the non-causal operator (no more segments than the
+// forward's).  Backward, us, with one
+// residency of segments by target_blocks alone, and with this: K=3 L=8 16 x 65536
+// 397, 322; K=6 L=5 (3 slices) 48 x 8192 1178, 802.
+int64_t own_tiles(const race_desc *d, const Plan &p, int64_t per, bool capped) {
+    const bool bf = d->dtype == RACE_DTYPE_BF16;
+    // 64 buckets in bf16: 16-column rows (K = 4) leave LDS for a third workgroup
+    const int64_t r = bf && p.SP == 64 ? (d->K == 4 ? 3 : 2) : target_blocks(bf, p.SP, true, false) / 256;
+    const int64_t most = 4 * 256 * r / per + 1;
+    int64_t best = 0;
+    double cost = 1e300;
+    for (int64_t nseg = 1; nseg <= most && nseg <= p.fnseg; ++nseg) {
+        int64_t tl = (p.ntiles + nseg - 1) / nseg;
+        if (capped && tl > kMaxSegTiles) tl = kMaxSegTiles;
+        const double c = rounds_cost(launch_wgs(p, (p.ntiles + tl - 1) / tl), r, tl);
+        if (c < cost) {
+            cost = c;
+            best = tl;
+        }
+    }
+    return best;
+}
+
+// Forward segments per backward segment of the causal operator, at most `most`.
+// 128 buckets: whole_rounds.  The others take the fewest segments that fill
+// target_blocks; of the counts that leave as many, the smallest, so that the last
+// is not a short one.  Backward of 48 streams x 8192,
+// us, the fewest that fill one residency and with this: K=6 L=5 2534, 1266, K=7 L=4
+// 3230, 1620.
+int64_t joined_segments(const race_desc *d, const Plan &p, int64_t per, int64_t most) {
+    const int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, true, true);
+    if (most > p.fnseg) most = p.fnseg;
+    int64_t m = (p.fnseg * per + tb - 1) / tb;
+    if (p.SP == 128) whole_rounds(p, p.fnseg, p.tps, most, m);
+    if (m > most) m = most;
+    if (m < 1) return 1;
+    const int64_t nb = (p.fnseg + m - 1) / m;
+    return (p.fnseg + nb - 1) / nb;
 }
 
 // bwd: the backward's plan (longer segments of whole forward ones, at most
@@ -219,21 +294,15 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true, 
         // (a segment is at most kMaxSegTiles long: m * tps tiles, or the whole
         // sequence when that is shorter)
         // The non-causal backward reads no state row but the totals, so its
-        // segments are its own: one residency of them.
-        const int64_t tb = target_blocks(d->dtype == RACE_DTYPE_BF16, p.SP, true, d->causal);
+        // segments are its own.
+        const int64_t per = p.N * p.nslice;
+        const bool capped = walks && p.ntiles > kMaxSegTiles;
         if (!d->causal) {
-            int64_t nb = tb / (p.N * p.nslice);
-            nb = nb < 1 ? 1 : (nb > p.ntiles ? p.ntiles : nb);
-            int64_t tl = (p.ntiles + nb - 1) / nb;
-            if (walks && tl > kMaxSegTiles) tl = kMaxSegTiles;
-            p.tps = (int)tl;
-            p.nseg = (int)((p.ntiles + tl - 1) / tl);
-        }
-        int64_t m = !d->causal ? 1 : ((int64_t)p.fnseg * p.N * p.nslice + tb - 1) / tb;
-        if (walks && p.ntiles > kMaxSegTiles && m > kMaxSegTiles / p.tps) m = kMaxSegTiles / p.tps;
-        if (m > 1) {
+            p.tps = (int)own_tiles(d, p, per, capped);
+            p.nseg = (int)((p.ntiles + p.tps - 1) / p.tps);
+        } else if (const int64_t m = joined_segments(d, p, per, capped ? kMaxSegTiles / p.tps : p.fnseg); m > 1) {
             const int64_t tl = (int64_t)p.tps * m;
-            p.fmul = m < p.fnseg ? (int)m : p.fnseg;
+            p.fmul = (int)m;
             p.tps = (int)(tl < p.ntiles ? tl : p.ntiles);
             p.nseg = (int)((p.ntiles + p.tps - 1) / p.tps);
         }
