@@ -3556,12 +3556,15 @@ void k_bwd_out(Args a) {
 // forward: 3) write more streams at once and are slower; the layout is padded
 // to that many.  Forward + backward, 16 x 65536, us: K=4 L=8 391 with registers,
 // 376 with rows, K=4 L=4 245 and 229; at K=2 L=5 registers 170, rows 243, K=3 L=2
-// 157 and 230, K=3 L=8 237 and 238; fp32 K=4 L=8 8 x 65536 230 and 781.
-template <typename T, int SP, int KB> __host__ __device__ constexpr bool probs_planes_reg() {
-    return !(is_bf16<T>() && KB == 4 && SP >= 64);
+// 157 and 230, K=3 L=8 237 and 238; fp32 K=4 L=8 8 x 65536 230 and 781.  Rows too
+// in the 128-bucket backward of 3 and 6 bits, whose registers cost a workgroup per
+// CU (89 and 95 VGPRs, 2 in place of 3): K=3 L=10 200 with registers, 179 with
+// rows, K=6 L=5 790 and 672; 5, 7 and 8 bits run 2 either way (K=7 L=4 930, 999).
+template <typename T, int SP, int KB, bool BWD> __host__ __device__ constexpr bool probs_planes_reg() {
+    return !(is_bf16<T>() && (SP == 128 && BWD ? KB == 3 || KB == 4 || KB == 6 : KB == 4 && SP >= 64));
 }
 template <typename T, int SP, int KB, bool BWD> struct ProbsL {
-    using PS = PlaneSrc<T, NatL<T, true>, probs_planes_reg<T, SP, KB>()>;
+    using PS = PlaneSrc<T, NatL<T, true>, probs_planes_reg<T, SP, KB, BWD>()>;
     static constexpr int NW_ = SP / WB, NC = ncol_of<SP, KB>();
     static constexpr int LDN = NatL<T, true>::LD, LDC = ld_of<float>(NC), LDDP = sw_ld<T, NCOL>();
     static constexpr size_t oX = 0;

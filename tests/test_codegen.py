@@ -70,3 +70,22 @@ def test_no_mixed_depth_srcc_chain(tmp_path):
     assert "v_mfma_f32_16x16x16_bf16" not in asm
     bad = mixed_srcc_chains(asm)
     assert not bad, bad[:5]
+
+
+def _vgprs(name):
+    """VGPRs of a kernel of the built library, from the metadata its code object carries."""
+    from race_attention_amd import _lib
+    with open(_lib.LIB_PATH, "rb") as f:
+        blob = f.read()
+    # MessagePack maps with sorted keys: .name, a string, ..., .vgpr_count, an integer below 128 or a byte after 0xcc
+    m = re.search(rb"\.name.{1,2}" + name.encode() + rb".{1,400}?\.vgpr_count(\xcc.|[\x00-\x7f])", blob, re.S)
+    assert m, name
+    return m.group(1)[-1]
+
+
+@pytest.mark.parametrize("KB,workgroups", [(3, 3), (4, 4), (6, 3)])
+def test_probability_backward_keeps_its_workgroups(KB, workgroups):
+    """The bf16 backward of 128 buckets: 8-wave workgroups per CU that its
+    registers allow (512 a SIMD lane in steps of 8, 4 SIMDs)."""
+    vgprs = _vgprs(f"_ZN4race7k_probsIDF16bLi128ELi{KB}ELb1EEEvNS_4ArgsE")
+    assert vgprs <= 512 // (2 * workgroups) // 8 * 8, vgprs
