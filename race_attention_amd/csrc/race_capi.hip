@@ -84,10 +84,6 @@ constexpr int64_t kMaxSegTiles = 256;
 
 struct Plan {
     int SP = 0, S = 0, R = 0, nslice = 1, Spad = 0;
-    // slices that the buffer sizes count: fp32 buffers keep the room of
-    // 32-bucket slices' partial outputs, which programs may have sized by that
-    // rule, also where one workgroup holds all buckets
-    int wslice = 0;
     bool parts = false;  // partial outputs + slice sum (sliced<KB>() instantiations)
     int64_t N = 0, ntiles = 0;
     int nseg = 0, tps = 0;
@@ -253,7 +249,8 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true, 
     p.R = 1 << d->K;
     p.S = d->L * p.R;
     slice_plan(d->dtype, d->K, p.S, p.SP, p.nslice);
-    p.Spad = p.nslice * p.SP;
+    // (fp32: the rows of 65 to 96 buckets in a workgroup of 128 stay 96, StateRows)
+    p.Spad = d->dtype == RACE_DTYPE_F32 && p.nslice == 1 ? (p.S + 31) / 32 * 32 : p.nslice * p.SP;
     p.parts = d->K > 4;
     p.N = d->M * d->B * d->H;
     if (p.N > 65535) return fail(RACE_E_UNSUPPORTED, "M*B*H=%lld streams exceed 65535", (long long)p.N);
@@ -314,15 +311,15 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true, 
         return fail(RACE_E_UNSUPPORTED, "M*B*H*T=%lld token-heads exceed one dX launch's 2^32 work-items",
                     (long long)(p.N * d->T));
     const bool f32 = d->dtype == RACE_DTYPE_F32;
-    p.wslice = f32 ? (p.S + 31) / 32 : (p.parts ? p.nslice : 0);
-    p.part_bytes = align16((size_t)p.wslice * p.N * d->T * D * p.esize);
+    const int parts = p.parts ? p.nslice : 0;  // slices that leave partial outputs
+    p.part_bytes = align16((size_t)parts * p.N * d->T * D * p.esize);
     const size_t xesize = xpart_f32(!f32, p.SP, d->K) ? sizeof(float) : p.esize;
-    p.xpart_bytes = align16((size_t)p.wslice * p.N * d->T * xcols_of(f32 ? 32 : p.SP, d->K) * xesize);
+    p.xpart_bytes = align16((size_t)parts * p.N * d->T * xcols_of(p.SP, d->K) * xesize);
     p.fws = p.fws_core + p.part_bytes;                         // partial O
     p.bws = p.bws_core + 2 * p.xpart_bytes + p.part_bytes;     // dproj columns for dQ, dK; partial dV
     p.tok_bytes = align16((size_t)p.N * d->T * sizeof(float));
-    p.gfws = p.fws + p.wslice * p.tok_bytes;
-    p.gbws = p.bws + (2 + p.wslice) * p.tok_bytes;  // + the slices' gsum
+    p.gfws = p.fws + parts * p.tok_bytes;
+    p.gbws = p.bws + (2 + parts) * p.tok_bytes;  // + the slices' gsum
     return RACE_OK;
 }
 
@@ -843,7 +840,16 @@ int scratch_address(void **out) {
 }
 
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-size_t noalloc_need(const Plan &p) { return align256(p.state_bytes) + p.fws; }
+// What a call is measured by: its state and workspace, and in fp32 the partial
+// outputs of slices of 32 buckets also where one workgroup holds all of them and
+// there are none.  That keeps the calls that this entry takes, and those it sends
+// to race_fwd, what they have been.
+size_t noalloc_parts(const race_desc *d, const Plan &p) {
+    return d->dtype == RACE_DTYPE_F32 ? align16((size_t)((p.S + 31) / 32) * p.N * d->T * D * sizeof(float)) : p.part_bytes;
+}
+size_t noalloc_need(const race_desc *d, const Plan &p) {
+    return align256(p.state_bytes) + p.fws_core + noalloc_parts(d, p);
+}
 
 // Plan of the no-allocation forward: the descriptor's seg_tiles if set, else
 // the default segmentation, coarsened (longer segments) until the state and
@@ -854,22 +860,21 @@ int noalloc_plan(const race_desc *d, race_desc &dd, Plan &p) {
     dd = *d;
     int rc = make_plan(&dd, p, false, false);
     if (rc) return rc;
-    if (d->seg_tiles <= 0 && noalloc_need(p) > RACE_NOALLOC_SCRATCH_BYTES) {
+    if (d->seg_tiles <= 0 && noalloc_need(d, p) > RACE_NOALLOC_SCRATCH_BYTES) {
         // state (nseg + 1 rows) and sums (nseg rows) of N * Spad * (D+1) fp64 each
         const size_t row = (size_t)p.N * p.Spad * SROW * sizeof(double);
-        const size_t fixed = p.part_bytes + row + 512;
+        const size_t fixed = noalloc_parts(d, p) + row + 512;
         const int64_t nseg = fixed < RACE_NOALLOC_SCRATCH_BYTES
                                  ? (int64_t)((RACE_NOALLOC_SCRATCH_BYTES - fixed) / (2 * row)) : 0;
-        if (nseg >= 1) {
-            dd.seg_tiles = (int32_t)((p.ntiles + nseg - 1) / nseg);
-            if ((rc = make_plan(&dd, p, false, false))) return rc;
-        }
+        dd.seg_tiles = (int32_t)(nseg > 1 ? (p.ntiles + nseg - 1) / nseg : p.ntiles);
+        if ((rc = make_plan(&dd, p, false, false))) return rc;
     }
-    if (noalloc_need(p) > RACE_NOALLOC_SCRATCH_BYTES)
+    if (noalloc_need(d, p) > RACE_NOALLOC_SCRATCH_BYTES)
         return fail(RACE_E_UNSUPPORTED,
                     "race_fwd_noalloc: this call needs %zu bytes of scratch (state %zu, segment sums and partial "
                     "outputs %zu); the no-allocation forward holds %zu -- use race_fwd with caller buffers",
-                    noalloc_need(p), p.state_bytes, p.fws, (size_t)RACE_NOALLOC_SCRATCH_BYTES);
+                    noalloc_need(d, p), p.state_bytes, p.fws_core + noalloc_parts(d, p),
+                    (size_t)RACE_NOALLOC_SCRATCH_BYTES);
     return RACE_OK;
 }
 

@@ -62,7 +62,7 @@ struct Args {
     // forward segments (fstate rows per stream - 1) and forward segments per
     // segment: the backward's segment s starts at forward boundary s * fmul
     int fnseg, fmul;
-    int nslice, Spad;  // bucket slices (grid z) of SP buckets each; Spad = nslice * SP
+    int nslice, Spad;  // bucket slices (grid z) of SP buckets each; rows of buckets in the state (StateRows)
     double *fstate;  // [N][fnseg+1][Spad][D+1] exclusive forward-segment prefixes; [fnseg] = totals
     double *fdelta;  // [N][nseg][Spad][D+1], streams fdrows rows apart
     int fdrows;
@@ -1623,6 +1623,21 @@ template <int NTH> __device__ double block_sum_f64(double v, float *scratch) {
 // state row index of (bucket s, column d)
 __device__ __forceinline__ int64_t sidx(int s, int d) { return (int64_t)s * SROW + d; }
 
+// The state rows of a wave's buckets sg .. sg+15.  The state holds nslice * SP
+// rows, but of fp32's 65 to 96 buckets in a workgroup of 128 only 96 (the rows of
+// three slices of 32): the last two waves, whose buckets are padding and whose
+// sums are zero, load row 0 in their place, as zeros, and store nothing.
+template <typename T, int SP> struct StateRows {
+    static constexpr bool ALL = is_bf16<T>() || SP < 128;
+    bool live;
+    int s0;  // first row
+    __device__ __forceinline__ StateRows(int sg, int rows) : live(ALL || sg < rows), s0(live ? sg : 0) {}
+    template <typename V> __device__ __forceinline__ V operator()(const V *st, int s, int d) const {
+        const V x = st[sidx(s0 + s, d)];
+        return live ? x : V(0);
+    }
+};
+
 // Waves per SIMD that the forward tile kernels are compiled for: their LDS
 // allows this many and more, so the register bound is what decides.
 __host__ __device__ constexpr int fwd_waves(bool bf, int SP) { return bf ? (SP == 128 ? 4 : 3) : 2; }
@@ -1853,6 +1868,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
         }
     }
     double *out = a.fdelta + ((int64_t)n * a.fdrows + seg) * a.Spad * SROW;
+    if (!StateRows<T, SP>(sg, a.Spad).live) return;
     for (int md = 0; md < 4; ++md)
         for (int e = 0; e < 4; ++e)
             out[sidx(sg + i, 16 * md + 4 * g + e)] = BM ? (double)accBm[md][e] : accB[md][e];
@@ -2125,11 +2141,12 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
     // carried state: causal = prefix at the segment start, non-causal = totals.
     // B in bucket-row layout: lane holds B[s = sw + 4g + e][d = 16md + i]
     const double *st = a.fstate + ((int64_t)n * (a.fnseg + 1) + (CAUSAL ? seg * a.fmul : a.fnseg)) * a.Spad * SROW;
+    const StateRows<T, SP> rows(sg, a.Spad);
     f32x4 Bc[4];
     CarryA<T> a0[4];  // A at the tile start
     for (int e = 0; e < 4; ++e) {
-        for (int md = 0; md < 4; ++md) Bc[md][e] = (float)st[sidx(sg + 4 * g + e, 16 * md + i)];
-        a0[e] = (CarryA<T>)st[sidx(sg + 4 * g + e, D)];
+        for (int md = 0; md < 4; ++md) Bc[md][e] = (float)rows(st, 4 * g + e, 16 * md + i);
+        a0[e] = (CarryA<T>)rows(st, 4 * g + e, D);
     }
     if constexpr (!CAUSAL) store_ds<T, SP>(sBT, sw, Bc);  // constant totals
 
@@ -2562,15 +2579,16 @@ void k_bwd_reduce(Args a) {
     zero_lds<T>(sDproj, TT * LDDP, NTH);
     // forward state in d-row layout: lane holds B^T[d = 16md + 4g + e][s = sw + i]
     const double *st = a.fstate + ((int64_t)n * (a.fnseg + 1) + (CAUSAL ? seg * a.fmul : a.fnseg)) * a.Spad * SROW;
+    const StateRows<T, SP> rows(sg, a.Spad);
     f32x4 Bt[4], Ut[4];
     CarryA<T> a0[4];  // A at the tile start
     double al[4];
     for (int md = 0; md < 4; ++md) {
         Ut[md] = zero4();
-        for (int e = 0; e < 4; ++e) Bt[md][e] = (float)st[sidx(sg + i, 16 * md + 4 * g + e)];
+        for (int e = 0; e < 4; ++e) Bt[md][e] = (float)rows(st, i, 16 * md + 4 * g + e);
     }
     for (int e = 0; e < 4; ++e) {
-        a0[e] = (CarryA<T>)st[sidx(sg + 4 * g + e, D)];
+        a0[e] = (CarryA<T>)rows(st, 4 * g + e, D);
         al[e] = 0.0;
     }
     CarryA<T> tsum = 0;  // this thread's share of sum du * th
@@ -2830,10 +2848,11 @@ void k_bwd_reduce(Args a) {
         dx_store<T, NW_, XC, AL, XF>(sDproj, sPlT, dqp, a.sg.t, (int64_t)(j1 - 1) * TT, a.T, xpart, xc0);
     }
     float *out = a.rdelta + ((int64_t)n * a.nseg + seg) * a.Spad * SROW;
-    for (int md = 0; md < 4; ++md)
-        for (int e = 0; e < 4; ++e) out[sidx(sg + i, 16 * md + 4 * g + e)] = Ut[md][e];
+    if (rows.live)
+        for (int md = 0; md < 4; ++md)
+            for (int e = 0; e < 4; ++e) out[sidx(sg + i, 16 * md + 4 * g + e)] = Ut[md][e];
     for (int e = 0; e < 4; ++e) al[e] = row_sum_f64(al[e]);
-    if (i == 0)
+    if (i == 0 && rows.live)
         for (int e = 0; e < 4; ++e) out[sidx(sg + 4 * g + e, D)] = (float)al[e];
     const double ts = block_sum_f64<NTH>((double)tsum, sRed);
     if (threadIdx.x == 0) a.tpart[((int64_t)n * a.nseg + seg) * a.nslice + z] = ts;
@@ -3124,6 +3143,7 @@ void k_bwd_out(Args a) {
     const float *rs = a.rstate + ((int64_t)n * a.nseg + (CAUSAL ? seg : 0)) * a.Spad * SROW;
     const double *fs =
         a.fstate + ((int64_t)n * (a.fnseg + 1) + min((seg + 1) * a.fmul, a.fnseg)) * a.Spad * SROW;
+    const StateRows<T, SP> rows(sg, a.Spad);
     f32x4 Ut[4];  // U^T[d = 16md + 4g + e][s = sw + i]
     // Forward state, walked back from the segment end.  B only feeds the
     // G product's operand: the whole-tile bf16 instantiations carry it in
@@ -3137,16 +3157,15 @@ void k_bwd_out(Args a) {
     constexpr bool FSTATE = CAUSAL && !GN;
     for (int md = 0; md < 4; ++md)
         for (int e = 0; e < 4; ++e) {
-            const int64_t r = sidx(sg + i, 16 * md + 4 * g + e);
-            Ut[md][e] = rs[r];
+            Ut[md][e] = rows(rs, i, 16 * md + 4 * g + e);
             if constexpr (BM)
-                Bm[md][e] = FSTATE ? (float)fs[r] : 0.f;
+                Bm[md][e] = FSTATE ? (float)rows(fs, i, 16 * md + 4 * g + e) : 0.f;
             else
-                Be[md][e] = FSTATE ? fs[r] : 0.0;
+                Be[md][e] = FSTATE ? rows(fs, i, 16 * md + 4 * g + e) : 0.0;
         }
     for (int e = 0; e < 4; ++e) {
-        al[e] = rs[sidx(sg + 4 * g + e, D)];
-        Ae[e] = FSTATE ? fs[sidx(sg + 4 * g + e, D)] : 0.0;
+        al[e] = rows(rs, 4 * g + e, D);
+        Ae[e] = FSTATE ? rows(fs, 4 * g + e, D) : 0.0;
     }
     if constexpr (!CAUSAL) store_ut<T, SP>(sUT, sw, Ut, cst, po);  // constant totals
     CarryA<T> tsum = 0;  // this thread's share of sum du * th

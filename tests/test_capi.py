@@ -168,8 +168,8 @@ def _plan(**kw):
 
 
 @pytest.mark.parametrize("dtype,K,L,M,B,H,T,spad", [
-    # fp32: slices of 32 buckets, L*2^K = 128 -> 4 slices
-    (_lib.RACE_DTYPE_F32, 4, 8, 1, 1, 8, 4096, 128),
+    # fp32, 2^K > 16: slices of 32 buckets, L*2^K = 128 -> 4 slices
+    (_lib.RACE_DTYPE_F32, 5, 4, 1, 1, 8, 4096, 128),
     # bf16, 2^K > 16: slices of 128 buckets; the decoder config's K=8, L=4
     # (1024 buckets, 8 slices), M=2 estimators, 8 x 12 heads
     (_lib.RACE_DTYPE_BF16, 8, 4, 2, 8, 12, 8192, 1024),
@@ -299,11 +299,40 @@ def test_global_workspace_sizes():
     tok = N * T * 4
     assert lib.race_fwd_global_workspace_bytes(ctypes.byref(d)) == lib.race_fwd_workspace_bytes(ctypes.byref(d))
     assert lib.race_bwd_global_workspace_bytes(ctypes.byref(d)) == lib.race_bwd_workspace_bytes(ctypes.byref(d)) + 2 * tok
-    d = _desc(dtype=_lib.RACE_DTYPE_F32, T=4096)      # 4 slices of 32 buckets
+    d = _desc(dtype=_lib.RACE_DTYPE_F32, T=4096)      # one workgroup: as bf16
+    assert lib.race_fwd_global_workspace_bytes(ctypes.byref(d)) == lib.race_fwd_workspace_bytes(ctypes.byref(d))
+    assert (lib.race_bwd_global_workspace_bytes(ctypes.byref(d)) ==
+            lib.race_bwd_workspace_bytes(ctypes.byref(d)) + 2 * N * 4096 * 4)
+    d = _desc(dtype=_lib.RACE_DTYPE_F32, T=4096, K=5, L=4)  # 4 slices of 32 buckets
     f1 = lib.race_fwd_workspace_bytes(ctypes.byref(d))
     assert lib.race_fwd_global_workspace_bytes(ctypes.byref(d)) == f1 + 4 * N * 4096 * 4
     b1 = lib.race_bwd_workspace_bytes(ctypes.byref(d))
     assert lib.race_bwd_global_workspace_bytes(ctypes.byref(d)) == b1 + (2 + 4) * N * 4096 * 4
+
+
+def test_fp32_workspaces_hold_what_the_kernels_use():
+    """Up to 4 hash bits fp32 runs one workgroup for all buckets, so there are no
+    slices' partial outputs to hold; the state has a row for every 32 buckets in
+    use, 96 of a workgroup of 128 too; wider tables still hold the partials."""
+    lib = _lib.load()
+    for K, L, rows in ((4, 8, 128), (4, 6, 96), (3, 9, 96), (4, 4, 64), (2, 5, 32)):
+        d = _desc(dtype=_lib.RACE_DTYPE_F32, T=4096, L=L, K=K, seg_tiles=16)
+        seg = 8 * rows * 65 * 8  # a segment's sums of 8 streams, fp64
+        assert lib.race_state_bytes(ctypes.byref(d)) == 9 * seg
+        assert lib.race_fwd_workspace_bytes(ctypes.byref(d)) == 8 * seg
+        assert lib.race_bwd_workspace_bytes(ctypes.byref(d)) == 8 * seg + 16 * 8 * 8
+    d = _desc(dtype=_lib.RACE_DTYPE_F32, T=4096, K=8, L=1, seg_tiles=16)
+    assert lib.race_fwd_workspace_bytes(ctypes.byref(d)) == 8 * 8 * 256 * 65 * 8 + 8 * 8 * 4096 * 64 * 4
+
+
+def test_noalloc_takes_and_refuses_what_it_did():
+    """fp32 counts slices of 32 buckets and 96 state rows for 65 to 96 buckets: the
+    bytes at which a call goes to race_fwd (the checks come before the NULL ones)."""
+    lib = _lib.load()
+    refused = lambda **kw: (lib.race_fwd_noalloc(ctypes.byref(_desc(dtype=_lib.RACE_DTYPE_F32, **kw)),  # noqa: E731
+                                                 *[None] * 6) == -2 and "use race_fwd" in _lib.last_error())
+    assert not refused(H=384, T=32, K=4, L=6) and refused(H=440, T=32, K=4, L=6)
+    assert not refused(H=8, T=7000, K=4, L=8) and refused(H=8, T=8192, K=4, L=8)
 
 
 @pytest.mark.parametrize("field,value,code,msg", [

@@ -50,3 +50,41 @@ def test_bucket_counts_global_fp32(dev, K, L):
         e = relerr(to64(a), b)
         print(f"[global fp32 K={K} L={L}] {nm} {e:.2e}", flush=True)
         assert e <= TOL[torch.float32], nm
+
+
+@pytest.mark.parametrize("K,L", [(4, 6), (3, 9)])
+@pytest.mark.parametrize("causal", [1, 0])
+def test_buffers_of_65_to_96_fp32_buckets(dev, K, L, causal):
+    """96 state rows for a workgroup of 128 buckets: buffers of exactly the sizes
+    asked for, full of NaN, in front of guard words that stay as they are."""
+    import ctypes
+
+    from race_attention_amd import _lib
+    from race_attention_amd.functional import _strides4, make_desc
+    lib, T, B = _lib.load(), 230, 2
+    q, k, v, do, planes = make_case(B=B, T=T, H=3, L=L, K=K, dtype=torch.float32, seed=K)
+    x = [t.to(dev) for t in (q, k, v, do)]
+    pd = planes.to(dev).contiguous()
+    d = make_desc(*x[:3], pd, L=L, K=K, causal=causal, eps=1e-6, inv_temp=0.3, seg_tiles=2)
+    d.o_stride = d.do_stride = d.g_stride = _strides4(x[0])
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def buf(n):
+        b = torch.full(((n + 7) // 8 + 4096,), float("nan"), dtype=torch.float64, device=dev)
+        b[(n + 7) // 8:] = 123.0
+        return b, n
+
+    state, wf, wb = [buf(f(ctypes.byref(d))) for f in (lib.race_state_bytes, lib.race_fwd_workspace_bytes,
+                                                       lib.race_bwd_workspace_bytes)]
+    out, dq, dk, dv = [torch.empty_like(x[0]) for _ in range(4)]
+    git = torch.empty((), device=dev)
+    _lib.check(lib.race_fwd(ctypes.byref(d), *map(P, x[:3]), P(pd), P(out), P(state[0]), P(wf[0]), wf[1], st), "fwd")
+    _lib.check(lib.race_bwd(ctypes.byref(d), *map(P, x[:3]), P(pd), P(x[3]), P(state[0]), P(dq), P(dk), P(dv), P(git),
+                            P(wb[0]), wb[1], st), "bwd")
+    torch.cuda.synchronize()
+    for b, n in (state, wf, wb):
+        assert (b[(n + 7) // 8:] == 123.0).all()
+    ref = run_oracle(q, k, v, do, planes, causal=bool(causal), inv_temp=0.3)
+    gpu = [t.cpu() for t in (out, dq, dk, dv)] + [float(git)]
+    compare(f"rows K={K} L={L} causal={causal}", gpu, ref, TOL[torch.float32])

@@ -152,9 +152,11 @@ def test_noalloc_automatic_segmentation_fits(dev):
 
 
 @pytest.mark.gpu
-def test_noalloc_fp32_partials_in_scratch(dev):
-    """fp32 runs bucket slices whose fp32 partial outputs also live in the array."""
-    L, K, T, H = 5, 3, 1000, 2
+@pytest.mark.parametrize("L,K", [(5, 3), (3, 5)])
+def test_noalloc_fp32_partials_in_scratch(dev, L, K):
+    """fp32 runs one workgroup for all buckets of 3 bits, and at 5 bits bucket
+    slices whose fp32 partial outputs also live in the array."""
+    T, H = 1000, 2
     q, k, v, do, planes = make_case(B=2, T=T, H=H, L=L, K=K, dtype=torch.float32, unit=False, seed=5)
     qd, kd, vd = [x.to(dev) for x in (q, k, v)]
     pd = planes.to(dev).float().contiguous()
@@ -167,9 +169,9 @@ def test_noalloc_fp32_partials_in_scratch(dev):
 
 
 def test_noalloc_rejects_oversized_scratch():
-    """fp32, 4 bucket slices, 8 heads x 2^20 tokens: 8.6 GB of partial
-    outputs cannot live in the 64 MiB array -- a clear error before any GPU
-    call (runs on the CPU)."""
+    """fp32, 8 heads x 2^20 tokens: counted with the 8.6 GB of partial outputs
+    that slices of 32 buckets would have, the call does not go into the 64 MiB
+    array -- a clear error before any GPU call (runs on the CPU)."""
     from race_attention_amd import _lib
     lib = _lib.load()
     d = _lib.RaceDesc()
