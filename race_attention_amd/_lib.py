@@ -9,6 +9,7 @@ import ctypes
 import importlib.util
 import os
 import threading
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 # RACE_ATTENTION_LIB selects another build of the library (e.g. the host-side
@@ -119,21 +120,34 @@ _calls = None
 
 
 def calls():
-    """The C++ autograd calls (csrc/race_torch.cpp), bound to this library (raises if they have not been built)."""
+    """The C++ autograd calls (csrc/race_torch.cpp), bound to this library, or
+    None where they are not built or do not load with the installed torch: the
+    Python Functions make the same calls, at more host time each.  That is said
+    once, as a RuntimeWarning."""
     global _calls
     if _calls is None:
         load()
         with _lock:
             if _calls is None:
-                if not os.path.exists(TORCH_PATH):
-                    raise RaceError(f"{TORCH_PATH} is not built; run `python race_attention_amd/build.py`")
-                import torch  # noqa: F401  (its libraries)
-                spec = importlib.util.spec_from_file_location("_race_torch", TORCH_PATH)
-                mod = importlib.util.module_from_spec(spec)
-                spec.loader.exec_module(mod)
-                mod.bind(LIB_PATH, RaceError)
-                _calls = mod
-    return _calls
+                try:
+                    _calls = _load_calls()
+                except (ImportError, OSError, RuntimeError) as e:
+                    _calls = False
+                    warnings.warn(f"{TORCH_PATH} is not used ({e}): operator calls go through Python, with the same "
+                                  "results; `python race_attention_amd/build.py` builds it", RuntimeWarning,
+                                  stacklevel=2)
+    return _calls or None
+
+
+def _load_calls():
+    import torch  # noqa: F401  (its libraries)
+    if not os.path.exists(TORCH_PATH):
+        raise ImportError("not built")
+    spec = importlib.util.spec_from_file_location("_race_torch", TORCH_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.bind(LIB_PATH, RaceError)
+    return mod
 
 
 def check(rc: int, what: str) -> None:

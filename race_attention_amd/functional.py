@@ -239,12 +239,14 @@ def _native(kind, q, k, v, planes, temp, kmask, L, K, causal, want_den, eps):
     """The C++ call of an operator, or None where it is not one that those take."""
     if not (torch.is_tensor(q) and q.is_cuda):
         return None
+    mod = _lib.calls()
+    if mod is None:
+        return None
     lo = hi = -1.0
     if isinstance(temp, LogitTemp):
         temp, lo, hi = temp.logit, temp.lo, temp.hi
     elif isinstance(temp, int):
         temp = float(temp)
-    mod = _lib.calls()
     return mod.call(getattr(mod, kind), q, k, v, planes, temp, kmask, int(L), int(K), bool(causal), want_den,
                     float(eps), lo, hi)
 

@@ -370,3 +370,35 @@ def test_a_scale_put_on_the_class_and_an_attribute_of_any_name(dev, monkeypatch)
 
     got = race_bucket_probs_from_qk(SimpleNamespace(ace=Own, M=1), q[0], k[0])
     _equal(got, [race_bucket_probs(t, planes, L=L, K=K, inv_temp=0.5) for t in (q, k)])
+
+
+@pytest.mark.parametrize("why", ["absent", "not a library"])
+def test_the_python_functions_alone(dev, why, monkeypatch, tmp_path):
+    """Where the C++ calls are not built, or do not load, the Python Functions
+    make every call; it is said once."""
+    import warnings
+
+    from race_attention_amd import _lib, vit
+    from race_attention_amd.functional import race_attention, race_attention_global, race_bucket_probs
+    (q, k, v), do, planes = _inputs(dev)
+    ace = vit.BatchedACE(d_k=64, K=K, L=L, M=1).to(dev)
+
+    def calls():
+        a, b, c = _leaves((q, k, v))
+        out = race_attention(a, b, c, planes, L=L, K=K, causal=True, inv_temp=0.5)
+        layer = ace(b, c, a)  # (no gradient of its temperature: that sums in another order as torch expressions)
+        return [out, *torch.autograd.grad(out, (a, b, c), do), *torch.autograd.grad(layer, (a, b, c), do),
+                *race_attention_global(q, k, v, planes, L=L, K=K, beta=1.0),
+                race_bucket_probs(q, planes, L=L, K=K, inv_temp=0.5)]
+
+    want = calls()
+    path = tmp_path / "_race_torch.so"
+    if why != "absent":
+        path.write_bytes(b"no library")
+    monkeypatch.setattr(_lib, "TORCH_PATH", str(path))
+    monkeypatch.setattr(_lib, "_calls", None)
+    with pytest.warns(RuntimeWarning, match="operator calls go through Python"):
+        race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error", RuntimeWarning)
+        _equal(calls(), want)

@@ -152,10 +152,18 @@ def test_noalloc_automatic_segmentation_fits(dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("L,K", [(5, 3), (3, 5)])
-def test_noalloc_fp32_partials_in_scratch(dev, L, K):
-    """fp32 runs one workgroup for all buckets of 3 bits, and at 5 bits bucket
-    slices whose fp32 partial outputs also live in the array."""
+def test_noalloc_fp32_partials_in_scratch(dev):
+    """fp32: one workgroup for all buckets of 3 bits."""
+    _fp32_in_scratch(dev, L=5, K=3)
+
+
+@pytest.mark.gpu
+def test_noalloc_fp32_slices_in_scratch(dev):
+    """fp32 at 5 bits runs bucket slices whose partial outputs also live in the array."""
+    _fp32_in_scratch(dev, L=3, K=5)
+
+
+def _fp32_in_scratch(dev, L, K):
     T, H = 1000, 2
     q, k, v, do, planes = make_case(B=2, T=T, H=H, L=L, K=K, dtype=torch.float32, unit=False, seed=5)
     qd, kd, vd = [x.to(dev) for x in (q, k, v)]
