@@ -13,11 +13,12 @@
 // These functions take the ordinary calls: plain CUDA tensors on the current
 // device, bf16 or fp32, shapes and arguments that agree.  For everything else
 // (mismatched shapes, CPU tensors, tensor subclasses, functorch transforms,
-// tracing, a status other than RACE_OK) they return None and the caller takes the
+// tracing, an active dispatch mode, a status other than RACE_OK) they return None and the caller takes the
 // Python path, whose errors and conversions are then what they always were.
 #include <dlfcn.h>
 #include <torch/extension.h>
 
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -302,7 +303,8 @@ std::optional<Tensor> given(const Tensor &x) { return x.defined() ? std::optiona
 // the logit of an fp32 temperature clamped to [lo, hi].
 py::object call(int64_t kind, py::handle hq, py::handle hk, py::handle hv, py::handle hplanes, py::handle htemp,
                 py::handle hmask, int64_t L, int64_t K, bool causal, bool want_den, double eps, double lo, double hi) {
-    if (!is_tensor(hq) || !is_tensor(hk) || !is_tensor(hv) || !is_tensor(hplanes) || torch::jit::tracer::isTracing())
+    if (!is_tensor(hq) || !is_tensor(hk) || !is_tensor(hv) || !is_tensor(hplanes) || torch::jit::tracer::isTracing() ||
+        c10::impl::TorchDispatchModeTLS::any_modes_set())
         return py::none();
     const Tensor &q = THPVariable_Unpack(hq.ptr()), &k = THPVariable_Unpack(hk.ptr()), &v = THPVariable_Unpack(hv.ptr());
     Tensor planes = THPVariable_Unpack(hplanes.ptr()), temp, mask;

@@ -402,3 +402,34 @@ def test_the_python_functions_alone(dev, why, monkeypatch, tmp_path):
     with warnings.catch_warnings():
         warnings.simplefilter("error", RuntimeWarning)
         _equal(calls(), want)
+
+
+def test_an_active_dispatch_mode_sees_the_python_call(dev):
+    """Under a TorchDispatchMode the Python Functions run, whose allocations and
+    conversions the mode sees as ever; a function mode (as set_default_device
+    installs) leaves the C++ call in place.  Results are the same."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from race_attention_amd.functional import _native, race_attention
+    (q, k, v), do, planes = _inputs(dev)
+    want = race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5)
+    native = lambda: _native("F1", q, k, v, planes, 0.5, None, L, K, True, False, 1e-6)  # noqa: E731
+    seen = []
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Through(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Log():
+        assert native() is None
+        _equal([race_attention(q, k, v, planes, L=L, K=K, causal=True, inv_temp=0.5)], [want])
+    assert any("empty" in f for f in seen)
+    with Through():
+        _equal([native()], [want])
+    _equal([native()], [want])
