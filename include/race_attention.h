@@ -57,7 +57,8 @@ typedef struct race_desc {
     int64_t do_stride[4];     /* upstream gradient */
     int64_t g_stride[4];      /* dq, dk, dv */
     int32_t seg_tiles;        /* 32-token tiles per scan segment, forward and backward; 0 = automatic
-                                 (the backward then joins whole forward segments into fewer ones).
+                                 (the causal backward then joins whole forward segments into
+                                 fewer ones, the non-causal one takes its own).
                                  Automatic segments are at most 256 tiles at any T, and the
                                  backward calls reject an explicit value above 256: the
                                  whole-tile bf16 kernels walk B in fp32 through a segment, so
@@ -72,7 +73,11 @@ typedef struct race_desc {
 } race_desc;
 
 /* Bytes of the forward->backward state buffer (per-segment prefix carries,
- * fp64).  race_fwd writes it; race_bwd reads it. */
+ * fp64; the non-causal operator fills the totals only).  race_fwd writes it;
+ * race_bwd reads it.  A state belongs to the descriptor that made it, seg_tiles
+ * included: with another seg_tiles its rows lie elsewhere, which a call cannot
+ * see (automatic segments are one tile long, as with seg_tiles = 1, only up to
+ * 1024 tiles x streams x bucket slices). */
 size_t race_state_bytes(const race_desc *d);
 
 /* Scratch bytes needed by race_fwd / race_bwd. */

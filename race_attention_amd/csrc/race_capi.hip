@@ -49,9 +49,10 @@ int ok() {
 // 3 280, 768 of 8 234; fp32 K=4 L=8 8 x 8192: 2048 of 1 433, 256 of 8 282.
 constexpr int64_t kTargetBlocks = 2048;
 constexpr int64_t kLongSegTiles = 64;
-// Up to this many tiles (and slices) in all, segments stay one tile each: there
-// the state of an automatic forward is also that of seg_tiles = 1, which
-// backward calls with either are used with.
+// Up to this many tiles (and slices) in all, segments stay one tile each: not for
+// time (of 513 to 1024 tiles of 128 buckets short_tiles would join two), but
+// because the state of an automatic forward is there also that of seg_tiles = 1,
+// and backward calls with either are used with it.
 constexpr int64_t kOneTileBlocks = 1024;
 // Workgroups that a launch of the forward and of the backward tile kernels aims
 // at, by slice size (8-, 4- and 2-wave workgroups; 256 CUs).  128 buckets: what is
@@ -453,8 +454,11 @@ void dx_finish(const Plan &p, const race_desc *d, const void *part, const Args &
 // for the causal bf16 slices of 128 buckets at 4 and 8 hash bits and of 32 and
 // 64 at 2 to 4, and used when every tile holds TT tokens (T % TT == 0) and
 // every bucket of every slice is one of the S buckets, so no load, store or
-// probability needs a row or bucket guard.  Those of 32 and 64 buckets do the
-// general ones' arithmetic (walk_f64) without the guards: forward + backward of
+// probability needs a row or bucket guard.  Those of 32 and 64 buckets walk B in
+// fp64 as the general ones do (walk_f64); without the guards the compiler forms
+// P_K's lo part with the product that makes P_K, one rounding fewer, so outputs
+// differ from the general kernels' (by 3e-5 of 2e-3 and more off 64 bits, either
+// way the same).  Forward + backward of
 // 48 x 8192, us: K=4 L=4 351 -> 319 (global 354 -> 324), L=2 354 -> 319 (396 ->
 // 358), K=3 L=8 390 -> 364, L=4 369 -> 332, K=2 L=16 374 -> 349, L=8 357 -> 323.
 // Elsewhere the template argument is false and both branches below launch the

@@ -1597,9 +1597,10 @@ template <typename T, int NW> __device__ __forceinline__ float wave_sum(const fl
 // would allow, at more than 128 registers).
 __host__ __device__ constexpr int bwd_max_waves(int SP, bool causal) { return causal && SP == 128 ? 2 : 8; }
 
-// Workgroups per CU of a backward tile kernel with nw waves and `bytes` of
-// LDS: the kernels need more than 128 VGPRs, so at most 2 waves per SIMD
-// (8 per CU) run, whatever the LDS allows.
+// Workgroups per CU of a backward tile kernel with nw waves and `bytes` of LDS, at
+// 2 waves per SIMD (8 per CU): what the causal kernels' 200 to 256 VGPRs allow.
+// The non-causal ones (100 to 200) would run more if their LDS let them; whether
+// one token block there pays is not measured.
 __host__ __device__ constexpr size_t bwd_wgs_per_cu(int nw, size_t bytes) {
     return (160 * 1024 / bytes) < (size_t)(8 / nw) ? 160 * 1024 / bytes : (size_t)(8 / nw);
 }
@@ -2449,7 +2450,7 @@ __global__ __launch_bounds__(threads_of(SP), fwd_waves(is_bf16<T>(), SP)) void k
 // enter G rounded to bf16 exactly as k_bwd_out's in-tile dP_K term takes
 // them (the same MFMA, the same rounding), so its t = tau terms, alpha's
 // gd P_Q against W v.g, cancel as well.
-// With every bucket of the stream in one workgroup (bf16, K <= 4: GC) the
+// With every bucket of the stream in one workgroup (K <= 4: GC) the
 // kernel sums S_t itself, over its waves, after the tile's G.  Bucket slices
 // (GS) take it from a pre-pass: the same kernel with GP set walks the tiles
 // as far as G and writes its slice's share of S_t; k_gn_terms adds the

@@ -95,6 +95,34 @@ def test_sliced_backward_takes_about_the_tiles_it_has(N, T, K, L, causal):
     assert rounds * longest <= 1.35 * ntiles * N * nslice / 256, (f, b, rounds, longest)
 
 
+@pytest.mark.parametrize("B,T,H,K,L,fnseg,nseg", [
+    (1, 8192, 8, 4, 8, 32, 32),    # 8 tiles for each of 256 workgroups of 128 buckets: one residency
+    (1, 8160, 8, 4, 8, 64, 32),    # 8 tiles fewer: two rounds, joined in pairs
+    (1, 8192, 8, 3, 10, 32, 32),   # 80 of 128 buckets
+    (1, 262001, 8, 4, 8, 32, 32),  # segments of 256 tiles, the longest
+    (4, 4001, 12, 3, 8, 10, 10),   # 64 buckets: 512
+    (1, 8192, 4, 4, 8, 256, 64),   # 1024 tiles: one-tile forward segments
+    (2, 4096, 8, 8, 1, 4, 4),      # 8 slices of 32 buckets
+    (1, 20, 1, 4, 8, 1, 1),
+])
+def test_fp32_plans(B, T, H, K, L, fnseg, nseg):
+    from race_attention_amd import _lib
+    assert _plan(B, T, H, K, L, _lib.RACE_DTYPE_F32, 1) == (fnseg, nseg)
+
+
+def test_all_plans_cover_the_sequence_within_the_walk_bound():
+    from race_attention_amd import _lib
+    for dtype in (_lib.RACE_DTYPE_F32, _lib.RACE_DTYPE_BF16):
+        for causal in (0, 1):
+            for B, H in ((1, 1), (1, 4), (2, 12), (12, 8), (64, 6)):
+                for K, L in ((2, 5), (3, 8), (3, 10), (4, 6), (4, 8), (5, 6), (6, 5), (8, 4)):
+                    for T in (1, 33, 785, 4097, 8160, 30000, 250001):
+                        f, b = _plan(B, T, H, K, L, dtype, causal)
+                        ntiles = -(-T // 32)
+                        assert 1 <= b <= f <= ntiles, (dtype, causal, B, H, K, L, T, f, b)
+                        assert -(-ntiles // f) <= 256 and (ntiles <= 256 or -(-ntiles // b) <= 256)
+
+
 def test_non_causal_backward_of_64_buckets_takes_whole_rounds():
     """Two workgroups of 64 buckets per CU (K = 4: three): 2048 tiles of 16 streams
     in one round of 512, not in one and a half."""
