@@ -136,11 +136,13 @@ double rounds_cost(int64_t wgs, int64_t r, int64_t tiles) {
 double whole_rounds(const Plan &p, int64_t fnseg, int64_t tps, int64_t most, int64_t &join) {
     double cost = 1e300;
     for (int64_t j = 1; j <= most && j <= fnseg; ++j) {
-        const double c = rounds_cost(launch_wgs(p, (fnseg + j - 1) / j), 1, j * tps);
+        const int64_t wgs = launch_wgs(p, (fnseg + j - 1) / j);
+        const double c = rounds_cost(wgs, 1, j * tps);
         if (c < cost) {
             cost = c;
             join = j;
         }
+        if (wgs <= 256) break;  // one round: longer segments only take longer
     }
     return cost;
 }
@@ -182,14 +184,20 @@ int64_t short_tiles(const race_desc *d, const Plan &p, int64_t per) {
 // forward's).  Backward, us, with one
 // residency of segments by target_blocks alone, and with this: K=3 L=8 16 x 65536
 // 397, 322; K=6 L=5 (3 slices) 48 x 8192 1178, 802.
-int64_t own_tiles(const race_desc *d, const Plan &p, int64_t per, bool capped) {
+int64_t own_tiles(const race_desc *d, const Plan &p, bool capped) {
     const bool bf = d->dtype == RACE_DTYPE_BF16;
     // 64 buckets in bf16: 16-column rows (K = 4) leave LDS for a third workgroup
     const int64_t r = bf && p.SP == 64 ? (d->K == 4 ? 3 : 2) : target_blocks(bf, p.SP, true, false) / 256;
-    const int64_t most = 4 * 256 * r / per + 1;
     int64_t best = 0;
     double cost = 1e300;
-    for (int64_t nseg = 1; nseg <= most && nseg <= p.fnseg; ++nseg) {
+    // one segment a stream, up to one more than fill four rounds; of the counts
+    // that put n workgroups on a CU the largest, whose segments are the shortest
+    const int64_t most = 4 * 256 * r / (p.N * p.nslice) + 1;
+    for (int64_t n = 0; n <= 8 * r; ++n) {
+        int64_t nseg = n ? 256 * n / (8 * p.nslice) * 8 / p.N : 1;
+        if (nseg < 1) continue;
+        if (nseg > most) nseg = most;
+        if (nseg > p.fnseg) nseg = p.fnseg;
         int64_t tl = (p.ntiles + nseg - 1) / nseg;
         if (capped && tl > kMaxSegTiles) tl = kMaxSegTiles;
         const double c = rounds_cost(launch_wgs(p, (p.ntiles + tl - 1) / tl), r, tl);
@@ -296,7 +304,7 @@ int make_plan(const race_desc *d, Plan &p, bool bwd = false, bool walks = true, 
         const int64_t per = p.N * p.nslice;
         const bool capped = walks && p.ntiles > kMaxSegTiles;
         if (!d->causal) {
-            p.tps = (int)own_tiles(d, p, per, capped);
+            p.tps = (int)own_tiles(d, p, capped);
             p.nseg = (int)((p.ntiles + p.tps - 1) / p.tps);
         } else if (const int64_t m = joined_segments(d, p, per, capped ? kMaxSegTiles / p.tps : p.fnseg); m > 1) {
             const int64_t tl = (int64_t)p.tps * m;
