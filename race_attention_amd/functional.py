@@ -223,8 +223,9 @@ class RACEFunction(torch.autograd.Function):
 class LogitTemp:
     """The inverse of a learnable temperature exp(logit) clamped to [lo, hi]
     (misc/vit.py:923), for the inv_temp argument of the operator: the C++ calls
-    compute it and its gradient in one launch each; value() is the same as
-    torch expressions."""
+    compute it and its gradient in one launch each (a first derivative: like the
+    operator's other gradients it is not differentiable again); value() is the
+    same as torch expressions."""
 
     __slots__ = ("logit", "lo", "hi")
 
